@@ -24,6 +24,7 @@
 
 #include "fx_mfma.h"
 #include "gemm_asm.h"
+#include "gemm_mid.h"
 
 namespace fx {
 
@@ -1045,6 +1046,26 @@ static int fast_gemm_nj(const GemmArgs& a) {
     return (int)nj;
 }
 
+// The small tile (gemm_mid.h) a forward runs on, or kMidNone for the 256-wide kernels: where
+// its modelled time is the lower one.  The whole-tile kernel's is fitted to the layer shapes
+// of 4,096 to 16,384 rows: a round of workgroups is 7 + 1.5 us per 64 values of K for 256 x 256
+// tiles, 6 + 1.2 us for 256 x 192.  Measured on both sides of the line (whole tiles / small
+// ones, us): 4096 x 512 x 512 15.6 / 6.5, 4096 x 2048 x 512 18.0 / 12.7, 8192 x 768 x 768
+// 18.1 / 14.7, 16384 x 512 x 2048 47.2 / 36.0; kept on whole tiles 16384 x 768 x 768 22.1 / 26.6,
+// 16384 x 2304 x 768 61.2 / 68.9, 16384 x 3072 x 768 77.2 / 83.6.  Without whole tiles the
+// small ones were faster than gemm_bias_act_kernel at every size tried (5001 x 768 x 3072
+// 98.7 / 34.7, 16001 x 3072 x 768 92 / 82), which keeps the residual and the comparisons.
+static int mid_forward_tile(const GemmArgs& a, int nj) {
+    if (a.res || a.nw || (a.Xg && !a.idx) || !whole_tile_kernels_enabled('f')) return kMidNone;
+    int tile;
+    const float mid = mid_cost(a.M, a.N, a.K, &tile);
+    if (nj == 0) return tile;
+    const float cus = (float)device_cus(), steps = (float)a.K / 64.f;
+    const float rounds = ceilf((float)(a.M / 256) * (float)(a.N / (64 * nj)) / cus);
+    const float whole = rounds * (nj == 4 ? 7.f + 1.5f * steps : 6.f + 1.2f * steps);
+    return mid < whole ? tile : kMidNone;
+}
+
 // ---------------------------------------------------------------------------
 // Weight gradient of a linear layer: C (M x N) = A^T B, A (K x M) = dY and B (K x N) =
 // X, both row-major with the contraction (tokens) down the rows, so dW = dY^T X.
@@ -1559,7 +1580,27 @@ static int linear_fwd(GemmArgs a, hipStream_t stream) {
     a.vec_r = a.res && a.ldres % 8 == 0 && ((uintptr_t)a.res & 15) == 0;
     const int64_t tiles = ((int64_t)(a.M + kGBM - 1) / kGBM) * ((a.N + kGBN - 1) / kGBN);
     FX_REQUIRE(tiles < 0x7fffffffLL, "fx_linear_fwd: too many tiles");
-    if (const int nj = fast_gemm_nj(a)) {
+    const int nj = fast_gemm_nj(a);
+    if (const int tile = mid_forward_tile(a, nj)) {
+        MidArgs m{};
+        m.A = MidOperand{a.A, a.lda, a.M, a.idx, a.F, a.R};
+        m.B = MidOperand{a.B, a.ldb, a.N, nullptr, 0, 0};
+        m.C = a.C;
+        m.ldc = a.ldc;
+        m.H = a.H;
+        m.ldh = a.ldh;
+        m.bias = a.bias;
+        m.Xg = a.idx ? a.Xg : nullptr;
+        m.ldxg = a.ldxg;
+        m.M = a.M;
+        m.N = a.N;
+        m.K = a.K;
+        m.vec_c = a.vec_c;
+        m.vec_h = a.vec_h;
+        return mid_forward(m, tile, (a.act != 0 ? 1 : 0) | (a.H ? 2 : 0) | (a.bias ? 4 : 0) | (a.act == 2 && a.H ? 16 : 0),
+                           stream);
+    }
+    if (nj) {
         const int64_t ft = (int64_t)(a.M / 256) * (a.N / (64 * nj));
         const int fe = (a.act != 0 ? 1 : 0) | (a.H ? 2 : 0) | (a.bias ? 4 : 0) | (a.act == 2 && a.H ? 8 : 0);
 #define FX_FAST_EPI(J, E) \

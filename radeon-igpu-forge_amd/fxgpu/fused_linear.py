@@ -11,9 +11,8 @@
   for the backward: dh = dy * gelu'(h) (one elementwise kernel), then dx = dh W
   on the library GEMM and dW = dh^T x on this build's split-K weight-gradient GEMM.
 * ``linear(x, weight)`` -- y = x W^T (no bias) with the same backward split: the
-  GPT's qkv, proj and fc2 projections.  Forwards of at most FEW_ROWS rows (decode
-  steps) run on the few-row kernel behind fx_linear_fwd, the whole_tiles() shapes on
-  its whole-tile kernel, the others on the library GEMM.
+  GPT's qkv, proj and fc2 projections.  Forwards that native_fwd() takes (few rows, whole
+  tiles, up to 16 GFLOP) run on fx_linear_fwd, the others on the library GEMM.
 * ``fused_mlp(x, w1, w2)`` -- gelu_tanh(x w1^T) w2^T as one autograd node: the GELU and
   its derivative g = gelu'(h) in the fc epilogue (g saved in place of the pre-activation),
   the product with g in the fc2 input gradient's epilogue (fx_linear_dgrad_gate).
@@ -82,6 +81,17 @@ def whole_tiles(M, N, K):
     return M % 256 == 0 and K % 32 == 0 and 128 <= K <= 1024 and (N % 256 == 0 or N % 192 == 0)
 
 
+def native_fwd(M, N, K):
+    """Forward products on fx_linear_fwd rather than the library GEMM: the few-row ones, the
+    whole_tiles() and those of up to 16 GFLOP, where the small tiles are at least as fast on the
+    GPU (4096 x 512 x 2048 16.4 us, 4096 x 2304 x 768 19.9) and a torch.mm call alone keeps the
+    host busy for 19 us.  Above, the library is ahead (4096 x 768 x 3072 25.5 against 32.1 us,
+    16384 x 512 x 2048 33.0 against 36.0, 16001 x 3072 x 768 66.7 against 82)."""
+    if 0 < M <= FEW_ROWS:
+        return True
+    return NATIVE_PROJ_FWD and (whole_tiles(M, N, K) or 0 < M * N * K <= 8 << 30)
+
+
 # Routing switches, set by interleaved A/Bs of the whole cfg5 training step (24 rounds of 5
 # steps, medians, one process).  With the two-step LDS buffers of the whole-tile kernels
 # (whole 128-byte lines from HBM), the qkv and proj forwards (whole_tiles()) on fx_linear_fwd
@@ -91,7 +101,7 @@ def whole_tiles(M, N, K):
 # tile epilogues that one workgroup per CU cannot overlap with its MFMA work).  fc2's, with
 # the saved GELU derivative multiplied in its epilogue, runs on this build's kernel.
 # NATIVE_INPUT_GRAD: input gradients on fx_linear_dgrad where input_grad() takes them;
-# NATIVE_PROJ_FWD: the whole_tiles() forwards on fx_linear_fwd.  False: the library GEMM.
+# NATIVE_PROJ_FWD: the native_fwd() forwards on fx_linear_fwd.  False: the library GEMM.
 NATIVE_INPUT_GRAD = False
 NATIVE_PROJ_FWD = True
 # NATIVE_GELU_INPUT_GRAD: only the input gradient with the GELU derivative folded in (the
@@ -163,7 +173,7 @@ class Linear(torch.autograd.Function):
         x2 = _rows(x)
         M, K = x2.shape
         native = x2.is_cuda and weight.is_contiguous() and weight.data_ptr() % 16 == 0 and K % 8 == 0
-        if native and (0 < M <= FEW_ROWS or (NATIVE_PROJ_FWD and whole_tiles(M, weight.shape[0], K))):
+        if native and native_fwd(M, weight.shape[0], K):
             y = _native_fwd(x2, weight)
         else:
             y = torch.mm(x2, weight.t())
@@ -329,7 +339,7 @@ class FusedMLP(torch.autograd.Function):
         call("fx_linear_fwd", ptr(x2), x2.stride(0), None, 0, 0, ptr(w1), None, ptr(u), ptr(gd), None,
              M, Fh, K, 2, stream_of(x))
         N = w2.shape[0]
-        if 0 < M <= FEW_ROWS or (NATIVE_PROJ_FWD and whole_tiles(M, N, Fh)):
+        if native_fwd(M, N, Fh) and w2.data_ptr() % 16 == 0:
             y = _native_fwd(u, w2)
         else:
             y = torch.mm(u, w2.t())

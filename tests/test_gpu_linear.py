@@ -571,3 +571,49 @@ def test_fused_mlp_against_composition_and_fp32(dev, monkeypatch, native, M, K, 
                             (w2a.grad, w2b.grad, w2r.grad)):
         assert oracle_close(ours, ref)
         assert oracle_close(comp, ref)
+
+
+# ---- small tiles (gemm_mid.hip): 256 x 128 and 64 x 128, whole or ragged, dense or gathered ---------
+# The same MFMAs on the same operands in the same K order as the 256-wide general kernel
+# (FX_GEMM_GENERAL), and the same roundings: equal bit for bit, at every edge of a tile.
+
+@pytest.mark.parametrize("M,K,N", [
+    (65, 8, 1),         # one row more than the few-row kernel takes, one K chunk, one column
+    (127, 72, 129),     # the last row and column of a tile, 8 values of K past a step; odd N
+    (513, 64, 640),     # one row in the last tile, a single K step
+    (300, 192, 136),    # three K steps: the stages wrap once
+    (2049, 200, 2560),  # 256 x 128 tiles with a one-row panel, a K tail
+    (4096, 512, 512),   # two 64 x 128 tiles a CU
+])
+@pytest.mark.parametrize("act,bias,want_h", [(0, False, False), (1, True, False), (2, True, True), (1, False, True)])
+def test_small_tiles_match_general_kernel(dev, monkeypatch, M, K, N, act, bias, want_h):
+    g = torch.Generator(device=dev).manual_seed(M + K + N)
+    x = torch.randn(M, K + 8, device=dev, generator=g).bfloat16()[:, :K]
+    W = (torch.randn(N, K, device=dev, generator=g) * K ** -0.5).bfloat16()
+    b = (torch.randn(N, device=dev, generator=g) * 0.1).bfloat16() if bias else None
+    print(f"small-tile fwd M={M} K={K} N={N} act={act} bias={bias}", flush=True)
+    y, h = _linear_fwd(x, W, b, act, want_h)
+    monkeypatch.setenv("FX_GEMM_GENERAL", "1")
+    yg, hg = _linear_fwd(x, W, b, act, want_h)
+    assert torch.equal(y, yg) and (not want_h or torch.equal(h, hg))
+
+
+@pytest.mark.parametrize("B,F,W,N", [(65, 8, 1, 24), (700, 40, 30, 256), (1003, 24, 5, 130)])
+def test_small_tiles_gather_matches_general_kernel(dev, monkeypatch, B, F, W, N):
+    from fxgpu.abi import call, ptr, stream_of
+    g = torch.Generator(device=dev).manual_seed(B + N)
+    R, K = 500, F * W
+    X = torch.randn(R, F, device=dev, generator=g).bfloat16()
+    idx = torch.randint(-2, R, (B,), device=dev, generator=g, dtype=torch.int32)   # some windows leave X
+    Wt = (torch.randn(N, K, device=dev, generator=g) * K ** -0.5).bfloat16()
+    b = torch.randn(N, device=dev, generator=g).bfloat16()
+
+    def run():
+        y = torch.empty(B, N, device=dev, dtype=torch.bfloat16)
+        xg = torch.full((B, K), 7.0, device=dev, dtype=torch.bfloat16)
+        call("fx_linear_fwd", ptr(X), F, ptr(idx), F, R, ptr(Wt), ptr(b), ptr(y), None, ptr(xg), B, N, K, 0, stream_of(X))
+        return y, xg
+    y, xg = run()
+    monkeypatch.setenv("FX_GEMM_GENERAL", "1")
+    yg, xgg = run()
+    assert torch.equal(y, yg) and torch.equal(xg, xgg)
