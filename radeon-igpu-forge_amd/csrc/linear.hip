@@ -1325,28 +1325,51 @@ __global__ void __launch_bounds__(256, 1) gemm_wgrad_fast_kernel(WgradArgs a) {
         store(a.C, a.ldc);
 }
 
-// C = bf16(sum over slices of the fp32 partials), slice 0 first; 8 consecutive
-// elements (one 16-byte store) per thread and step, N % 8 == 0
+// C = bf16(sum over slices of the fp32 partials), slice 0 first; N % 8 == 0.  V consecutive
+// elements per thread and step: 8 (one 16-byte store), or 4 where 8 would leave CUs without a
+// workgroup.  Four slices' loads are issued before their adds: a small output has too few
+// waves to hide one round trip per slice (512 x 512 in 8 slices, product and reduce: 17.7 ->
+// 16.0 us; no difference at 3072 x 768).
+template <int V>
 __global__ void __launch_bounds__(256)
 wgrad_reduce_kernel(const float* __restrict__ part, int slices, int64_t MN, int N, uint16_t* __restrict__ C,
                     int64_t ldc) {
     const int64_t stride = (int64_t)gridDim.x * 256;
-    for (int64_t v = (int64_t)blockIdx.x * 256 + threadIdx.x; v < MN / 8; v += stride) {
-        float s[8];
-        const float4* p = reinterpret_cast<const float4*>(part + v * 8);
-        float4 lo = p[0], hi = p[1];
-        s[0] = lo.x; s[1] = lo.y; s[2] = lo.z; s[3] = lo.w;
-        s[4] = hi.x; s[5] = hi.y; s[6] = hi.z; s[7] = hi.w;
-        for (int k = 1; k < slices; ++k) {
-            const float4* q = reinterpret_cast<const float4*>(part + (int64_t)k * MN + v * 8);
-            lo = q[0];
-            hi = q[1];
-            s[0] += lo.x; s[1] += lo.y; s[2] += lo.z; s[3] += lo.w;
-            s[4] += hi.x; s[5] += hi.y; s[6] += hi.z; s[7] += hi.w;
+    for (int64_t v = (int64_t)blockIdx.x * 256 + threadIdx.x; v < MN / V; v += stride) {
+        const float* p = part + v * V;
+        float4 s[V / 4];
+#pragma unroll
+        for (int h = 0; h < V / 4; ++h) s[h] = reinterpret_cast<const float4*>(p)[h];
+        int k = 1;
+        for (; k + 4 <= slices; k += 4) {
+            float4 t[4][V / 4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int h = 0; h < V / 4; ++h) t[u][h] = reinterpret_cast<const float4*>(p + (int64_t)(k + u) * MN)[h];
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int h = 0; h < V / 4; ++h) {
+                    s[h].x += t[u][h].x; s[h].y += t[u][h].y; s[h].z += t[u][h].z; s[h].w += t[u][h].w;
+                }
         }
-        const int64_t e = v * 8;
+        for (; k < slices; ++k)
+#pragma unroll
+            for (int h = 0; h < V / 4; ++h) {
+                const float4 t = reinterpret_cast<const float4*>(p + (int64_t)k * MN)[h];
+                s[h].x += t.x; s[h].y += t.y; s[h].z += t.z; s[h].w += t.w;
+            }
+        const int64_t e = v * V;
         const int64_t m = e / N, n = e - m * N;
-        st16(C + m * ldc + n, pack8(s));
+        uint32_t w[V / 2];
+#pragma unroll
+        for (int h = 0; h < V / 4; ++h) {
+            w[2 * h] = pack_bf16x2(s[h].x, s[h].y);
+            w[2 * h + 1] = pack_bf16x2(s[h].z, s[h].w);
+        }
+        if constexpr (V == 8) st16(C + m * ldc + n, make_uint4(w[0], w[1], w[2], w[3]));
+        else *reinterpret_cast<uint2*>(C + m * ldc + n) = make_uint2(w[0], w[1]);
     }
 }
 
@@ -1739,14 +1762,22 @@ extern "C" int fx_linear_fwd_ex(const fxLinearArgs* args, void* stream) {
 // would take as long as a full one) is split off: the rows from split_rows on (whole row
 // panels) run as a second product in tail_slices slices, one round.  The same plan drives the
 // general kernel (FX_GEMM_GENERAL), so the two agree bit for bit.
+// Small outputs of many tokens take the small tiles of gemm_mid.h where their modelled time is
+// the lower one: a 256-wide tile count of 2048 x 512 is 16, so filling the chip takes 16 slices,
+// 67 MB of fp32 partials written and read again, against 4 slices of 64 tiles of 128 x 128.
+// Measured with the reduce (256-wide / small, us, 4,096 tokens): 1536 x 512 27.9 / 21.3,
+// 2048 x 512 33.8 / 22.6, 512 x 512 22.5 / 15.7; kept on 256-wide tiles
+// the layers of 768 at 16,384 tokens (3072 x 768 76 us).  FX_WGRAD_TILE, set to anything, keeps
+// the 256-wide plan.
 struct WgradPlan {
     int nj, slices;
     bool fast;
     int64_t split_rows;  // 0: one product
     int tail_slices;
+    int mid;             // kMidNone, or the small tile
 };
 static WgradPlan wgrad_plan(int64_t M, int64_t N, int64_t K) {
-    WgradPlan p{0, 1, false, 0, 1};
+    WgradPlan p{0, 1, false, 0, 1, kMidNone};
     const char* tw = getenv("FX_WGRAD_TILE");
     const bool want4 = tw && tw[0] == '2' && tw[1] == '5' && tw[2] == '6';
     // M need not divide into whole 256-row panels: the last panel's loads are clamped and its
@@ -1778,6 +1809,22 @@ static WgradPlan wgrad_plan(int64_t M, int64_t N, int64_t K) {
             }
         }
     }
+    if (!tw) {
+        // rounds of 256-wide workgroups and, with slices, the partials' way through memory, fitted
+        // like mid_wgrad_cost; within 15 % of each other the 256-wide plan stays (768 x 768 of
+        // 16,384 tokens: 34.7 against 37.8 us; a head of 8192 x 512: 198 against 210 us with its losses)
+        const float per = p.nj == 3 ? 1.2f : p.nj == 4 ? 1.5f : 2.f;
+        auto rounds = [&](int64_t t, int sl) {
+            return ceilf((float)(t * sl) / (float)cus) * (5.f + per * (float)((nk + sl - 1) / sl)) +
+                   (sl > 1 ? 3.f + (float)sl * (float)M * (float)N * 8.f / 6.5e6f * ((float)t / (float)tiles) : 0.f);
+        };
+        const int64_t head = p.split_rows ? (p.split_rows / 256) * (N / (64 * p.nj)) : tiles;
+        const float whole = rounds(head, p.slices) + (p.split_rows ? rounds(tiles - head, p.tail_slices) : 0.f);
+        int tile, slices;
+        if (mid_wgrad_cost(M, N, K, &tile, &slices) < 0.85f * whole) {
+            p = WgradPlan{0, slices, false, 0, 1, whole_tile_kernels_enabled('w') ? tile : kMidNone};
+        }
+    }
     return p;
 }
 
@@ -1801,7 +1848,7 @@ extern "C" int fx_linear_wgrad(const uint16_t* dY, int64_t ldy, const uint16_t* 
                (long long)ldx, (long long)ldw);
     FX_REQUIRE(((((uintptr_t)dY) | ((uintptr_t)X) | ((uintptr_t)dW) | ((uintptr_t)work)) & 15) == 0,
                "fx_linear_wgrad: dY, X, dW and work must be 16-byte aligned");
-    const WgradPlan plan = K > 0 ? wgrad_plan(M, N, K) : WgradPlan{0, 1, false, 0, 1};
+    const WgradPlan plan = K > 0 ? wgrad_plan(M, N, K) : WgradPlan{0, 1, false, 0, 1, kMidNone};
     FX_REQUIRE((plan.slices == 1 && !plan.split_rows) || work != nullptr,
                "fx_linear_wgrad: null workspace (%d slices)", plan.split_rows ? plan.tail_slices : plan.slices);
     hipStream_t s = (hipStream_t)stream;
@@ -1819,6 +1866,19 @@ extern "C" int fx_linear_wgrad(const uint16_t* dY, int64_t ldy, const uint16_t* 
         a.N = (int)N;
         a.K = (int)K;
         a.slices = slices;
+        if (plan.mid) {
+            MidArgs m{};
+            m.A = MidOperand{a.A, a.lda, a.M, nullptr, 0, 0};
+            m.B = MidOperand{a.B, a.ldb, a.N, nullptr, 0, 0};
+            m.C = a.C;
+            m.ldc = a.ldc;
+            m.part = a.part;
+            m.M = a.M;
+            m.N = a.N;
+            m.K = a.K;
+            m.slices = slices;
+            if (int e = mid_wgrad(m, plan.mid, s)) return e;
+        } else
         // whole tiles and 32-token steps, every slice at least 4 steps: the generated loop (with
         // several slices each spans at least 4 64-token steps, the last perhaps 32 tokens short)
         if (plan.fast) {
@@ -1833,10 +1893,15 @@ extern "C" int fx_linear_wgrad(const uint16_t* dY, int64_t ldy, const uint16_t* 
         }
         if (int e = check_launch("gemm_wgrad")) return e;
         if (slices == 1) return 0;
-        int64_t blocks = (rows * N / 8 + 255) / 256;
+        const bool wide = rows * N / 8 >= 512 * (int64_t)device_cus();
+        int64_t blocks = (rows * N / (wide ? 8 : 4) + 255) / 256;
         if (blocks > 4096) blocks = 4096;
-        hipLaunchKernelGGL(wgrad_reduce_kernel, dim3((unsigned)blocks), dim3(256), 0, s, (const float*)work, slices,
-                           rows * N, (int)N, a.C, ldw);
+        if (wide)
+            hipLaunchKernelGGL(wgrad_reduce_kernel<8>, dim3((unsigned)blocks), dim3(256), 0, s, (const float*)work, slices,
+                               rows * N, (int)N, a.C, ldw);
+        else
+            hipLaunchKernelGGL(wgrad_reduce_kernel<4>, dim3((unsigned)blocks), dim3(256), 0, s, (const float*)work, slices,
+                               rows * N, (int)N, a.C, ldw);
         return check_launch("wgrad_reduce");
     };
     if (!plan.split_rows) return product(0, M, plan.slices);

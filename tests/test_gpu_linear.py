@@ -617,3 +617,26 @@ def test_small_tiles_gather_matches_general_kernel(dev, monkeypatch, B, F, W, N)
     monkeypatch.setenv("FX_GEMM_GENERAL", "1")
     yg, xgg = run()
     assert torch.equal(y, yg) and torch.equal(xg, xgg)
+
+
+@pytest.mark.parametrize("T,M,N,ld_pad", [
+    (64, 8, 8, 0),          # one step, one slice, one corner of a tile
+    (200, 136, 264, 8),     # a tail of 8 tokens, partial tiles both ways, strided rows
+    (4096, 512, 512, 0),    # 128 x 128 tiles, several slices
+    (2049, 1920, 640, 0),   # a one-token tail in the last slice
+    (8192, 256, 1200, 8),   # the last column tile 48 wide
+    (1024, 4000, 1000, 0),  # 256 x 128 tiles, or 128 x 128 in one slice
+])
+def test_small_tile_wgrad_matches_general(dev, monkeypatch, T, M, N, ld_pad):
+    # the same slices and K order as the general kernel: bit for bit
+    from fxgpu.fused_linear import linear_wgrad
+    g = torch.Generator(device=dev).manual_seed(T + M + N)
+    dy = torch.randn(T, M + ld_pad, device=dev, generator=g).bfloat16()[:, :M]
+    x = torch.randn(T, N + ld_pad, device=dev, generator=g).bfloat16()[:, :N]
+    print(f"small-tile wgrad T={T} M={M} N={N}", flush=True)
+    dw = linear_wgrad(dy, x)
+    monkeypatch.setenv("FX_GEMM_GENERAL", "1")
+    assert torch.equal(dw, linear_wgrad(dy, x))
+    ref = dy.double().t() @ x.double()
+    from tolerances import bf16_close
+    assert bf16_close(dw, ref, atol=1e-3 * float(ref.abs().max()), rtol=2.0 ** -8)
