@@ -1018,7 +1018,8 @@ __global__ void __launch_bounds__(256, 1) gemm_dgrad_fast_kernel(DgradArgs a) {
 
 // FX_GEMM_GENERAL in the environment routes products to the general kernels
 // (gemm_bias_act_kernel, gemm_wgrad_kernel): "1" all of them, a value containing 'f' the
-// forwards, one containing 'w' the weight gradients.  A diagnostic switch, read on every
+// forwards, one containing 'w' the weight gradients; one containing 'm' keeps forwards and
+// input gradients off the small tiles.  A diagnostic switch, read on every
 // call, that lets a test or a benchmark compare the whole-tile kernels with them.
 static bool whole_tile_kernels_enabled(char kind) {
     const char* v = getenv("FX_GEMM_GENERAL");
@@ -1046,6 +1047,12 @@ static int fast_gemm_nj(const GemmArgs& a) {
     return (int)nj;
 }
 
+static float whole_tile_cost(int64_t M, int64_t N, int64_t K, int nj) {
+    const float steps = (float)K / 64.f;
+    const float rounds = ceilf((float)(M / 256) * (float)(N / (64 * nj)) / (float)device_cus());
+    return rounds * (nj == 4 ? 7.f + 1.5f * steps : 6.f + 1.2f * steps);
+}
+
 // The small tile (gemm_mid.h) a forward runs on, or kMidNone for the 256-wide kernels: where
 // its modelled time is the lower one.  The whole-tile kernel's is fitted to the layer shapes
 // of 4,096 to 16,384 rows: a round of workgroups is 7 + 1.5 us per 64 values of K for 256 x 256
@@ -1056,14 +1063,11 @@ static int fast_gemm_nj(const GemmArgs& a) {
 // small ones were faster than gemm_bias_act_kernel at every size tried (5001 x 768 x 3072
 // 98.7 / 34.7, 16001 x 3072 x 768 92 / 82), which keeps the residual and the comparisons.
 static int mid_forward_tile(const GemmArgs& a, int nj) {
-    if (a.res || a.nw || (a.Xg && !a.idx) || !whole_tile_kernels_enabled('f')) return kMidNone;
+    if (a.res || a.nw || (a.Xg && !a.idx) || !whole_tile_kernels_enabled('f') || !whole_tile_kernels_enabled('m')) return kMidNone;
     int tile;
     const float mid = mid_cost(a.M, a.N, a.K, &tile);
     if (nj == 0) return tile;
-    const float cus = (float)device_cus(), steps = (float)a.K / 64.f;
-    const float rounds = ceilf((float)(a.M / 256) * (float)(a.N / (64 * nj)) / cus);
-    const float whole = rounds * (nj == 4 ? 7.f + 1.5f * steps : 6.f + 1.2f * steps);
-    return mid < whole ? tile : kMidNone;
+    return mid < whole_tile_cost(a.M, a.N, a.K, nj) ? tile : kMidNone;
 }
 
 // ---------------------------------------------------------------------------
@@ -1941,6 +1945,22 @@ static int dgrad_run(const char* fn, const uint16_t* dY, int64_t ldy, const uint
     FX_REQUIRE(((((uintptr_t)dY) | ((uintptr_t)W) | ((uintptr_t)H) | ((uintptr_t)dX)) & 15) == 0,
                "%s: dY, W, H and dX must be 16-byte aligned", fn);
     if (M == 0) return 0;
+    // the small tiles where their modelled time is the lower one, as in the forward
+    int tile;
+    if (mid_cost(M, N, K, &tile) < whole_tile_cost(M, N, K, nj) && whole_tile_kernels_enabled('m')) {
+        MidArgs m{};
+        m.A = MidOperand{dY, ldy, (int)M, nullptr, 0, 0};
+        m.B = MidOperand{W, ldw, (int)N, nullptr, 0, 0};
+        m.C = dX;
+        m.ldc = ldx;
+        m.G = H;
+        m.ldg = ldx;
+        m.M = (int)M;
+        m.N = (int)N;
+        m.K = (int)K;
+        m.vec_c = true;
+        return mid_dgrad(m, tile, epi, (hipStream_t)stream);
+    }
     DgradArgs a{dY, ldy, W, ldw, H, dX, ldx, (int)M, (int)N, (int)K};
     const unsigned tiles = (unsigned)((M / 256) * (N / (64 * nj)));
     hipStream_t s = (hipStream_t)stream;

@@ -111,6 +111,17 @@ NATIVE_PROJ_FWD = True
 # faster); evaluating the derivative from the pre-activation in that epilogue had measured
 # 0.04 ms slower than the library GEMM and fx_gelu_bwd.
 NATIVE_GELU_INPUT_GRAD = True
+# NATIVE_SMALL_INPUT_GRAD: the plain input gradients of small_dgrad() on fx_linear_dgrad.
+NATIVE_SMALL_INPUT_GRAD = True
+
+
+def small_dgrad(M, N, K):
+    """Plain input gradients where fx_linear_dgrad (small tiles) is at least as fast as the
+    library GEMM, up to 8,192 rows, K up to 3072 and 40 GFLOP: 4096 x 512 x 1536 15.9 us, 8192 x 256 x 768
+    9.2 (torch.mm: 19 us of host time alone), 4096 x 768 x 3072 35.3 against 37.0, 8192 x 3072
+    x 768 43.9 / 48.5, 8192 x 768 x 3072 47.2 / 48.2; not 4096 x 512 x 8192 (69.3 / 58.3) nor
+    16384 x 768 x 768 (1 % on a block's forward and backward)."""
+    return M <= 8192 and K <= 3072 and M * N * K <= 20 * 10 ** 9 and dgrad_tiles(M, N, K)
 
 
 def dgrad_tiles(M, N, K):
@@ -120,8 +131,8 @@ def dgrad_tiles(M, N, K):
 
 def input_grad(dy2, weight, g=None):
     """dx = dy2 @ weight (bf16), and with g (the GELU(tanh) derivative at the output of the
-    layer feeding this one, as fx_linear_fwd with act 2 stores it) bf16(dx) * g.  With
-    NATIVE_INPUT_GRAD, on fx_linear_dgrad for dgrad_tiles() shapes where it measured at
+    layer feeding this one, as fx_linear_fwd with act 2 stores it) bf16(dx) * g.  The
+    small_dgrad() products run on fx_linear_dgrad; with NATIVE_INPUT_GRAD, on fx_linear_dgrad for dgrad_tiles() shapes where it measured at
     least as fast as the library GEMM with the operands in the caches (input widths up to
     1024 columns: the cfg5 qkv, proj and fc input gradients, 52.1 / 22.9 / 66.0 us against
     60.5 / 25.4 / 67.2 us; from HBM 72.3 / 31.6 / 93.7 against 64.5 / 30.3 / 82.4 us); with
@@ -130,7 +141,8 @@ def input_grad(dy2, weight, g=None):
     fx_gelu_bwd, 125.5 against 133.6 from HBM); else torch.mm, then fx_gelu_bwd_gate for g."""
     M, K = dy2.shape
     N = weight.shape[1]
-    wanted = (NATIVE_INPUT_GRAD and (g is not None or N <= 1024)) or (NATIVE_GELU_INPUT_GRAD and g is not None)
+    wanted = ((NATIVE_INPUT_GRAD and (g is not None or N <= 1024)) or (NATIVE_GELU_INPUT_GRAD and g is not None)
+              or (NATIVE_SMALL_INPUT_GRAD and g is None and small_dgrad(M, N, K)))
     native = (wanted and dy2.is_cuda and dgrad_tiles(M, N, K)
               and weight.is_contiguous() and weight.data_ptr() % 16 == 0
               and dy2.stride(1) == 1 and dy2.stride(0) % 8 == 0 and dy2.data_ptr() % 16 == 0

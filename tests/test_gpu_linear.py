@@ -584,6 +584,9 @@ def test_fused_mlp_against_composition_and_fp32(dev, monkeypatch, native, M, K, 
     (300, 192, 136),    # three K steps: the stages wrap once
     (2049, 200, 2560),  # 256 x 128 tiles with a one-row panel, a K tail
     (4096, 512, 512),   # two 64 x 128 tiles a CU
+    (512, 160, 192),    # whole tiles of 256 x 192, an odd count of 32-wide K steps (2.5 of 64)
+    (512, 224, 256),    # whole tiles of 256 x 256, 7 K steps
+    (256, 288, 192),    # 9 K steps
 ])
 @pytest.mark.parametrize("act,bias,want_h", [(0, False, False), (1, True, False), (2, True, True), (1, False, True)])
 def test_small_tiles_match_general_kernel(dev, monkeypatch, M, K, N, act, bias, want_h):
@@ -593,9 +596,10 @@ def test_small_tiles_match_general_kernel(dev, monkeypatch, M, K, N, act, bias, 
     b = (torch.randn(N, device=dev, generator=g) * 0.1).bfloat16() if bias else None
     print(f"small-tile fwd M={M} K={K} N={N} act={act} bias={bias}", flush=True)
     y, h = _linear_fwd(x, W, b, act, want_h)
-    monkeypatch.setenv("FX_GEMM_GENERAL", "1")
-    yg, hg = _linear_fwd(x, W, b, act, want_h)
-    assert torch.equal(y, yg) and (not want_h or torch.equal(h, hg))
+    for route in ("1", "m"):   # the general kernel; the whole-tile one where it takes the shape
+        monkeypatch.setenv("FX_GEMM_GENERAL", route)
+        yg, hg = _linear_fwd(x, W, b, act, want_h)
+        assert torch.equal(y, yg) and (not want_h or torch.equal(h, hg))
 
 
 @pytest.mark.parametrize("B,F,W,N", [(65, 8, 1, 24), (700, 40, 30, 256), (1003, 24, 5, 130)])
@@ -640,3 +644,29 @@ def test_small_tile_wgrad_matches_general(dev, monkeypatch, T, M, N, ld_pad):
     ref = dy.double().t() @ x.double()
     from tolerances import bf16_close
     assert bf16_close(dw, ref, atol=1e-3 * float(ref.abs().max()), rtol=2.0 ** -8)
+
+
+@pytest.mark.parametrize("M,N,K,pad", [
+    (256, 256, 128, 0),     # two K steps
+    (512, 192, 160, 8),     # a K tail of 32, half a column tile, rows of dY strided
+    (256, 768, 288, 0),     # 4.5 K steps
+    (4096, 2048, 512, 0),   # 256 x 128 tiles
+    (4096, 512, 1536, 8),   # 64 x 128 tiles
+])
+def test_small_tile_dgrad_matches_whole_tiles(dev, monkeypatch, M, N, K, pad):
+    # plain, with the pre-activation and with the stored derivative: bit for bit the whole-tile kernel
+    from fxgpu.abi import call, ptr, stream_of
+    g = torch.Generator(device=dev).manual_seed(M + N + K)
+    dy = torch.randn(M, K + pad, device=dev, generator=g).bfloat16()[:, :K]
+    W = (torch.randn(K, N, device=dev, generator=g) * K ** -0.5).bfloat16()
+    h = torch.randn(M, N, device=dev, generator=g).bfloat16()
+
+    def run():
+        gated = torch.empty(M, N, device=dev, dtype=torch.bfloat16)
+        call("fx_linear_dgrad_gate", ptr(dy), dy.stride(0), ptr(W), N, ptr(h), ptr(gated), N, M, N, K, stream_of(dy))
+        return _dgrad(dy, W), _dgrad(dy, W, h), gated
+    print(f"small-tile dgrad M={M} N={N} K={K}", flush=True)
+    small = run()
+    monkeypatch.setenv("FX_GEMM_GENERAL", "m")
+    assert all(torch.equal(a, b) for a, b in zip(small, run()))
+    assert oracle_close(small[0], dy.float() @ W.float(), FRAC_OUT)
