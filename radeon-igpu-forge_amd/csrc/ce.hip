@@ -27,13 +27,34 @@ __device__ __forceinline__ void ms_merge(float& m, float& s, float m2, float s2)
     m = mn;
 }
 
-// Register-resident row: needs V % 8 == 0, ld % 8 == 0, ldg % 8 == 0 and 16-byte
-// aligned bases (checked by the host); V <= 8 * NT * NV.
+// The up to 8 elements of a 16-byte chunk that lie in [lo, hi) of it, one by one: the first and
+// last chunk of a row that starts or ends inside one (its neighbours' elements are neither read
+// nor written)
+__device__ __forceinline__ uint4 ce_ld_edge(const uint16_t* p, int lo, int hi) {
+    uint32_t w[4] = {0xff80ff80u, 0xff80ff80u, 0xff80ff80u, 0xff80ff80u};  // -inf: no maximum, no weight
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+        if (j >= lo && j < hi) w[j >> 1] = (w[j >> 1] & (0xffffu << (16 * (1 - (j & 1))))) | ((uint32_t)p[j] << (16 * (j & 1)));
+    return make_uint4(w[0], w[1], w[2], w[3]);
+}
+__device__ __forceinline__ void ce_st_edge(uint16_t* p, int lo, int hi, const uint4& u) {
+    const uint32_t w[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+        if (j >= lo && j < hi) p[j] = (uint16_t)(w[j >> 1] >> (16 * (j & 1)));
+}
+
+// Register-resident row: V <= 8 * NT * NV.  EDGE false: V % 8 == 0, ld % 8 == 0, ldg % 8 == 0
+// and 16-byte aligned bases (checked by the host).  EDGE true: any V, stride and alignment as
+// long as a row of grad starts at the same place of a 16-byte chunk as the row of logits does;
+// the row is cut at the 16-byte boundaries of memory, e elements of its first chunk being the
+// row before's (V <= 8 * NT * NV - 7).  An odd vocabulary puts every row at another offset:
+// [4096, 32003] took 287 us in the two-pass element-wise kernel (1.8 TB/s), 103 here (5.1).
 // Each thread reduces its own vectors to (max, sum exp(x - max)) without any
 // barrier; one block-wide merge of those pairs gives (M, Z); the gradient pass
 // then rereads the registers.  The target's gradient element is fixed up by the one
 // thread that holds it.
-template <int NT, int NV>
+template <int NT, int NV, bool EDGE>
 __global__ void __launch_bounds__(NT) ce_row_kernel(fxCEArgs a) {
     constexpr int NW = NT / 64;
     __shared__ float shm[NW], shs[NW];
@@ -41,19 +62,28 @@ __global__ void __launch_bounds__(NT) ce_row_kernel(fxCEArgs a) {
     const uint16_t* lr = a.logits + row * a.ld;
     const int64_t t = a.target[row];
     const bool valid = (t != a.ignore_index) && (t >= 0) && (t < a.V);
-    const int V8 = (int)(a.V >> 3);
+    const int e = EDGE ? (int)(((uintptr_t)lr >> 1) & 7) : 0;
+    const int V8 = EDGE ? (int)((a.V + e + 7) >> 3) : (int)(a.V >> 3);
+    const int tail = EDGE ? (int)(a.V + e) - 8 * (V8 - 1) : 8;  // elements of the last chunk, from its start
     const int tid = threadIdx.x;
+    // chunk c lies wholly inside the row (EDGE: neither a cut first nor a cut last one)
+    auto whole = [&](int c) { return !EDGE || ((c > 0 || e == 0) && (c < V8 - 1 || tail == 8)); };
+    auto store = [&](uint16_t* gb, int c, const uint4& v) {
+        if (whole(c)) st16_nt(gb + (int64_t)c * 8, v);
+        else ce_st_edge(gb + (int64_t)c * 8, c == 0 ? e : 0, c == V8 - 1 ? tail : 8, v);
+    };
     // x_t is read before the barrier: with grad == logits (in place) other threads
     // overwrite the row once the reduction is done.
     const float xt = (tid == 0 && valid) ? bf16_to_f32(lr[t]) : 0.f;
-    uint16_t* gr = a.grad != nullptr ? a.grad + row * a.ldg : nullptr;
+    uint16_t* gr = a.grad != nullptr ? a.grad + row * a.ldg - e : nullptr;  // chunk 0
+    const uint16_t* lb = lr - e;
     if (!valid) {  // no loss and a zero gradient row: the logits are not read
         if (tid == 0) a.row_loss[row] = 0.f;
         if (gr != nullptr) {
 #pragma unroll
             for (int i = 0; i < NV; ++i) {
                 const int c = i * NT + tid;
-                if (c < V8) st16_nt(gr + (int64_t)c * 8, make_uint4(0u, 0u, 0u, 0u));
+                if (c < V8) store(gr, c, make_uint4(0u, 0u, 0u, 0u));
             }
         }
         return;
@@ -64,7 +94,9 @@ __global__ void __launch_bounds__(NT) ce_row_kernel(fxCEArgs a) {
     for (int i = 0; i < NV; ++i) {
         const int c = i * NT + tid;
         xv[i] = make_uint4(0u, 0u, 0u, 0u);
-        if (c < V8) xv[i] = ld16_nt(lr + (int64_t)c * 8);
+        if (c < V8)
+            xv[i] = whole(c) ? ld16_nt(lb + (int64_t)c * 8)
+                             : ce_ld_edge(lb + (int64_t)c * 8, c == 0 ? e : 0, c == V8 - 1 ? tail : 8);
     }
     float m = kNegInf;
 #pragma unroll
@@ -109,7 +141,7 @@ __global__ void __launch_bounds__(NT) ce_row_kernel(fxCEArgs a) {
     const float gmul = *a.mul;
     const float scale = gmul / s;  // softmax * mul = exp(x - M) * (mul / Z)
     const float ml = m * kLog2e;
-    const int tc = (int)(t >> 3);
+    const int tc = (int)((t + e) >> 3);
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
         const int c = i * NT + tid;
@@ -119,17 +151,17 @@ __global__ void __launch_bounds__(NT) ce_row_kernel(fxCEArgs a) {
 #pragma unroll
             for (int j = 0; j < 8; ++j) f[j] = exp2_fast(fmaf(f[j], kLog2e, -ml)) * scale;
             if (c == tc) {
-                const int tj = (int)(t & 7);
+                const int tj = (int)((t + e) & 7);
 #pragma unroll
                 for (int j = 0; j < 8; ++j)
                     if (j == tj) f[j] -= gmul;
             }
-            st16_nt(gr + (int64_t)c * 8, pack8(f));
+            store(gr, c, pack8(f));
         }
     }
 }
 
-// Any V / stride / alignment: two passes over the row from global memory with an
+// Rows past the registers, or logits and gradient rows at different offsets of a 16-byte chunk: two passes over the row from global memory with an
 // online (max, sum) per thread merged across the block.
 __global__ void __launch_bounds__(256) ce_row_generic_kernel(fxCEArgs a) {
     __shared__ float shm[4], shl[4];
@@ -321,18 +353,7 @@ ce_lin_grad_scale_inplace_kernel(uint16_t* dw, int64_t nw, uint16_t* dx, int64_t
 
 using namespace fx;
 
-#define FX_CE_NV_CASES(NT, CALL)                                                            \
-    case 1: CALL(NT, 1); break;   case 2: CALL(NT, 2); break;   case 3: CALL(NT, 3); break;   \
-    case 4: CALL(NT, 4); break;   case 5: CALL(NT, 5); break;   case 6: CALL(NT, 6); break;   \
-    case 7: CALL(NT, 7); break;   case 8: CALL(NT, 8); break;   case 9: CALL(NT, 9); break;   \
-    case 10: CALL(NT, 10); break; case 11: CALL(NT, 11); break; case 12: CALL(NT, 12); break; \
-    case 13: CALL(NT, 13); break; case 14: CALL(NT, 14); break; case 15: CALL(NT, 15); break; \
-    case 16: CALL(NT, 16); break;
-#define FX_CE_NV_CASES10(NT, CALL)                                                          \
-    case 1: CALL(NT, 1); break;   case 2: CALL(NT, 2); break;   case 3: CALL(NT, 3); break;   \
-    case 4: CALL(NT, 4); break;   case 5: CALL(NT, 5); break;   case 6: CALL(NT, 6); break;   \
-    case 7: CALL(NT, 7); break;   case 8: CALL(NT, 8); break;   case 9: CALL(NT, 9); break;   \
-    case 10: CALL(NT, 10); break;
+#define FX_CE_CASE(NT, NV) case NV: FX_CALL(NT, NV); break;
 
 extern "C" int fx_ce_inv_nvalid(const int64_t* target, int64_t N, int64_t ignore_index,
                                 const float* grad_scale, float grad_scale_value, float* inv_n,
@@ -356,17 +377,19 @@ extern "C" int fx_ce_fwd_grad(const fxCEArgs* args, void* stream) {
     if (a.N == 0) return 0;
     const bool vec = (a.V % 8 == 0) && (a.ld % 8 == 0) && (((uintptr_t)a.logits & 15) == 0) &&
                      (a.grad == nullptr || ((a.ldg % 8 == 0) && (((uintptr_t)a.grad & 15) == 0)));
-    const int64_t V8 = a.V / 8;
+    // rows of logits and grad at the same offset of a 16-byte chunk, every row of them
+    const bool edge = !vec && (a.grad == nullptr || ((((uintptr_t)a.logits ^ (uintptr_t)a.grad) & 15) == 0 &&
+                                                     (a.ld - a.ldg) % 8 == 0));
+    const int64_t V8 = edge ? (a.V + 14) / 8 : a.V / 8;
     // block size: the first of 64, 256, 512, 768, 1024 threads that holds the row in at
-    // most 8 vectors per lane, else the first of 64, 256, 512, 1024 with at most 16.  Fewer
+    // most 8 vectors per lane, else 1024 with at most 16.  Fewer
     // vectors per lane shorten the phase in which a row's block computes instead of
     // loading: at [16384, 50304] 1024 x 7 ran 548 us against 560 us for 768 x 9 and 576 us
     // for 512 x 13 (one process, medians), and a plain copy with the same access pattern
     // 582 us.
     int nt = 0, nv = 0;
-    if (vec) {
+    if (vec || edge) {
         static const int nts8[] = {64, 256, 512, 768, 1024};
-        static const int nts16[] = {64, 256, 512, 1024};
         for (int cand : nts8) {
             const int64_t need = (V8 + cand - 1) / cand;
             if (need <= 8) {
@@ -375,12 +398,9 @@ extern "C" int fx_ce_fwd_grad(const fxCEArgs* args, void* stream) {
                 break;
             }
         }
-        for (int k = 0; nt == 0 && k < 4; ++k) {
-            const int64_t need = (V8 + nts16[k] - 1) / nts16[k];
-            if (need <= 16) {
-                nt = nts16[k];
-                nv = (int)need;
-            }
+        if (nt == 0 && V8 <= 1024 * 16) {
+            nt = 1024;
+            nv = (int)((V8 + 1023) / 1024);
         }
     }
     const dim3 grid((unsigned)a.N);
@@ -389,13 +409,20 @@ extern "C" int fx_ce_fwd_grad(const fxCEArgs* args, void* stream) {
         hipLaunchKernelGGL(ce_row_generic_kernel, grid, dim3(256), 0, s, a);
         return check_launch("ce_row_generic");
     }
-#define FX_CALL(NT, NV) hipLaunchKernelGGL((ce_row_kernel<NT, NV>), grid, dim3(NT), 0, s, a)
+#define FX_CALL(NT, NV)                                                                       \
+    if (edge) hipLaunchKernelGGL((ce_row_kernel<NT, NV, true>), grid, dim3(NT), 0, s, a);     \
+    else hipLaunchKernelGGL((ce_row_kernel<NT, NV, false>), grid, dim3(NT), 0, s, a)
     switch (nt) {
-        case 64: switch (nv) { FX_CE_NV_CASES(64, FX_CALL) } break;
-        case 256: switch (nv) { FX_CE_NV_CASES(256, FX_CALL) } break;
-        case 512: switch (nv) { FX_CE_NV_CASES(512, FX_CALL) } break;
-        case 768: switch (nv) { FX_CE_NV_CASES10(768, FX_CALL) } break;
-        case 1024: switch (nv) { FX_CE_NV_CASES(1024, FX_CALL) } break;
+        // the counts the selection above can ask for
+        case 64: switch (nv) { FX_CE_CASE(64, 1) FX_CE_CASE(64, 2) FX_CE_CASE(64, 3) FX_CE_CASE(64, 4)
+                               FX_CE_CASE(64, 5) FX_CE_CASE(64, 6) FX_CE_CASE(64, 7) FX_CE_CASE(64, 8) } break;
+        case 256: switch (nv) { FX_CE_CASE(256, 3) FX_CE_CASE(256, 4) FX_CE_CASE(256, 5) FX_CE_CASE(256, 6)
+                                FX_CE_CASE(256, 7) FX_CE_CASE(256, 8) } break;
+        case 512: switch (nv) { FX_CE_CASE(512, 5) FX_CE_CASE(512, 6) FX_CE_CASE(512, 7) FX_CE_CASE(512, 8) } break;
+        case 768: switch (nv) { FX_CE_CASE(768, 6) FX_CE_CASE(768, 7) FX_CE_CASE(768, 8) } break;
+        case 1024: switch (nv) { FX_CE_CASE(1024, 7) FX_CE_CASE(1024, 8) FX_CE_CASE(1024, 9) FX_CE_CASE(1024, 10)
+                                 FX_CE_CASE(1024, 11) FX_CE_CASE(1024, 12) FX_CE_CASE(1024, 13)
+                                 FX_CE_CASE(1024, 14) FX_CE_CASE(1024, 15) FX_CE_CASE(1024, 16) } break;
     }
 #undef FX_CALL
     return check_launch("ce_row");

@@ -355,3 +355,37 @@ def test_linear_ce_cfg5_head_one_chunk(dev):
         o = res[chunk][2].float()
         tol = 2.0 ** -8 * rdW.abs() + 2e-3 * float(rdW.abs().max()) + 1e-9
         assert bool(((o - rdW).abs() <= tol).all()), chunk
+
+
+@pytest.mark.parametrize("V", [1, 3, 7, 8, 15, 257, 4089, 4097, 16377, 32003, 50257, 131065, 131073])
+@pytest.mark.parametrize("off,ld_pad,in_place", [(0, 0, False), (5, 3, False), (0, 1, True)])
+def test_rows_cut_inside_a_16_byte_chunk(dev, V, off, ld_pad, in_place):
+    # rows that start and end anywhere in a 16-byte chunk (odd V or stride, a view with an
+    # offset): values, and the elements around each row untouched.  131073 is past the registers
+    from fxlm.cross_entropy import _ce_rows
+    N, ld = 6, V + ld_pad
+    g = torch.Generator(device=dev).manual_seed(V + off)
+    print(f"ce edge V={V} off={off} ld={ld}", flush=True)
+    flat = (torch.randn(off + N * ld + 8, device=dev, generator=g) * 2).bfloat16()
+    lg = flat[off:off + N * ld].view(N, ld)[:, :V]
+    t = torch.randint(0, V, (N,), device=dev, generator=g)
+    t[1], t[2], t[3] = -100, V - 1, 0
+    x, before = lg.double(), flat.clone()
+    out = flat if in_place else torch.full_like(flat, 7.0)
+    guard = before if in_place else out.clone()
+    gr = out[off:off + N * ld].view(N, ld)[:, :V]
+    loss = torch.empty(N, device=dev)
+    mul = torch.full((), 0.25, device=dev)
+    _ce_rows(lg, t, gr, loss, mul, -100)
+    ok = t != -100
+    lse = x.logsumexp(-1)
+    want = torch.where(ok, lse - x.gather(1, t.clamp_min(0)[:, None])[:, 0], torch.zeros_like(lse))
+    assert torch.allclose(loss.double(), want, rtol=1e-5, atol=1e-5)
+    p = x.softmax(-1)
+    p.scatter_add_(1, t.clamp_min(0)[:, None], torch.full((N, 1), -1.0, device=dev, dtype=torch.float64))
+    ref = p * 0.25 * ok[:, None]
+    # one bf16 rounding (2^-9 of the value) and fp32 sums and exponentials (1e-5 of the scale)
+    assert bool(((gr.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-5 * 0.25).all())
+    keep = torch.ones_like(flat, dtype=torch.bool)
+    keep[off:off + N * ld].view(N, ld)[:, :V] = False
+    assert torch.equal(out[keep], guard[keep])
