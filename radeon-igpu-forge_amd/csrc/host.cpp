@@ -1,0 +1,458 @@
+// Host side of the op wrappers in C++ (module fxgpu._host): the buffers a call needs are
+// allocated from torch's caching allocator and its kernels launched through the C ABI in one
+// call from Python, on torch's current stream.  The autograd functions stay in Python
+// (fxlm/*.py, fxgpu/fused_linear.py) and call these from their forward and backward.
+//
+// Why: a small layer's kernels take 5-15 us each, and the same work done from Python took
+// longer: about 1.3 us per allocation, 5 per ctypes call with a dozen arguments, and the
+// checks and views between them.  A function that takes a checked tensor returns nothing
+// (None) when a check fails: the Python wrapper then goes through its own checks, which
+// raise the error or make the aligned copy.
+#include <torch/extension.h>
+#include <torch/csrc/utils/pybind.h>
+#include <c10/hip/HIPStream.h>
+
+#include <tuple>
+#include <vector>
+
+#include "../../include/fx_abi.h"
+
+namespace {
+
+using at::Tensor;
+using OptT = std::optional<Tensor>;
+
+void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.get_device()).stream(); }
+uint16_t* bf(const Tensor& t) { return static_cast<uint16_t*>(t.data_ptr()); }
+uint16_t* bf(const OptT& t) { return t.has_value() ? bf(*t) : nullptr; }
+float* f32(const Tensor& t) { return static_cast<float*>(t.data_ptr()); }
+bool aligned(const Tensor& t) { return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0; }
+bool is_bf(const Tensor& t) { return t.scalar_type() == at::kBFloat16; }
+at::TensorOptions as_f32(const Tensor& t) { return t.options().dtype(at::kFloat); }
+
+[[noreturn]] void raise(PyObject* type, const std::string& msg) {
+    PyErr_SetString(type, msg.c_str());
+    throw py::error_already_set();
+}
+
+// the C ABI's return code as the Python wrappers report it (fxgpu.abi.call)
+void check(int rc, const char* name) {
+    if (rc == 0) return;
+    const std::string msg = fx_last_error();
+    if (rc == FX_EINVAL) raise(PyExc_ValueError, msg);
+    raise(PyExc_RuntimeError, std::string(name) + " failed: hipError=" + std::to_string(rc) + " (" + msg + ")");
+}
+
+// ---- RMSNorm ---------------------------------------------------------------------------
+
+bool norm_ok(const Tensor& x, const Tensor& w) {
+    if (!is_bf(x) || !is_bf(w) || !x.is_cuda() || !w.is_cuda() || x.dim() < 1) return false;
+    const int64_t D = x.size(-1);
+    return w.dim() == 1 && w.size(0) == D && D >= 8 && D % 8 == 0 && D <= 8192 && x.is_contiguous() &&
+           w.is_contiguous() && aligned(x) && aligned(w);
+}
+
+// (y, rstd), or None when x or w need a check or a copy
+std::optional<std::tuple<Tensor, Tensor>> norm_fwd(const Tensor& x, const Tensor& w, double eps) {
+    if (!norm_ok(x, w)) return std::nullopt;
+    const int64_t D = x.size(-1), N = x.numel() / D;
+    Tensor y = at::empty(x.sizes(), x.options());
+    Tensor rstd = at::empty({N}, as_f32(x));
+    check(fx_rms_norm_fwd(bf(x), bf(w), bf(y), f32(rstd), N, (int32_t)D, (float)eps, stream_of(x)), "fx_rms_norm_fwd");
+    return std::make_tuple(y, rstd);
+}
+
+// (s, y, rstd) for s = x + r
+std::optional<std::tuple<Tensor, Tensor, Tensor>> norm_add_fwd(const Tensor& x, const Tensor& r, const Tensor& w,
+                                                               double eps) {
+    if (!norm_ok(x, w) || r.sizes() != x.sizes() || !is_bf(r) || !r.is_cuda() || !r.is_contiguous() || !aligned(r))
+        return std::nullopt;
+    const int64_t D = x.size(-1), N = x.numel() / D;
+    Tensor s = at::empty(x.sizes(), x.options());
+    Tensor y = at::empty(x.sizes(), x.options());
+    Tensor rstd = at::empty({N}, as_f32(x));
+    check(fx_rms_norm_fwd_add(bf(x), bf(r), bf(w), bf(s), bf(y), f32(rstd), N, (int32_t)D, (float)eps, stream_of(x)),
+          "fx_rms_norm_fwd_add");
+    return std::make_tuple(s, y, rstd);
+}
+
+// a gradient as the kernels read it: contiguous, 16-byte aligned, bf16
+Tensor grad_rows(const Tensor& g) {
+    Tensor t = g.contiguous();
+    if (!aligned(t)) t = t.clone();
+    if (!is_bf(t)) t = t.to(at::kBFloat16);
+    return t;
+}
+
+// (dx shaped like x, dw); dx += dres in the same pass when given
+std::tuple<Tensor, Tensor> norm_bwd(const Tensor& x, const Tensor& dy, const Tensor& w, const Tensor& rstd,
+                                    const OptT& dres) {
+    const int64_t D = x.size(-1), N = x.numel() / D;
+    const Tensor g = grad_rows(dy);
+    Tensor dx = at::empty(x.sizes(), x.options());
+    Tensor dw = at::empty({D}, w.options());
+    // fp32 dw, then the kernel's workspace
+    const int64_t nwork = fx_rms_norm_bwd_workspace(N, (int32_t)D) / 4, d4 = (D + 3) / 4 * 4;
+    Tensor buf = at::empty({d4 + (nwork < 1 ? 1 : nwork)}, as_f32(x));
+    float* dw32 = f32(buf);
+    if (dres.has_value()) {
+        const Tensor r = grad_rows(*dres);
+        check(fx_rms_norm_bwd_add(bf(x), bf(g), bf(r), bf(w), f32(rstd), bf(dx), dw32, bf(dw), dw32 + d4, N, (int32_t)D,
+                                  stream_of(x)),
+              "fx_rms_norm_bwd_add");
+    } else {
+        check(fx_rms_norm_bwd(bf(x), bf(g), bf(w), f32(rstd), bf(dx), dw32, bf(dw), dw32 + d4, N, (int32_t)D,
+                              stream_of(x)),
+              "fx_rms_norm_bwd");
+    }
+    return std::make_tuple(dx, dw);
+}
+
+// ---- attention -------------------------------------------------------------------------
+
+bool attn_ok(const Tensor& t) {
+    return is_bf(t) && t.is_cuda() && t.stride(-1) == 1 && t.stride(0) % 8 == 0 && t.stride(1) % 8 == 0 &&
+           t.stride(2) % 8 == 0 && aligned(t);
+}
+
+// q, k, v as the three slices of one (B, T, 3, H, Dh) tensor
+fxAttnArgs packed_args(const Tensor& qkv, bool causal, double scale) {
+    fxAttnArgs a{};
+    a.q = bf(qkv);
+    a.k = a.q + qkv.stride(2);
+    a.v = a.k + qkv.stride(2);
+    a.qsb = a.ksb = a.vsb = qkv.stride(0);
+    a.qst = a.kst = a.vst = qkv.stride(1);
+    a.qsh = a.ksh = a.vsh = qkv.stride(3);
+    a.B = (int32_t)qkv.size(0);
+    a.T = (int32_t)qkv.size(1);
+    a.H = (int32_t)qkv.size(3);
+    a.D = (int32_t)qkv.size(4);
+    a.scale = (float)scale;
+    a.causal = causal;
+    return a;
+}
+
+fxAttnArgs split_args(const Tensor& q, const Tensor& k, const Tensor& v, bool causal, double scale) {
+    fxAttnArgs a{};
+    a.q = bf(q);
+    a.k = bf(k);
+    a.v = bf(v);
+    a.qsb = q.stride(0), a.qst = q.stride(1), a.qsh = q.stride(2);
+    a.ksb = k.stride(0), a.kst = k.stride(1), a.ksh = k.stride(2);
+    a.vsb = v.stride(0), a.vst = v.stride(1), a.vsh = v.stride(2);
+    a.B = (int32_t)q.size(0);
+    a.T = (int32_t)q.size(1);
+    a.H = (int32_t)q.size(2);
+    a.D = (int32_t)q.size(3);
+    a.scale = (float)scale;
+    a.causal = causal;
+    return a;
+}
+
+std::tuple<Tensor, Tensor> attn_run_fwd(fxAttnArgs& a, const Tensor& like) {
+    Tensor o = at::empty({a.B, a.T, a.H, a.D}, like.options());
+    Tensor lse = at::empty({a.B, a.H, a.T}, as_f32(like));
+    a.o_out = bf(o);
+    a.lse_out = f32(lse);
+    check(fx_attn_fwd(&a, stream_of(like)), "fx_attn_fwd");
+    return std::make_tuple(o, lse);
+}
+
+// (o, lse), or None when a check of q, k, v fails
+std::optional<std::tuple<Tensor, Tensor>> attn_fwd(const Tensor& q, const Tensor& k, const Tensor& v, bool causal,
+                                                   double scale) {
+    if (q.dim() != 4 || k.sizes() != q.sizes() || v.sizes() != q.sizes()) return std::nullopt;
+    const int64_t Dh = q.size(3);
+    if ((Dh != 64 && Dh != 128) || q.numel() < 1 || q.numel() >= (int64_t)1 << 31 || !attn_ok(q) || !attn_ok(k) ||
+        !attn_ok(v))
+        return std::nullopt;
+    fxAttnArgs a = split_args(q, k, v, causal, scale);
+    return attn_run_fwd(a, q);
+}
+
+std::optional<std::tuple<Tensor, Tensor>> attn_fwd_qkv(const Tensor& qkv, bool causal, double scale) {
+    if (qkv.dim() != 5 || qkv.size(2) != 3 || !qkv.is_contiguous() || !is_bf(qkv) || !qkv.is_cuda() || !aligned(qkv))
+        return std::nullopt;
+    const int64_t Dh = qkv.size(4);
+    if ((Dh != 64 && Dh != 128) || qkv.numel() < 1 || qkv.numel() / 3 >= (int64_t)1 << 31) return std::nullopt;
+    fxAttnArgs a = packed_args(qkv, causal, scale);
+    return attn_run_fwd(a, qkv);
+}
+
+void attn_run_bwd(fxAttnArgs& a, const Tensor& o, const Tensor& lse, const Tensor& dout) {
+    Tensor d = dout.contiguous();
+    if (!is_bf(d)) d = d.to(at::kBFloat16);
+    Tensor delta = at::empty({a.B, a.H, a.T}, lse.options());
+    a.o = bf(o);
+    a.dout = bf(d);
+    a.lse = f32(lse);
+    a.delta = f32(delta);
+    check(fx_attn_bwd(&a, stream_of(o)), "fx_attn_bwd");
+}
+
+std::tuple<Tensor, Tensor, Tensor> attn_bwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o,
+                                            const Tensor& lse, const Tensor& dout, bool causal, double scale) {
+    fxAttnArgs a = split_args(q, k, v, causal, scale);
+    Tensor dq = at::empty(q.sizes(), q.options()), dk = at::empty(q.sizes(), q.options()),
+           dv = at::empty(q.sizes(), q.options());
+    a.dq = bf(dq);
+    a.dk = bf(dk);
+    a.dv = bf(dv);
+    const int64_t sh = a.D, st = sh * a.H, sb = st * a.T;
+    a.dqb = a.dkb = a.dvb = sb;
+    a.dqt = a.dkt = a.dvt = st;
+    a.dqh = a.dkh = a.dvh = sh;
+    attn_run_bwd(a, o, lse, dout);
+    return std::make_tuple(dq, dk, dv);
+}
+
+Tensor attn_bwd_qkv(const Tensor& qkv, const Tensor& o, const Tensor& lse, const Tensor& dout, bool causal,
+                    double scale) {
+    fxAttnArgs a = packed_args(qkv, causal, scale);
+    Tensor dqkv = at::empty(qkv.sizes(), qkv.options());
+    a.dq = bf(dqkv);
+    a.dk = a.dq + dqkv.stride(2);
+    a.dv = a.dk + dqkv.stride(2);
+    a.dqb = a.dkb = a.dvb = dqkv.stride(0);
+    a.dqt = a.dkt = a.dvt = dqkv.stride(1);
+    a.dqh = a.dkh = a.dvh = dqkv.stride(3);
+    attn_run_bwd(a, o, lse, dout);
+    return dqkv;
+}
+
+// ---- linear layers ---------------------------------------------------------------------
+
+// t as a (rows, cols) view whose rows are 16-byte aligned and unit-stride
+Tensor rows(const Tensor& t) {
+    Tensor r = t.dim() == 2 ? t : t.reshape({-1, t.size(-1)});
+    if (r.stride(1) != 1 || r.stride(0) % 8 || !aligned(r)) r = r.contiguous();
+    return r;
+}
+
+// y = act(x2 w^T + bias), and h (the pre-activation, act 2: the GELU derivative) when wanted
+std::tuple<Tensor, OptT> linear_fwd(const Tensor& x2, const Tensor& w, const OptT& bias, int64_t act, bool want_h) {
+    const int64_t M = x2.size(0), K = x2.size(1), N = w.size(0);
+    Tensor y = at::empty({M, N}, x2.options());
+    OptT h;
+    if (want_h) h = at::empty({M, N}, x2.options());
+    check(fx_linear_fwd(bf(x2), x2.stride(0), nullptr, 0, 0, bf(w), bf(bias), bf(y), bf(h), nullptr, M, N, K, (int32_t)act,
+                        stream_of(x2)),
+          "fx_linear_fwd");
+    return std::make_tuple(y, h);
+}
+
+// (out, Xg or None), or None when a check of the gather's inputs fails
+std::optional<std::tuple<Tensor, OptT>> gather_fwd(const Tensor& X, const Tensor& idx, const Tensor& w, const Tensor& b,
+                                                   bool want_xg) {
+    if (X.dim() != 2 || w.dim() != 2 || b.dim() != 1 || idx.dim() != 1) return std::nullopt;
+    const int64_t F = X.size(1), K = w.size(1), N = w.size(0), B = idx.size(0);
+    if (F < 8 || F % 8 || K % F || b.size(0) != N || !is_bf(X) || !is_bf(w) || !is_bf(b) || idx.scalar_type() != at::kInt ||
+        !X.is_cuda() || !idx.is_cuda() || !w.is_cuda() || !b.is_cuda() || !X.is_contiguous() || !idx.is_contiguous() ||
+        !w.is_contiguous() || !b.is_contiguous())
+        return std::nullopt;
+    Tensor out = at::empty({B, N}, X.options());
+    OptT xg;
+    if (want_xg) xg = at::empty({B, K}, X.options());
+    check(fx_linear_fwd(bf(X), F, static_cast<int32_t*>(idx.data_ptr()), F, X.size(0), bf(w), bf(b), bf(out), nullptr,
+                        bf(xg), B, N, K, 0, stream_of(X)),
+          "fx_linear_fwd");
+    return std::make_tuple(out, xg);
+}
+
+// dW = dy^T x
+Tensor wgrad(const Tensor& dy, const Tensor& x) {
+    if (!is_bf(dy) || !is_bf(x)) raise(PyExc_TypeError, "dy and x must be bfloat16");
+    if (!dy.is_cuda() || !x.is_cuda()) raise(PyExc_TypeError, "dy and x must be cuda tensors");
+    const Tensor dy2 = rows(dy), x2 = rows(x);
+    if (dy2.size(0) != x2.size(0))
+        raise(PyExc_ValueError, "dy has " + std::to_string(dy2.size(0)) + " rows, x has " + std::to_string(x2.size(0)));
+    const int64_t T = dy2.size(0), N = dy2.size(1), K = x2.size(1);
+    if (N % 8 || K % 8) return at::mm(dy2.t(), x2);
+    Tensor dW = at::empty({N, K}, x2.options());
+    const int64_t nbytes = fx_linear_wgrad_workspace(N, K, T);
+    Tensor work;
+    if (nbytes) work = at::empty({(nbytes + 3) / 4}, as_f32(x2));
+    check(fx_linear_wgrad(bf(dy2), dy2.stride(0), bf(x2), x2.stride(0), bf(dW), K, nbytes ? f32(work) : nullptr, N, K, T,
+                          stream_of(x2)),
+          "fx_linear_wgrad");
+    return dW;
+}
+
+// dx = dy2 w (times g), or None when a layout check fails
+OptT dgrad(const Tensor& dy2, const Tensor& w, const OptT& g) {
+    if (!dy2.is_cuda() || !w.is_contiguous() || !aligned(w) || dy2.stride(1) != 1 || dy2.stride(0) % 8 || !aligned(dy2) ||
+        (g.has_value() && (!g->is_contiguous() || !aligned(*g))))
+        return std::nullopt;
+    const int64_t M = dy2.size(0), K = dy2.size(1), N = w.size(1);
+    Tensor dx = at::empty({M, N}, dy2.options());
+    if (g.has_value())
+        check(fx_linear_dgrad_gate(bf(dy2), dy2.stride(0), bf(w), N, bf(*g), bf(dx), N, M, N, K, stream_of(dy2)),
+              "fx_linear_dgrad_gate");
+    else
+        check(fx_linear_dgrad(bf(dy2), dy2.stride(0), bf(w), N, nullptr, bf(dx), N, M, N, K, stream_of(dy2)),
+              "fx_linear_dgrad");
+    return dx;
+}
+
+// ---- cross-entropy ---------------------------------------------------------------------
+
+// device scalars (1 / n_valid, that times the gradient scale)
+std::tuple<Tensor, Tensor> ce_inv_nvalid(const Tensor& target, int64_t ignore, const OptT& gs, double gs_value) {
+    const auto o = target.options().dtype(at::kFloat);
+    Tensor inv_n = at::empty({}, o), mul = at::empty({}, o), g;
+    if (gs.has_value()) g = gs->detach().to(target.device(), at::kFloat).reshape({});
+    check(fx_ce_inv_nvalid(static_cast<int64_t*>(target.data_ptr()), target.numel(), ignore, gs.has_value() ? f32(g) : nullptr,
+                           (float)gs_value, f32(inv_n), f32(mul), stream_of(target)),
+          "fx_ce_inv_nvalid");
+    return std::make_tuple(inv_n, mul);
+}
+
+void ce_rows(const Tensor& logits, const Tensor& target, const OptT& grad, const Tensor& row_loss, const Tensor& mul,
+             int64_t ignore) {
+    fxCEArgs a{};
+    a.logits = bf(logits);
+    a.target = static_cast<int64_t*>(target.data_ptr());
+    a.grad = bf(grad);
+    a.row_loss = f32(row_loss);
+    a.mul = f32(mul);
+    a.N = logits.size(0);
+    a.V = logits.size(1);
+    a.ld = logits.stride(0);
+    a.ldg = grad.has_value() ? grad->stride(0) : a.V;
+    a.ignore_index = ignore;
+    check(fx_ce_fwd_grad(&a, stream_of(logits)), "fx_ce_fwd_grad");
+}
+
+Tensor ce_finalize(const Tensor& row_loss, const Tensor& inv_n) {
+    Tensor loss = at::empty({}, row_loss.options());
+    check(fx_ce_loss_finalize(f32(row_loss), row_loss.numel(), f32(inv_n), f32(loss), stream_of(row_loss)),
+          "fx_ce_loss_finalize");
+    return loss;
+}
+
+// (loss, dlogits or None) of checked logits and targets, or None when a check fails
+std::optional<std::tuple<Tensor, OptT>> ce_fwd(const Tensor& logits, const Tensor& target, int64_t ignore, bool want_grad) {
+    if (!is_bf(logits) || !logits.is_cuda() || !target.is_cuda() || !logits.is_contiguous() || !target.is_contiguous() ||
+        target.scalar_type() != at::kLong || logits.dim() != 2 || target.dim() != 1 || target.size(0) != logits.size(0))
+        return std::nullopt;
+    auto [inv_n, mul] = ce_inv_nvalid(target, ignore, std::nullopt, 1.0);
+    Tensor row_loss = at::empty({logits.size(0)}, as_f32(logits));
+    OptT grad;
+    if (want_grad) grad = at::empty(logits.sizes(), logits.options());
+    ce_rows(logits, target, grad, row_loss, mul, ignore);
+    return std::make_tuple(ce_finalize(row_loss, inv_n), grad);
+}
+
+void ce_scale_grad(const Tensor& grad, const Tensor& g32, const Tensor& applied, int64_t src) {
+    check(fx_ce_scale_grad(bf(grad), grad.numel(), f32(g32), f32(applied), (int32_t)src, stream_of(grad)),
+          "fx_ce_scale_grad");
+}
+
+void ce_lin_scale_inplace(const Tensor& dW, const Tensor& dx, const Tensor& g32, const OptT& gs, double inv) {
+    check(fx_ce_lin_grad_scale_inplace(bf(dW), dW.numel(), bf(dx), dx.numel(), f32(g32), gs.has_value() ? f32(*gs) : nullptr,
+                                       (float)inv, stream_of(dx)),
+          "fx_ce_lin_grad_scale_inplace");
+}
+
+// ---- optimiser -------------------------------------------------------------------------
+
+// The flat layout of FlatAdamW: per parameter its offset, size and weight-decay flag.
+struct FlatLayout {
+    std::vector<int64_t> off, n;
+    std::vector<int32_t> wd;
+    std::vector<fxTensorList> lists;   // filled anew by every step
+};
+
+// One optimiser step over the parameters that have a gradient.  t: master, m, v, flat16, step,
+// found_inf, grad norm, scale, growth.  h: lr, beta1, beta2, eps, weight decay, max norm,
+// growth interval.  Returns the workspace (grown when too small) and -1, or the index of a
+// parameter whose gradient is not bf16 (-2 - index: not 16-byte aligned), nothing launched.
+std::tuple<Tensor, int64_t> adamw_step(FlatLayout& f, const std::vector<Tensor>& params, const std::vector<Tensor>& t,
+                                       const std::vector<double>& h, Tensor work) {
+    std::vector<Tensor> keep;   // contiguous copies, alive until the launches are queued
+    f.lists.clear();
+    for (size_t i = 0; i < params.size(); ++i) {
+        Tensor g = params[i].grad();
+        if (!g.defined()) continue;
+        if (!is_bf(g)) return std::make_tuple(work, (int64_t)i);
+        if (!g.is_contiguous()) {
+            g = g.contiguous();
+            keep.push_back(g);
+        }
+        if (!aligned(g)) return std::make_tuple(work, -2 - (int64_t)i);
+        if (f.lists.empty() || f.lists.back().count == FX_ADAMW_MAX_TENSORS) {
+            f.lists.emplace_back();
+            f.lists.back().count = 0;
+        }
+        fxTensorList& l = f.lists.back();
+        l.g[l.count] = bf(g);
+        l.off[l.count] = f.off[i];
+        l.n[l.count] = f.n[i];
+        l.wd[l.count] = f.wd[i];
+        ++l.count;
+    }
+    fxTensorList none{};
+    const fxTensorList* lists = f.lists.empty() ? &none : f.lists.data();
+    const int32_t nl = (int32_t)f.lists.size();
+    const int64_t need = fx_adamw_workspace(lists, nl) / 4;
+    if (work.numel() < need) work = at::empty({need}, t[0].options());
+    fxAdamWState s{};
+    s.master = f32(t[0]);
+    s.m = f32(t[1]);
+    s.v = f32(t[2]);
+    s.p16 = bf(t[3]);
+    s.step = static_cast<int32_t*>(t[4].data_ptr());
+    s.found_inf = f32(t[5]);
+    s.grad_norm = f32(t[6]);
+    s.scale = f32(t[7]);
+    s.growth = static_cast<int32_t*>(t[8].data_ptr());
+    s.work = f32(work);
+    s.lr = (float)h[0];
+    s.beta1 = (float)h[1];
+    s.beta2 = (float)h[2];
+    s.eps = (float)h[3];
+    s.weight_decay = (float)h[4];
+    s.max_grad_norm = (float)h[5];
+    s.growth_factor = 2.f;
+    s.backoff_factor = 0.5f;
+    s.growth_interval = (int32_t)h[6];
+    check(fx_adamw_step(&s, lists, nl, stream_of(t[0])), "fx_adamw_step");
+    return std::make_tuple(work, (int64_t)-1);
+}
+
+}  // namespace
+
+// every function: torch's exceptions (out of memory among them) reach Python as themselves
+#define FX_DEF(name) m.def(#name, torch::wrap_pybind_function(name))
+
+PYBIND11_MODULE(_host, m) {
+    FX_DEF(norm_fwd);
+    FX_DEF(norm_add_fwd);
+    FX_DEF(norm_bwd);
+    FX_DEF(attn_fwd);
+    FX_DEF(attn_fwd_qkv);
+    FX_DEF(attn_bwd);
+    FX_DEF(attn_bwd_qkv);
+    FX_DEF(rows);
+    FX_DEF(linear_fwd);
+    FX_DEF(gather_fwd);
+    FX_DEF(wgrad);
+    FX_DEF(dgrad);
+    FX_DEF(ce_inv_nvalid);
+    FX_DEF(ce_rows);
+    FX_DEF(ce_finalize);
+    FX_DEF(ce_fwd);
+    FX_DEF(ce_scale_grad);
+    FX_DEF(ce_lin_scale_inplace);
+    py::class_<FlatLayout>(m, "FlatLayout")
+        .def(py::init([](std::vector<int64_t> off, std::vector<int64_t> n, std::vector<int32_t> wd) {
+            return FlatLayout{std::move(off), std::move(n), std::move(wd), {}};
+        }))
+        .def(py::pickle([](const FlatLayout& f) { return py::make_tuple(f.off, f.n, f.wd); },
+                        [](const py::tuple& t) {
+                            return FlatLayout{t[0].cast<std::vector<int64_t>>(), t[1].cast<std::vector<int64_t>>(),
+                                              t[2].cast<std::vector<int32_t>>(), {}};
+                        }));
+    FX_DEF(adamw_step);
+}

@@ -174,6 +174,24 @@ def lib():
     return _LIB
 
 
+class _Host:
+    """The host module (csrc/host.cpp): its functions allocate an op's buffers and launch its
+    kernels in one call.  Loaded on the first use, after torch and the library."""
+
+    def __getattr__(self, name):
+        lib()
+        try:
+            from . import _host
+        except ImportError as e:
+            raise RuntimeError(f"fxgpu/_host.so could not be loaded ({e}): build it first "
+                               "(python __graft_entry__.py build)") from e
+        v = getattr(_host, name)
+        setattr(self, name, v)
+        return v
+
+
+host = _Host()
+
 _FUNCS = {}
 
 

@@ -28,17 +28,14 @@ import ctypes
 
 import torch
 
-from fxgpu.abi import call, fxLinearArgs, lib, ptr, stream_of
+from fxgpu.abi import call, fxLinearArgs, host, ptr, stream_of
 
 _ACTS = {None: 0, "none": 0, "identity": 0, "gelu_tanh": 1}
 
 
 def _rows(t):
     """t as a (rows, cols) view whose rows are 16-byte aligned and unit-stride."""
-    t2 = t.reshape(-1, t.shape[-1])
-    if t2.stride(1) != 1 or t2.stride(0) % 8 or t2.data_ptr() % 16:
-        t2 = t2.contiguous()
-    return t2
+    return host.rows(t)
 
 
 def linear_wgrad(dy, x):
@@ -46,23 +43,7 @@ def linear_wgrad(dy, x):
     same leading shape; returns (N, K).  Widths that are not multiples of 8 (the
     kernel stages 16-byte column chunks) take the library GEMM, as the reference's
     rocBLAS dW does for every shape (ml/fxgpu/fused_linear.py:90-101)."""
-    if dy.dtype != torch.bfloat16 or x.dtype != torch.bfloat16:
-        raise TypeError("dy and x must be bfloat16")
-    if not (dy.is_cuda and x.is_cuda):
-        raise TypeError("dy and x must be cuda tensors")
-    dy2, x2 = _rows(dy), _rows(x)
-    if dy2.shape[0] != x2.shape[0]:
-        raise ValueError(f"dy has {dy2.shape[0]} rows, x has {x2.shape[0]}")
-    T, N = dy2.shape
-    K = x2.shape[1]
-    if N % 8 or K % 8:
-        return torch.mm(dy2.t(), x2)
-    dW = torch.empty(N, K, device=x.device, dtype=torch.bfloat16)
-    nbytes = int(lib().fx_linear_wgrad_workspace(N, K, T))
-    work = torch.empty((nbytes + 3) // 4, device=x.device, dtype=torch.float32) if nbytes else None
-    call("fx_linear_wgrad", ptr(dy2), dy2.stride(0), ptr(x2), x2.stride(0), ptr(dW), K, ptr(work), N, K, T,
-         stream_of(x))
-    return dW
+    return host.wgrad(dy, x)
 
 
 # Up to this many rows the forward GEMM is a stream over the weight (decoding, small
@@ -143,19 +124,10 @@ def input_grad(dy2, weight, g=None):
     N = weight.shape[1]
     wanted = ((NATIVE_INPUT_GRAD and (g is not None or N <= 1024)) or (NATIVE_GELU_INPUT_GRAD and g is not None)
               or (NATIVE_SMALL_INPUT_GRAD and g is None and small_dgrad(M, N, K)))
-    native = (wanted and dy2.is_cuda and dgrad_tiles(M, N, K)
-              and weight.is_contiguous() and weight.data_ptr() % 16 == 0
-              and dy2.stride(1) == 1 and dy2.stride(0) % 8 == 0 and dy2.data_ptr() % 16 == 0
-              and (g is None or (g.is_contiguous() and g.data_ptr() % 16 == 0)))
-    if native:
-        dx = torch.empty(M, N, device=dy2.device, dtype=torch.bfloat16)
-        if g is None:
-            call("fx_linear_dgrad", ptr(dy2), dy2.stride(0), ptr(weight), N, None, ptr(dx), N, M, N, K,
-                 stream_of(dy2))
-        else:
-            call("fx_linear_dgrad_gate", ptr(dy2), dy2.stride(0), ptr(weight), N, ptr(g), ptr(dx), N, M, N,
-                 K, stream_of(dy2))
-        return dx
+    if wanted and dgrad_tiles(M, N, K):
+        dx = host.dgrad(dy2, weight, g)     # None: a layout the kernel does not take
+        if dx is not None:
+            return dx
     dx = torch.mm(dy2, weight)
     if g is None:
         return dx
@@ -166,11 +138,7 @@ def input_grad(dy2, weight, g=None):
 
 def _native_fwd(x2, weight):
     """y = x2 W^T on fx_linear_fwd (the few-row kernel for M <= FEW_ROWS, else the tiled ones)."""
-    M, K = x2.shape
-    y = torch.empty(M, weight.shape[0], device=x2.device, dtype=torch.bfloat16)
-    call("fx_linear_fwd", ptr(x2), x2.stride(0), None, 0, 0, ptr(weight), None, ptr(y), None, None,
-         M, weight.shape[0], K, 0, stream_of(x2))
-    return y
+    return host.linear_fwd(x2, weight, None, 0, False)[0]
 
 
 class Linear(torch.autograd.Function):
@@ -217,6 +185,18 @@ class FusedGatherLinear(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, X16, idx32, weight, bias):
+        # Xg only serves the backward (dW); inference skips the write-out.
+        need_grad = any(ctx.needs_input_grad)
+        r = host.gather_fwd(X16, idx32, weight, bias, need_grad)
+        if r is None:
+            FusedGatherLinear._refuse(X16, idx32, weight, bias)
+        if need_grad:
+            ctx.save_for_backward(r[1])
+        return r[0]
+
+    @staticmethod
+    def _refuse(X16, idx32, weight, bias):
+        """Raise the error of the check that failed."""
         F = X16.shape[1]
         K = weight.shape[1]
         if K % F != 0:
@@ -240,17 +220,8 @@ class FusedGatherLinear(torch.autograd.Function):
             raise ValueError(f"idx32 must be (B,), shape={tuple(idx32.shape)}")
         if weight.dim() != 2 or bias.dim() != 1 or bias.shape[0] != weight.shape[0]:
             raise ValueError("weight must be (N,K) and bias (N,)")
-        Bsz = idx32.numel()
-        N = weight.shape[0]
-        C = torch.empty(Bsz, N, device=X16.device, dtype=torch.bfloat16)
-        need_grad = any(ctx.needs_input_grad)
-        # Xg only serves the backward (dW); inference skips the write-out.
-        Xg = torch.empty(Bsz, K, device=X16.device, dtype=torch.bfloat16) if need_grad else None
-        call("fx_linear_fwd", ptr(X16), F, ptr(idx32), F, X16.shape[0], ptr(weight), ptr(bias),
-             ptr(C), None, ptr(Xg), Bsz, N, K, 0, stream_of(X16))
-        if need_grad:
-            ctx.save_for_backward(Xg)
-        return C
+        raise ValueError(f"invalid shapes: X16 {tuple(X16.shape)}, idx32 {tuple(idx32.shape)}, "
+                         f"weight {tuple(weight.shape)}, bias {tuple(bias.shape)}")
 
     @staticmethod
     def backward(ctx, g):
@@ -290,11 +261,7 @@ class FusedLinear(torch.autograd.Function):
         x2 = x.reshape(-1, K)
         if x2.stride(1) != 1 or x2.stride(0) % 8 or x2.data_ptr() % 16:
             x2 = x2.contiguous()
-        M = x2.shape[0]
-        y = torch.empty(M, N, device=x.device, dtype=torch.bfloat16)
-        h = torch.empty_like(y) if (act and any(ctx.needs_input_grad)) else None
-        call("fx_linear_fwd", ptr(x2), x2.stride(0), None, 0, 0, ptr(weight), ptr(bias), ptr(y),
-             ptr(h), None, M, N, K, act, stream_of(x))
+        y, h = host.linear_fwd(x2, weight, bias, act, bool(act and any(ctx.needs_input_grad)))
         ctx.save_for_backward(x2, weight, h)
         ctx.act, ctx.has_bias, ctx.xshape = act, bias is not None, x.shape
         return y.view(*x.shape[:-1], N)
@@ -346,10 +313,7 @@ class FusedMLP(torch.autograd.Function):
             raise ValueError("weights must be contiguous")
         x2 = _rows(x)
         M, Fh = x2.shape[0], w1.shape[0]
-        u = torch.empty(M, Fh, device=x.device, dtype=torch.bfloat16)
-        gd = torch.empty_like(u) if any(ctx.needs_input_grad) else None
-        call("fx_linear_fwd", ptr(x2), x2.stride(0), None, 0, 0, ptr(w1), None, ptr(u), ptr(gd), None,
-             M, Fh, K, 2, stream_of(x))
+        u, gd = host.linear_fwd(x2, w1, None, 2, any(ctx.needs_input_grad))
         N = w2.shape[0]
         if native_fwd(M, N, Fh) and w2.data_ptr() % 16 == 0:
             y = _native_fwd(u, w2)

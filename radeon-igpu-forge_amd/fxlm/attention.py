@@ -11,7 +11,7 @@ import math
 
 import torch
 
-from fxgpu.abi import call, fxAttnArgs, fxAttnDecodeArgs, lib, stream_of
+from fxgpu.abi import call, host, fxAttnArgs, fxAttnDecodeArgs, lib, stream_of
 
 
 def _check_qkv(q, k, v):
@@ -88,7 +88,10 @@ class _FlashAttn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, q, k, v, causal, scale):
-        o, lse = _fwd(q, k, v, causal, scale)
+        r = host.attn_fwd(q, k, v, causal, scale)
+        if r is None:
+            r = _fwd(q, k, v, causal, scale)
+        o, lse = r
         ctx.save_for_backward(q, k, v, o, lse)
         ctx.causal, ctx.scale = causal, scale
         return o
@@ -96,12 +99,7 @@ class _FlashAttn(torch.autograd.Function):
     @staticmethod
     def backward(ctx, do):
         q, k, v, o, lse = ctx.saved_tensors
-        B, T, H, Dh = q.shape
-        dq = torch.empty(B, T, H, Dh, device=q.device, dtype=torch.bfloat16)
-        dk = torch.empty_like(dq)
-        dv = torch.empty_like(dq)
-        _bwd(q, k, v, o, lse, do, ctx.causal, ctx.scale, dq, dk, dv)
-        return dq, dk, dv, None, None
+        return *host.attn_bwd(q, k, v, o, lse, do, ctx.causal, ctx.scale), None, None
 
 
 class _FlashAttnQKV(torch.autograd.Function):
@@ -109,12 +107,14 @@ class _FlashAttnQKV(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, qkv, causal, scale):
-        if qkv.dim() != 5 or qkv.shape[2] != 3:
-            raise ValueError(f"qkv must be (B,T,3,H,Dh), got {tuple(qkv.shape)}")
-        if not qkv.is_contiguous():
-            raise ValueError("qkv must be contiguous")
-        q, k, v = qkv[:, :, 0], qkv[:, :, 1], qkv[:, :, 2]
-        o, lse = _fwd(q, k, v, causal, scale)
+        r = host.attn_fwd_qkv(qkv, causal, scale)
+        if r is None:
+            if qkv.dim() != 5 or qkv.shape[2] != 3:
+                raise ValueError(f"qkv must be (B,T,3,H,Dh), got {tuple(qkv.shape)}")
+            if not qkv.is_contiguous():
+                raise ValueError("qkv must be contiguous")
+            r = _fwd(qkv[:, :, 0], qkv[:, :, 1], qkv[:, :, 2], causal, scale)
+        o, lse = r
         ctx.save_for_backward(qkv, o, lse)
         ctx.causal, ctx.scale = causal, scale
         return o
@@ -122,10 +122,7 @@ class _FlashAttnQKV(torch.autograd.Function):
     @staticmethod
     def backward(ctx, do):
         qkv, o, lse = ctx.saved_tensors
-        dqkv = torch.empty_like(qkv)
-        _bwd(qkv[:, :, 0], qkv[:, :, 1], qkv[:, :, 2], o, lse, do, ctx.causal, ctx.scale,
-             dqkv[:, :, 0], dqkv[:, :, 1], dqkv[:, :, 2])
-        return dqkv, None, None
+        return host.attn_bwd_qkv(qkv, o, lse, do, ctx.causal, ctx.scale), None, None
 
 
 def flash_attention(q, k, v, causal=True, scale=None):

@@ -19,11 +19,9 @@ n_valid counts targets != ignore_index (out-of-range targets count, but their
 rows get no loss and no gradient); n_valid == 0 gives loss 0 (reference
 behaviour, ml/fxlm/cross_entropy.py:41-44 and ml/fxlm/kernels/ce.hip:43).
 """
-import ctypes
-
 import torch
 
-from fxgpu.abi import call, fxCEArgs, lib, ptr, stream_of
+from fxgpu.abi import call, host, lib, ptr, stream_of
 from fxgpu.fused_linear import linear_wgrad
 
 # rows per linear-CE chunk: bound the chunk's bf16 logits to this many bytes
@@ -32,41 +30,18 @@ _CHUNK_BYTES = 2 << 30
 
 def _inv_nvalid(target, ignore_index, grad_scale=None):
     """(inv_n, mul) device scalars: inv_n = 1/n_valid (0 if none), mul = inv_n*grad_scale."""
-    dev = target.device
-    inv_n = torch.empty((), device=dev, dtype=torch.float32)
-    mul = torch.empty((), device=dev, dtype=torch.float32)
-    gs_ptr, gs_val = None, 1.0
     if torch.is_tensor(grad_scale):
-        gs_t = grad_scale.detach().to(device=dev, dtype=torch.float32).reshape(())
-        gs_ptr = ptr(gs_t)
-    elif grad_scale is not None:
-        gs_val = float(grad_scale)
-    call("fx_ce_inv_nvalid", ptr(target), target.numel(), int(ignore_index), gs_ptr,
-         float(gs_val), ptr(inv_n), ptr(mul), stream_of(target))
-    return inv_n, mul
+        return host.ce_inv_nvalid(target, ignore_index, grad_scale, 1.0)
+    return host.ce_inv_nvalid(target, ignore_index, None, 1.0 if grad_scale is None else float(grad_scale))
 
 
 def _ce_rows(logits, target, grad, row_loss, mul, ignore_index):
     """One launch over the rows of (C, V) logits: per-row loss and, if grad, dlogits."""
-    N, V = logits.shape
-    a = fxCEArgs()
-    a.logits = logits.data_ptr()
-    a.target = target.data_ptr()
-    a.grad = grad.data_ptr() if grad is not None else None
-    a.row_loss = row_loss.data_ptr()
-    a.mul = mul.data_ptr()
-    a.N, a.V = N, V
-    a.ld = logits.stride(0)
-    a.ldg = grad.stride(0) if grad is not None else V
-    a.ignore_index = int(ignore_index)
-    call("fx_ce_fwd_grad", ctypes.byref(a), stream_of(logits))
+    host.ce_rows(logits, target, grad, row_loss, mul, ignore_index)
 
 
 def _finalize(row_loss, inv_n):
-    loss = torch.empty((), device=row_loss.device, dtype=torch.float32)
-    call("fx_ce_loss_finalize", ptr(row_loss), row_loss.numel(), ptr(inv_n), ptr(loss),
-         stream_of(row_loss))
-    return loss
+    return host.ce_finalize(row_loss, inv_n)
 
 
 # Fused linear-CE head (fx_lce_fwd / fx_lce_grad), where fx_lce_workspace takes the shape.
@@ -131,21 +106,16 @@ def _check_logits(logits, target):
 class _FusedCE(torch.autograd.Function):
     @staticmethod
     def forward(ctx, logits, target, ignore_index):
-        _check_logits(logits, target)
-        N, V = logits.shape
-        dev = logits.device
-        inv_n, mul = _inv_nvalid(target, ignore_index)
-        row_loss = torch.empty(N, device=dev, dtype=torch.float32)
-        grad = None
-        if ctx.needs_input_grad[0]:
-            grad = torch.empty(N, V, device=dev, dtype=torch.bfloat16)
-        _ce_rows(logits, target, grad, row_loss, mul, ignore_index)
+        r = host.ce_fwd(logits, target, ignore_index, ctx.needs_input_grad[0])
+        if r is None:
+            _check_logits(logits, target)
+        loss, grad = r
         ctx.save_for_backward(grad)
         # the first backward's kernel takes the multiplier in grad as written to be 1
         # (src -1) and stores its g in applied[1]
-        ctx.applied = torch.empty(2, device=dev, dtype=torch.float32)
+        ctx.applied = torch.empty(2, device=logits.device, dtype=torch.float32)
         ctx.calls = 0
-        return _finalize(row_loss, inv_n)
+        return loss
 
     @staticmethod
     def backward(ctx, g):
@@ -155,8 +125,7 @@ class _FusedCE(torch.autograd.Function):
         if ctx.calls == 1:
             # the usual single backward: scale the saved dlogits in place (no pass at all
             # when g == 1) and hand them over
-            call("fx_ce_scale_grad", ptr(grad), grad.numel(), ptr(g32), ptr(ctx.applied), -1,
-                 stream_of(grad))
+            host.ce_scale_grad(grad, g32, ctx.applied, -1)
             return grad, None, None
         # a further backward through a retained graph: a fresh tensor, so the gradient the
         # first backward returned stays as it was
@@ -247,8 +216,7 @@ class _LinearCE(torch.autograd.Function):
                 # the usual single backward (one chunk, so dW is the bf16 product): scale the
                 # saved gradients in place and hand them over; in the training step the
                 # factor g / grad_scale is exactly 1 and the kernel makes no pass at all
-                call("fx_ce_lin_grad_scale_inplace", ptr(dW), dW.numel(), ptr(dx), dx.numel(), ptr(g32),
-                     ptr(gs_t), inv_value, stream_of(dx))
+                host.ce_lin_scale_inplace(dW, dx, g32, gs_t, inv_value)
                 ctx.first = (g32, gs_t, inv_value)
                 return dx, dW, None, None, None, None
             if dW.dtype == torch.bfloat16:

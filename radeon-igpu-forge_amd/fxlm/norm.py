@@ -8,7 +8,7 @@ gradients of x are summed inside that pass (fx_rms_norm_bwd_add).
 """
 import torch
 
-from fxgpu.abi import call, lib, ptr, stream_of
+from fxgpu.abi import call, host, lib, ptr, stream_of
 
 
 def _check(x, w):
@@ -33,55 +33,33 @@ def _al(t):
     return t if t.data_ptr() % 16 == 0 else t.clone()
 
 
+def _fwd(x, w, eps):
+    """(y, rstd, x, w): x and w as the kernels read them (an aligned copy where needed)."""
+    r = host.norm_fwd(x, w, eps)
+    if r is None:
+        _check(x, w)
+        x, w = _al(x), _al(w)
+        r = host.norm_fwd(x, w, eps)
+    return r[0], r[1], x, w
+
+
 class _RMSNorm(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, w, eps):
-        D = _check(x, w)
-        w = _al(w)
-        N = x.numel() // D
-        x2 = _al(x.view(N, D))
-        y = torch.empty_like(x2)
-        rstd = torch.empty(N, device=x.device, dtype=torch.float32)
-        call("fx_rms_norm_fwd", ptr(x2), ptr(w), ptr(y), ptr(rstd), N, D, float(eps),
-             stream_of(x))
-        ctx.save_for_backward(x2, w, rstd)
-        ctx.eps = eps
-        ctx.oshape = x.shape
-        return y.view(x.shape)
+        y, rstd, x, w = _fwd(x, w, eps)
+        ctx.save_for_backward(x, w, rstd)
+        return y
 
     @staticmethod
     def backward(ctx, dy):
-        x2, w, rstd = ctx.saved_tensors
-        dx, dw = _bwd_into(x2, dy, w, rstd)
-        return dx.view(ctx.oshape), dw, None
+        x, w, rstd = ctx.saved_tensors
+        dx, dw = host.norm_bwd(x, dy, w, rstd, None)
+        return dx, dw, None
 
 
 def rms_norm(x, weight, eps=1e-6):
     """x (..., D) bf16, weight (D,) bf16 -> y (..., D) bf16."""
     return _RMSNorm.apply(x, weight, float(eps))
-
-
-def _bwd_into(x2, dy, w, rstd, dres=None):
-    """(dx, dw) of the norm for x2 (N, D); dx += dres in the same pass when given."""
-    N, D = x2.shape
-    dy2 = _al(dy.contiguous().view(N, D))
-    if dy2.dtype != torch.bfloat16:
-        dy2 = dy2.to(torch.bfloat16)
-    dx = torch.empty_like(x2)
-    dw32 = torch.empty(D, device=x2.device, dtype=torch.float32)
-    dw = torch.empty(D, device=x2.device, dtype=w.dtype)
-    work = torch.empty(max(1, lib().fx_rms_norm_bwd_workspace(N, D) // 4), device=x2.device,
-                       dtype=torch.float32)
-    if dres is None:
-        call("fx_rms_norm_bwd", ptr(x2), ptr(dy2), ptr(w), ptr(rstd), ptr(dx), ptr(dw32),
-             ptr(dw), ptr(work), N, D, stream_of(x2))
-    else:
-        r2 = _al(dres.contiguous().view(N, D))
-        if r2.dtype != torch.bfloat16:
-            r2 = r2.to(torch.bfloat16)
-        call("fx_rms_norm_bwd_add", ptr(x2), ptr(dy2), ptr(r2), ptr(w), ptr(rstd), ptr(dx),
-             ptr(dw32), ptr(dw), ptr(work), N, D, stream_of(x2))
-    return dx, dw
 
 
 class _PreNorm(torch.autograd.Function):
@@ -92,26 +70,18 @@ class _PreNorm(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, w, eps):
-        D = _check(x, w)
-        w = _al(w)
-        N = x.numel() // D
-        x2 = _al(x.view(N, D))
-        y = torch.empty_like(x2)
-        rstd = torch.empty(N, device=x.device, dtype=torch.float32)
-        call("fx_rms_norm_fwd", ptr(x2), ptr(w), ptr(y), ptr(rstd), N, D, float(eps),
-             stream_of(x))
-        ctx.save_for_backward(x2, w, rstd)
-        ctx.oshape = x.shape
+        y, rstd, xa, w = _fwd(x, w, eps)
+        ctx.save_for_backward(xa, w, rstd)
         ctx.set_materialize_grads(False)
-        return x, y.view(x.shape)
+        return x, y
 
     @staticmethod
     def backward(ctx, dres, dy):
-        x2, w, rstd = ctx.saved_tensors
+        x, w, rstd = ctx.saved_tensors
         if dy is None:
             return dres, None, None
-        dx, dw = _bwd_into(x2, dy, w, rstd, dres)
-        return dx.view(ctx.oshape), dw, None
+        dx, dw = host.norm_bwd(x, dy, w, rstd, dres)
+        return dx, dw, None
 
 
 def pre_norm(x, weight, eps=1e-6):
@@ -128,29 +98,24 @@ class _AddPreNorm(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, r, w, eps):
-        D = _check(x, w)
-        if r.shape != x.shape or r.dtype != x.dtype or not r.is_contiguous():
-            raise ValueError(f"r must be a contiguous {tuple(x.shape)} {x.dtype} tensor")
-        w, r = _al(w), _al(r)
-        N = x.numel() // D
-        x2 = _al(x.view(N, D))
-        s = torch.empty_like(x2)
-        y = torch.empty_like(x2)
-        rstd = torch.empty(N, device=x.device, dtype=torch.float32)
-        call("fx_rms_norm_fwd_add", ptr(x2), ptr(r), ptr(w), ptr(s), ptr(y), ptr(rstd), N, D, float(eps),
-             stream_of(x))
+        got = host.norm_add_fwd(x, r, w, eps)
+        if got is None:
+            _check(x, w)
+            if r.shape != x.shape or r.dtype != x.dtype or not r.is_contiguous():
+                raise ValueError(f"r must be a contiguous {tuple(x.shape)} {x.dtype} tensor")
+            w = _al(w)
+            got = host.norm_add_fwd(_al(x), _al(r), w, eps)
+        s, y, rstd = got
         ctx.save_for_backward(s, w, rstd)
-        ctx.oshape = x.shape
         ctx.set_materialize_grads(False)
-        return s.view(x.shape), y.view(x.shape)
+        return s, y
 
     @staticmethod
     def backward(ctx, ds, dy):
         s, w, rstd = ctx.saved_tensors
         if dy is None:
             return ds, ds, None, None
-        dx, dw = _bwd_into(s, dy, w, rstd, ds)
-        dx = dx.view(ctx.oshape)
+        dx, dw = host.norm_bwd(s, dy, w, rstd, ds)
         return dx, dx, dw, None
 
 

@@ -8,11 +8,9 @@ computes with (``p.data`` becomes a view of it).  ``step()`` is one C-ABI call
 / loss-scale update -> flat AdamW with the bf16 write-back.  No host sync and
 no host-to-device copy.
 """
-import ctypes
-
 import torch
 
-from fxgpu.abi import MAX_TENSORS, call, fxAdamWState, fxTensorList, lib, stream_of
+from fxgpu.abi import MAX_TENSORS, fxAdamWState, fxTensorList, host
 
 
 def _align8(n):
@@ -67,6 +65,9 @@ class FlatAdamW:
         self.scale = torch.full((), float(init_scale), device=dev, dtype=torch.float32)
         self._growth = torch.zeros((), device=dev, dtype=torch.int32)
         self._work = torch.empty(0, device=dev, dtype=torch.float32)
+        self._params = [p for _n, p, _o, _el, _w in self._info]
+        self._layout = host.FlatLayout([i[2] for i in self._info], [i[3] for i in self._info],
+                                       [i[4] for i in self._info])
 
     # -- helpers -------------------------------------------------------------
 
@@ -105,12 +106,14 @@ class FlatAdamW:
 
     def step(self, lr=None):
         lr_v = self.lr if lr is None else float(lr)
-        lists, nl, _keep = self._lists()   # _keep holds contiguous grad copies alive
-        need = lib().fx_adamw_workspace(lists, nl) // 4
-        if self._work.numel() < need:
-            self._work = torch.empty(need, device=self.master.device, dtype=torch.float32)
-        st = self._state(lr_v, self._work.data_ptr())
-        call("fx_adamw_step", ctypes.byref(st), lists, nl, stream_of(self.master))
+        self._work, bad = host.adamw_step(
+            self._layout, self._params,
+            [self.master, self.m, self.v, self.flat16, self._step_ctr, self._found_inf, self._norm, self.scale,
+             self._growth],
+            [lr_v, self.betas[0], self.betas[1], self.eps, self.weight_decay, self.max_grad_norm,
+             self.growth_interval], self._work)
+        if bad != -1:
+            self._lists()   # raises the error of the gradient that was refused
         return {"grad_norm": self._norm, "found_inf": self._found_inf, "scale": self.scale}
 
     def _state(self, lr_v, work):

@@ -1,0 +1,67 @@
+"""The op wrappers' host module on the GPU: what the autograd functions around it still do
+(saved-tensor hooks, side streams, refusals) and the optimiser's copies."""
+import copy
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _block(dev):
+    from fxlm.model import Block, GPTConfig
+    torch.manual_seed(0)
+    return Block(GPTConfig(vocab_size=64, seq_len=64, n_layer=1, n_head=2, d_model=128)).to(dev).bfloat16()
+
+
+def _grads(block, x, dy):
+    out = block(x)
+    return [out, *torch.autograd.grad(out, [x, *block.parameters()], dy)]
+
+
+def test_block_through_saved_tensor_hooks_and_a_side_stream(dev):
+    block = _block(dev)
+    x = torch.randn(4, 64, 128, device=dev).bfloat16().requires_grad_()
+    dy = torch.randn(4, 64, 128, device=dev).bfloat16()
+    ref = _grads(block, x, dy)
+    with torch.autograd.graph.save_on_cpu():
+        assert all(torch.equal(a, b) for a, b in zip(ref, _grads(block, x, dy)))
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        got = _grads(block, x, dy)
+    torch.cuda.current_stream().wait_stream(s)
+    assert all(torch.equal(a, b) for a, b in zip(ref, got))
+
+
+def test_misaligned_and_refused_inputs(dev):
+    from fxlm.attention import flash_attention
+    from fxlm.norm import add_pre_norm, rms_norm
+    w = torch.ones(64, device=dev).bfloat16()
+    flat = torch.randn(3 + 10 * 64, device=dev).bfloat16()
+    x = flat[3:].view(10, 64)                              # contiguous, 6 bytes past an aligned address
+    assert torch.equal(rms_norm(x, w), rms_norm(x.clone(), w))
+    assert all(torch.equal(a, b) for a, b in zip(add_pre_norm(x, x, w), add_pre_norm(x.clone(), x.clone(), w)))
+    with pytest.raises(TypeError, match="must be bfloat16"):
+        rms_norm(x.float(), w)
+    with pytest.raises(ValueError, match="contiguous"):
+        rms_norm(torch.randn(64, 64, device=dev).bfloat16().t(), w)
+    q = torch.randn(1, 8, 2, 64, device=dev).bfloat16()
+    with pytest.raises(TypeError, match="q must be bfloat16"):
+        flash_attention(q.float(), q.float(), q.float())
+    with pytest.raises(ValueError, match="share one 4-D shape"):
+        flash_attention(q, q[:, :4], q)
+    with pytest.raises(ValueError, match="must be positive"):   # the library's own check
+        flash_attention(q, q, q, scale=-1.0)
+
+
+def test_optimizer_deepcopy_takes_the_same_step(dev):
+    from fxlm.optim import FlatAdamW
+    model = torch.nn.Linear(64, 40).to(dev)
+    opt = FlatAdamW(model, init_scale=1.0)
+    twin_model, twin = copy.deepcopy((model, opt))
+    for m, o in ((model, opt), (twin_model, twin)):
+        for p in m.parameters():
+            p.grad = torch.ones_like(p)
+        o.step()
+    assert torch.equal(opt.master, twin.master) and float(opt._step_ctr) == 1
