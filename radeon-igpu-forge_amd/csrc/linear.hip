@@ -1407,14 +1407,104 @@ __device__ __forceinline__ const uint16_t* xrow_base(const GemmArgs& a, int m) {
     return a.A + (int64_t)m * a.lda;
 }
 
+static constexpr int skinny_batch(int nt, int mt, bool norm) {
+    return nt * mt >= 8 && norm ? 1 : nt * mt >= (norm ? 3 : 4) ? 2 : nt * mt == 1 && !norm ? 8 : 4;
+}
+
+// 16 bytes at p, or zeros
+__device__ __forceinline__ uint4 ld16_if(bool ok, const uint16_t* p) {
+    uint4 v = make_uint4(0u, 0u, 0u, 0u);
+    if (ok) v = ld16(p);
+    return v;
+}
+
+// sum over the sw waves' partials (stride `vals` floats), in wave order; four at a time so that
+// their LDS reads overlap
+__device__ __forceinline__ float skinny_sum(const float* p, int vals, int sw) {
+    float sum = 0.f;
+    int w = 0;
+    for (; w + 4 <= sw; w += 4) {
+        const float v0 = p[w * vals], v1 = p[(w + 1) * vals], v2 = p[(w + 2) * vals], v3 = p[(w + 3) * vals];
+        sum += v0;
+        sum += v1;
+        sum += v2;
+        sum += v3;
+    }
+    for (; w < sw; ++w) sum += p[w * vals];
+    return sum;
+}
+
+// bias, activation, residual and the store of one output value
+__device__ __forceinline__ void skinny_store(const GemmArgs& a, float sum, int m, int n) {
+    const float h = sum + (a.bias ? bf16_to_f32(a.bias[n]) : 0.f);
+    float y = h;
+    if (a.act == 2) {
+        float d;
+        gelu_tanh_and_grad(h, y, d);
+        if (a.H) a.H[(int64_t)m * a.ldh + n] = f32_to_bf16(d);
+    } else {
+        if (a.H) a.H[(int64_t)m * a.ldh + n] = f32_to_bf16(h);
+        if (a.act == 1) y = gelu_tanh(h);
+    }
+    if (a.res) y += bf16_to_f32(a.res[(int64_t)m * a.ldres + n]);
+    a.C[(int64_t)m * a.ldc + n] = f32_to_bf16(y);
+}
+
+// rstd of the rows of X from the operands of one batch that spans each wave's K range: the sum
+// of squares over a wave's lanes, then over the waves in order.  `red` is scratch (free again
+// after the call's last barrier).
+template <int U, int MT>
+__device__ __forceinline__ void skinny_rstd(const GemmArgs& a, const uint4 (&xv)[U][MT], float* red, int sw, int w, int lane,
+                                            float (&rs)[MT]) {
+    const int r = lane & 15, kg = lane >> 4;
+#pragma unroll
+    for (int j = 0; j < MT; ++j) {
+        float q = 0.f;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            float f[8];
+            unpack8(xv[u][j], f);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) q = fmaf(f[e], f[e], q);
+        }
+        q += __shfl_xor(q, 16, 64);
+        q += __shfl_xor(q, 32, 64);
+        if (kg == 0) red[w * (16 * MT) + 16 * j + r] = q;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < MT; ++j) {
+        const float q = skinny_sum(red + 16 * j + r, 16 * MT, sw);
+        rs[j] = 16 * j + r < a.M ? 1.f / sqrtf(q / (float)a.K + a.eps) : 0.f;
+    }
+    __syncthreads();
+}
+
+// x * rstd * nw of one K step, rounded to bf16 as the norm kernel writes them
+template <int MT>
+__device__ __forceinline__ void skinny_normalise(uint4 (&xv)[MT], const uint4& nv, const float (&rs)[MT]) {
+    float fw[8];
+    unpack8(nv, fw);
+#pragma unroll
+    for (int j = 0; j < MT; ++j) {
+        float f[8];
+        unpack8(xv[j], f);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) f[e] = f[e] * rs[j] * fw[e];
+        xv[j] = pack8(f);
+    }
+}
+
 template <int NT, int MT, bool NORM>
-__global__ void __launch_bounds__(1024) gemm_skinny_kernel(GemmArgs a, int sw) {
-    constexpr int U = NT * MT >= 4 ? 2 : 4;  // K steps per load batch
+__global__ void __launch_bounds__(1024) gemm_skinny_kernel(GemmArgs a, int sw, int tr) {
+    // K steps per load batch: as many as the 128 registers of 16 waves hold (one round trip to
+    // memory per batch; most layers' waves have a single one)
+    constexpr int U = skinny_batch(NT, MT, NORM);
     __shared__ __attribute__((aligned(16))) float red[kSKMaxTiles * 256];
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r = lane & 15, kg = lane >> 4;
-    const int n0 = blockIdx.x * 16 * NT;
+    const int n0 = blockIdx.x * tr * NT;
     const int ks = (a.K + 31) / 32;
     const int kb = w * ks / sw, ke = (w + 1) * ks / sw;
 
@@ -1422,7 +1512,7 @@ __global__ void __launch_bounds__(1024) gemm_skinny_kernel(GemmArgs a, int sw) {
 #pragma unroll
     for (int i = 0; i < NT; ++i) {
         const int n = n0 + 16 * i + r;
-        wrow[i] = n < a.N ? a.B + (int64_t)n * a.ldb + 8 * kg : nullptr;
+        wrow[i] = n < a.N && r < tr ? a.B + (int64_t)n * a.ldb + 8 * kg : nullptr;
     }
     const uint16_t* xrow[MT];
 #pragma unroll
@@ -1432,29 +1522,60 @@ __global__ void __launch_bounds__(1024) gemm_skinny_kernel(GemmArgs a, int sw) {
         xrow[j] = row ? row + 8 * kg : nullptr;
     }
     const bool wxg = a.Xg != nullptr && blockIdx.x == 0;
+    uint4 wv[U][NT], xv[U][MT], nv[NORM ? U : 1];
+    auto load = [&](int s0) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int s = s0 + u;
+            const bool ok = s < ke && s * 32 + 8 * kg < a.K;
+#pragma unroll
+            for (int i = 0; i < NT; ++i) wv[u][i] = ld16_if(ok && wrow[i], wrow[i] + s * 32);
+#pragma unroll
+            for (int j = 0; j < MT; ++j) xv[u][j] = ld16_if(ok && xrow[j], xrow[j] + s * 32);
+            if constexpr (NORM) nv[u] = ld16_if(ok, a.nw + s * 32 + 8 * kg);
+        }
+    };
+    load(kb);
 
     // NORM: A rows are RMS-normalised on the fly, x * rstd[m] * nw[k] rounded to bf16 as
-    // the norm kernel writes them.  Each workgroup first computes rstd of every row: wave
-    // v sums rows v, v + sw, ... (lane partials, then a butterfly: a fixed order).
+    // the norm kernel writes them.  Each workgroup first computes rstd of every row.  Where the
+    // first batch is a wave's whole K range (the host asks for that many waves when it can), the
+    // squares come from the operands just loaded: lanes, then waves, in a fixed order, and no
+    // second read of x (a 768 x 2304 product of 16 rows 6.4 -> 4.7 us, 4.0 without the norm).
+    // Otherwise wave v sums rows v, v + sw, ..., four rows' loads issued at a time.
     __shared__ float srstd[kSKMaxM];
     float rs[MT];
     if constexpr (NORM) {
-        for (int m = w; m < a.M; m += sw) {
-            const uint16_t* row = xrow_base(a, m);
-            float q = 0.f;
-            if (row)
+        if ((ks + sw - 1) / sw <= U) {
+            skinny_rstd<U, MT>(a, xv, red, sw, w, lane, rs);
+        } else {
+            for (int mb = w; mb < a.M; mb += 4 * sw) {
+                const uint16_t* row[4];
+                float q[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int t = 0; t < 4; ++t) row[t] = mb + t * sw < a.M ? xrow_base(a, mb + t * sw) : nullptr;
                 for (int c = lane; c < a.K / 8; c += 64) {
-                    float f[8];
-                    unpack8(ld16(row + c * 8), f);
+                    uint4 v[4];
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) q = fmaf(f[e], f[e], q);
+                    for (int t = 0; t < 4; ++t) v[t] = ld16_if(row[t] != nullptr, row[t] + c * 8);
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) {
+                        float f[8];
+                        unpack8(v[t], f);
+#pragma unroll
+                        for (int e = 0; e < 8; ++e) q[t] = fmaf(f[e], f[e], q[t]);
+                    }
                 }
-            q = group_sum<64>(q);
-            if (lane == 0) srstd[m] = 1.f / sqrtf(q / (float)a.K + a.eps);
-        }
-        __syncthreads();
 #pragma unroll
-        for (int j = 0; j < MT; ++j) rs[j] = 16 * j + r < a.M ? srstd[16 * j + r] : 0.f;
+                for (int t = 0; t < 4; ++t) {
+                    const float sum = group_sum<64>(q[t]);
+                    if (lane == 0 && mb + t * sw < a.M) srstd[mb + t * sw] = 1.f / sqrtf(sum / (float)a.K + a.eps);
+                }
+            }
+            __syncthreads();
+#pragma unroll
+            for (int j = 0; j < MT; ++j) rs[j] = 16 * j + r < a.M ? srstd[16 * j + r] : 0.f;
+        }
     }
 
     f32x4 acc[NT][MT];
@@ -1462,30 +1583,11 @@ __global__ void __launch_bounds__(1024) gemm_skinny_kernel(GemmArgs a, int sw) {
     for (int i = 0; i < NT; ++i)
 #pragma unroll
         for (int j = 0; j < MT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const uint4 zero = make_uint4(0u, 0u, 0u, 0u);
     for (int s0 = kb; s0 < ke; s0 += U) {
-        uint4 wv[U][NT], xv[U][MT];
+        if (s0 > kb) load(s0);
+        if constexpr (NORM) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int s = s0 + u;
-            const bool ok = s < ke && s * 32 + 8 * kg < a.K;
-#pragma unroll
-            for (int i = 0; i < NT; ++i) wv[u][i] = ok && wrow[i] ? ld16(wrow[i] + s * 32) : zero;
-#pragma unroll
-            for (int j = 0; j < MT; ++j) xv[u][j] = ok && xrow[j] ? ld16(xrow[j] + s * 32) : zero;
-            if constexpr (NORM) {
-                const uint4 wn = ok ? ld16(a.nw + s * 32 + 8 * kg) : zero;
-                float fw[8];
-                unpack8(wn, fw);
-#pragma unroll
-                for (int j = 0; j < MT; ++j) {
-                    float f[8];
-                    unpack8(xv[u][j], f);
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) f[e] = f[e] * rs[j] * fw[e];
-                    xv[u][j] = pack8(f);
-                }
-            }
+            for (int u = 0; u < U; ++u) skinny_normalise<MT>(xv[u], nv[u], rs);
         }
         if (wxg) {
 #pragma unroll
@@ -1519,46 +1621,131 @@ __global__ void __launch_bounds__(1024) gemm_skinny_kernel(GemmArgs a, int sw) {
     for (int v = threadIdx.x; v < kVals; v += blockDim.x) {
         const int tile = v >> 8, ml = (v >> 4) & 15, nl = v & 15;
         const int off = tile * 256 + (ml + 16 * (nl >> 2)) * 4 + (nl & 3);
-        float sum = 0.f;
-        for (int ww = 0; ww < sw; ++ww) sum += red[ww * kVals + off];
         const int n = n0 + 16 * (tile / MT) + nl, m = 16 * (tile % MT) + ml;
-        if (n < a.N && m < a.M) {
-            const float h = sum + (a.bias ? bf16_to_f32(a.bias[n]) : 0.f);
-            float y = h;
-            if (a.act == 2) {
-                float d;
-                gelu_tanh_and_grad(h, y, d);
-                if (a.H) a.H[(int64_t)m * a.ldh + n] = f32_to_bf16(d);
-            } else {
-                if (a.H) a.H[(int64_t)m * a.ldh + n] = f32_to_bf16(h);
-                if (a.act == 1) y = gelu_tanh(h);
-            }
-            if (a.res) y += bf16_to_f32(a.res[(int64_t)m * a.ldres + n]);
-            a.C[(int64_t)m * a.ldc + n] = f32_to_bf16(y);
+        if (n < a.N && m < a.M && nl < tr) skinny_store(a, skinny_sum(red + off, kVals, sw), m, n);
+    }
+}
+
+// The same product for a wide W (a head: 50,304 rows of 768): a workgroup keeps its X operands
+// (normalised once) in registers and walks the 16-row tiles of W, the next tile's rows loading
+// during the current one's products and sums.  One workgroup per tile read X and summed its
+// squares 1,572 times over: 40 us for 16 rows, 26 this way (3 TB/s of W).  Every wave's K
+// range is one batch of kSKLoopU steps (the host checks); the partial tiles alternate between
+// two LDS buffers, so a tile costs one barrier.
+constexpr int kSKLoopU = 4;
+template <int MT, bool NORM>
+__global__ void __launch_bounds__(1024) gemm_skinny_loop_kernel(GemmArgs a, int sw, int ntiles) {
+    constexpr int U = kSKLoopU, kVals = MT * 256;
+    extern __shared__ __attribute__((aligned(16))) float lred[];   // 2 x sw x kVals
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = lane & 15, kg = lane >> 4;
+    const int ks = (a.K + 31) / 32;
+    const int kb = w * ks / sw, ke = (w + 1) * ks / sw;
+    uint4 wv[U], xv[U][MT];
+    auto load_w = [&](int t) {
+        const int n = 16 * t + r;
+        const uint16_t* row = a.B + (int64_t)(n < a.N ? n : 0) * a.ldb + 8 * kg;
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            wv[u] = ld16_if(t < ntiles && n < a.N && kb + u < ke && (kb + u) * 32 + 8 * kg < a.K, row + (kb + u) * 32);
+    };
+    load_w(blockIdx.x);
+#pragma unroll
+    for (int j = 0; j < MT; ++j) {
+        const int m = 16 * j + r;
+        const uint16_t* row = a.A + (int64_t)(m < a.M ? m : 0) * a.lda + 8 * kg;
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            xv[u][j] = ld16_if(m < a.M && kb + u < ke && (kb + u) * 32 + 8 * kg < a.K, row + (kb + u) * 32);
+    }
+    if constexpr (NORM) {
+        uint4 nv[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            nv[u] = ld16_if(kb + u < ke && (kb + u) * 32 + 8 * kg < a.K, a.nw + (kb + u) * 32 + 8 * kg);
+        float rs[MT];
+        skinny_rstd<U, MT>(a, xv, lred, sw, w, lane, rs);
+#pragma unroll
+        for (int u = 0; u < U; ++u) skinny_normalise<MT>(xv[u], nv[u], rs);
+    }
+    int p = 0;
+    for (int t = blockIdx.x; t < ntiles; t += gridDim.x, p ^= 1) {
+        f32x4 acc[MT];
+#pragma unroll
+        for (int j = 0; j < MT; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int j = 0; j < MT; ++j) acc[j] = mfma16(wv[u], xv[u][j], acc[j]);
+        load_w(t + gridDim.x);
+        float* red = lred + p * sw * kVals;
+#pragma unroll
+        for (int j = 0; j < MT; ++j) *reinterpret_cast<f32x4*>(&red[(w * MT + j) * 256 + lane * 4]) = acc[j];
+        __syncthreads();
+        for (int v = threadIdx.x; v < kVals; v += blockDim.x) {
+            const int tile = v >> 8, ml = (v >> 4) & 15, nl = v & 15;
+            const int off = tile * 256 + (ml + 16 * (nl >> 2)) * 4 + (nl & 3);
+            const int n = 16 * t + nl, m = 16 * tile + ml;
+            if (n < a.N && m < a.M) skinny_store(a, skinny_sum(red + off, kVals, sw), m, n);
         }
     }
+}
+
+template <int MT, bool NORM>
+static int skinny_loop_launch(const GemmArgs& a, int sw, hipStream_t st) {
+    const int64_t ntiles = ((int64_t)a.N + 15) / 16, cus = device_cus();
+    const int64_t per = (ntiles + 2 * cus - 1) / (2 * cus);
+    hipLaunchKernelGGL((gemm_skinny_loop_kernel<MT, NORM>), dim3((unsigned)((ntiles + per - 1) / per)), dim3(64 * sw),
+                       2 * sw * MT * 256 * sizeof(float), st, a, sw, (int)ntiles);
+    return check_launch("gemm_skinny_loop");
 }
 
 template <int NT, bool NORM>
 static int skinny_launch(const GemmArgs& a, hipStream_t st) {
     const int mt = (a.M + 15) / 16;
-    const int64_t nblk = ((int64_t)a.N + 16 * NT - 1) / (16 * NT);
-    const int64_t ks = (a.K + 31) / 32;
-    const int64_t target = 4LL * device_cus();  // waves
+    const int64_t cus = device_cus(), ks = (a.K + 31) / 32;
+    // A narrow layer's tiles take 8 or 4 rows of W (the MFMA's other rows are zeros) until half
+    // the CUs have one: a workgroup's bytes, not the MFMAs, set its time (768 x 3072 of 16 rows,
+    // 98 KB of W and 98 KB of X in each of 48 workgroups: 9.0 -> 7.5 us; 768 x 768 4.1 -> 3.8).
+    // 144 tiles of 2304 x 768 stay whole (5.5 us, 6.5 in 288 halves).
+    int tr = 16;
+    while (NT == 1 && tr > 4 && ((int64_t)a.N + tr - 1) / tr * 2 < cus) tr /= 2;
+    const int64_t nblk = ((int64_t)a.N + tr * NT - 1) / (tr * NT);
+    const int64_t target = 4 * cus;  // waves
+    // with the norm, as many waves as make a wave's K range one batch, where LDS allows
+    const int64_t want = NORM ? (ks + skinny_batch(NT, mt, true) - 1) / skinny_batch(NT, mt, true) : 1;
     int sw = 1;
-    while (sw < 16 && nblk * sw < target && 2 * sw <= ks && 2 * sw * NT * mt <= kSKMaxTiles) sw *= 2;
+    while (sw < 16 && (nblk * sw < target || sw < want) && 2 * sw <= ks && 2 * sw * NT * mt <= kSKMaxTiles) sw *= 2;
     const dim3 grid((unsigned)nblk), block(64 * sw);
     switch (mt) {
-        case 1: hipLaunchKernelGGL((gemm_skinny_kernel<NT, 1, NORM>), grid, block, 0, st, a, sw); break;
-        case 2: hipLaunchKernelGGL((gemm_skinny_kernel<NT, 2, NORM>), grid, block, 0, st, a, sw); break;
-        case 3: hipLaunchKernelGGL((gemm_skinny_kernel<NT, 3, NORM>), grid, block, 0, st, a, sw); break;
-        default: hipLaunchKernelGGL((gemm_skinny_kernel<NT, 4, NORM>), grid, block, 0, st, a, sw); break;
+        case 1: hipLaunchKernelGGL((gemm_skinny_kernel<NT, 1, NORM>), grid, block, 0, st, a, sw, tr); break;
+        case 2: hipLaunchKernelGGL((gemm_skinny_kernel<NT, 2, NORM>), grid, block, 0, st, a, sw, tr); break;
+        case 3: hipLaunchKernelGGL((gemm_skinny_kernel<NT, 3, NORM>), grid, block, 0, st, a, sw, tr); break;
+        default: hipLaunchKernelGGL((gemm_skinny_kernel<NT, 4, NORM>), grid, block, 0, st, a, sw, tr); break;
     }
     return check_launch("gemm_skinny");
 }
 
-// two W row tiles per workgroup once there are enough workgroups (fewer re-reads of X)
+template <bool NORM>
+static int skinny_loop(const GemmArgs& a, int sw, hipStream_t st) {
+    const int mt = (a.M + 15) / 16;
+    if (mt == 1) return skinny_loop_launch<1, NORM>(a, sw, st);
+    if (NORM || mt == 2) return skinny_loop_launch<2, NORM>(a, sw, st);
+    return mt == 3 ? skinny_loop_launch<3, false>(a, sw, st) : skinny_loop_launch<4, false>(a, sw, st);
+}
+
+// the walking kernel from four 16-row tiles of W per CU on, where 16 waves hold K in one batch
+// each (and with the norm X fits the registers beside it); else two W row tiles per workgroup once there are enough workgroups (fewer re-reads
+// of X)
 static int linear_skinny(const GemmArgs& a, hipStream_t st) {
+    const int64_t ks = (a.K + 31) / 32;
+    if (((int64_t)a.N + 15) / 16 >= 4LL * device_cus() && ks <= 16 * kSKLoopU && !a.idx && !a.Xg &&
+        !(a.nw && a.M > 32)) {
+        int sw = 4;
+        while (sw < 16 && sw * kSKLoopU < ks) sw *= 2;
+        return a.nw ? skinny_loop<true>(a, sw, st) : skinny_loop<false>(a, sw, st);
+    }
     const bool two = (a.N + 31) / 32 >= 2LL * device_cus();
     if (a.nw) return two ? skinny_launch<2, true>(a, st) : skinny_launch<1, true>(a, st);
     return two ? skinny_launch<2, false>(a, st) : skinny_launch<1, false>(a, st);

@@ -670,3 +670,35 @@ def test_small_tile_dgrad_matches_whole_tiles(dev, monkeypatch, M, N, K, pad):
     monkeypatch.setenv("FX_GEMM_GENERAL", "m")
     assert all(torch.equal(a, b) for a, b in zip(small, run()))
     assert oracle_close(small[0], dy.float() @ W.float(), FRAC_OUT)
+
+
+@pytest.mark.parametrize("M,K,N,norm,res,act", [
+    (1, 8, 16400, True, False, None),             # the walking kernel: one K chunk, most waves without work
+    (17, 768, 16391, True, True, "gelu_tanh"),    # a last tile of 7 rows, two row tiles of X
+    (32, 2048, 16384, True, False, None),         # the deepest K: four steps in each of 16 waves
+    (33, 768, 16400, True, False, None),          # past its rows with the norm
+    (64, 520, 16400, False, True, None),          # four row tiles of X, a K tail of 8
+    (16, 2056, 16400, False, False, None),        # K past its registers
+    (16, 3072, 768, True, False, None),           # tiles of 4 rows; the norm in a second read of x
+    (5, 72, 3, False, True, "gelu_tanh"),         # less than one tile of 4 rows
+])
+def test_few_rows_tile_choices(dev, M, K, N, norm, res, act):
+    from fxgpu.fused_linear import linear_ex
+    g = torch.Generator(device=dev).manual_seed(M + K + N)
+
+    def rn(*s):
+        return torch.randn(*s, device=dev, generator=g)
+    x, W, b = rn(M, K).bfloat16(), (rn(N, K) * K ** -0.5).bfloat16(), (rn(N) * 0.1).bfloat16()
+    nw = (rn(K) * 0.1 + 1).bfloat16() if norm else None
+    r = (rn(M, N) * 0.5).bfloat16() if res else None
+    print(f"few rows M={M} K={K} N={N} norm={norm}", flush=True)
+    y = linear_ex(x, W, bias=b, residual=r, norm_weight=nw, eps=1e-6, activation=act)
+    h = x.double()
+    if norm:
+        h = (h * torch.rsqrt(h.square().mean(-1, keepdim=True) + 1e-6) * nw.double()).bfloat16().double()
+    z = h @ W.double().t() + b.double()
+    if act:
+        z = F.gelu(z, approximate="tanh")
+    if res:
+        z = z + r.double()
+    assert oracle_close(y, z.cpu(), FRAC_OUT)
