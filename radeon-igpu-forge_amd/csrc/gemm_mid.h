@@ -224,7 +224,8 @@ enum MidTile { kMidNone = 0, kMidBig = 1, kMidSmall = 2 };   // 256 x 128; 64 x 
 // launch (gemm_mid.hip); epi: bit 0 GELU, bit 1 H out, bit 2 bias, bit 4 (with 0 and 1) H is the
 // GELU derivative
 int mid_forward(const MidArgs& a, int tile, int epi, hipStream_t s);
-// gate 0: dX = dY W; 1: times gelu'(G); 2: times G
+// gate 0: dX = dY W (slices > 1: the slices' fp32 products, summed by the caller); 1: times
+// gelu'(G); 2: times G
 int mid_dgrad(const MidArgs& a, int tile, int gate, hipStream_t s);
 // partials (slices > 1, summed by the caller) or C
 int mid_wgrad(const MidArgs& a, int tile, hipStream_t s);

@@ -33,18 +33,46 @@ __device__ __forceinline__ void mid_put(uint16_t* o, int n, int N, bool vec, con
     }
 }
 
+// The fp32 accumulators of a wave's part of a tile into the slice's partial (M x N, N % 4 == 0),
+// each 32-row block through the wave's LDS share as 16-byte row chunks.
+template <int TI, int TJ>
+__device__ __forceinline__ void mid_store_part(float* stg, float* part, int row, int col, int M, int N, int lane,
+                                               const f32x16 (&acc)[TJ][TI]) {
+    constexpr int LDF = 32 * TJ + 4;   // floats per staged row
+    const int g = lane >> 5;
+#pragma unroll
+    for (int i = 0; i < TI; ++i) {
+#pragma unroll
+        for (int j = 0; j < TJ; ++j)
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                *reinterpret_cast<float4*>(stg + (lane & 31) * LDF + 32 * j + 8 * q + 4 * g) =
+                    make_float4(acc[j][i][4 * q], acc[j][i][4 * q + 1], acc[j][i][4 * q + 2], acc[j][i][4 * q + 3]);
+        const int row0 = row + 32 * i;
+#pragma unroll
+        for (int k = 0; k < 4 * TJ; ++k) {
+            const int v = lane + 64 * k, r = v / (8 * TJ), c = (v - r * (8 * TJ)) * 4;
+            if (row0 + r < M && col + c < N)
+                *reinterpret_cast<float4*>(part + (int64_t)(row0 + r) * N + col + c) =
+                    *reinterpret_cast<const float4*>(stg + r * LDF + c);
+        }
+    }
+}
+
 // C = act(A B^T + bias) (forward, B rows along K) or C = (A B) [* gate] (input gradient, B's
 // K down its rows).  EPI: bit 0 GELU, 1 H out, 2 bias, 4 H is the GELU derivative, 5 times the
-// bf16 values of G, 6 times gelu'(G); values are rounded as the 256-wide kernels round them.
+// bf16 values of G, 6 times gelu'(G), 7 the fp32 products of a K slice; values are rounded as the 256-wide kernels round them.
 // The accumulators hold C^T, so a lane has 4 consecutive columns of a row; each 32-row block
 // leaves through the wave's LDS share as 16-byte row chunks.
 template <int BM, int BN, int TI, int TJ, int NST, int AK, int BK, int EPI>
 __global__ void __launch_bounds__(64 * (BM / (32 * TI)) * (BN / (32 * TJ)), BM == 256 ? 2 : (BN / (32 * TJ)) * (BM / (32 * TI)) / 2)
 gemm_mid_kernel(MidArgs a) {
-    constexpr bool kGelu = EPI & 1, kH = EPI & 2, kBias = EPI & 4, kDeriv = EPI & 16, kGate = EPI & 32, kGateH = EPI & 64;
+    constexpr bool kGelu = EPI & 1, kH = EPI & 2, kBias = EPI & 4, kDeriv = EPI & 16, kGate = EPI & 32, kGateH = EPI & 64,
+                   kPart = EPI & 128;
     constexpr int kWaves = (BM / (32 * TI)) * (BN / (32 * TJ)), kWN = BN / (32 * TJ);
     constexpr int LDE = 32 * TJ + 8;
-    constexpr int kStg = 32 * LDE * (kH || kGate || kGateH ? 2 : 1);   // elements per wave
+    constexpr int kStg = kPart ? 2 * 32 * (32 * TJ + 4)                // elements per wave
+                               : 32 * LDE * (kH || kGate || kGateH ? 2 : 1);
     static_assert(kWaves * kStg <= NST * (BM + BN) * 64, "staging fits the stages");
     __shared__ __attribute__((aligned(16))) uint16_t lds[NST * (BM + BN) * 64];
     __shared__ __attribute__((aligned(16))) uint16_t sbias[kBias ? BN : 1];
@@ -52,8 +80,10 @@ gemm_mid_kernel(MidArgs a) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = (wave / kWN) * 32 * TI, wn = (wave % kWN) * 32 * TJ;
     const int nm = (a.M + BM - 1) / BM, nn = (a.N + BN - 1) / BN;
+    const int item = mid_item(blockIdx.x, nm * nn * (kPart ? a.slices : 1));
+    const int sl = kPart ? item / (nm * nn) : 0, nk = (a.K + 63) / 64;
     int mt, nt;
-    mid_tile(mid_item(blockIdx.x, nm * nn), nm, nn, mt, nt);
+    mid_tile(item - sl * nm * nn, nm, nn, mt, nt);
     const int m0 = mt * BM, n0 = nt * BN;
     if constexpr (kBias) {
         if (threadIdx.x < BN) sbias[threadIdx.x] = n0 + (int)threadIdx.x < a.N ? a.bias[n0 + threadIdx.x] : (uint16_t)0;
@@ -73,7 +103,8 @@ gemm_mid_kernel(MidArgs a) {
     }
     f32x16 acc[TJ][TI];
     mid_product<BM, BN, TI, TJ, AK, BK, NST, true>(
-        a.A, a.B, m0, n0, a.K, 0, (a.K + 63) / 64, lds, wave, lane, wm, wn, acc, [&](int kt, const uint16_t* sa) {
+        a.A, a.B, m0, n0, a.K, kPart ? (int)((int64_t)nk * sl / a.slices) : 0,
+        kPart ? (int)((int64_t)nk * (sl + 1) / a.slices) : nk, lds, wave, lane, wm, wn, acc, [&](int kt, const uint16_t* sa) {
             if constexpr (AK == kGather) {
                 // gathered rows out, the K steps of a row panel dealt to its column tiles
                 if (a.Xg == nullptr || kt % nn != nt) return;
@@ -85,6 +116,11 @@ gemm_mid_kernel(MidArgs a) {
                 }
             }
         });
+    if constexpr (kPart) {
+        mid_store_part<TI, TJ>(reinterpret_cast<float*>(lds) + wave * 32 * (32 * TJ + 4), a.part + (int64_t)sl * a.M * a.N,
+                               m0 + wm, n0 + wn, a.M, a.N, lane, acc);
+        return;
+    }
     uint16_t* stg = lds + wave * kStg;
     uint16_t* stg2 = stg + 32 * LDE;
 #pragma unroll
@@ -157,7 +193,10 @@ __global__ void __launch_bounds__(64 * (BM / (32 * TI)) * (BN / (32 * TJ)), BM =
     mid_product<BM, BN, TI, TJ, kColK, kColK, NST, false>(a.A, a.B, m0, n0, a.K, kb, ke, lds, wave, lane, wm, wn, acc,
                                                           [](int, const uint16_t*) {});
     float* stg = reinterpret_cast<float*>(lds) + wave * 32 * LDF;
-    float* part = a.part + (int64_t)sl * a.M * a.N;
+    if (a.slices > 1) {
+        mid_store_part<TI, TJ>(stg, a.part + (int64_t)sl * a.M * a.N, m0 + wm, n0 + wn, a.M, a.N, lane, acc);
+        return;
+    }
 #pragma unroll
     for (int i = 0; i < TI; ++i) {
 #pragma unroll
@@ -167,25 +206,15 @@ __global__ void __launch_bounds__(64 * (BM / (32 * TI)) * (BN / (32 * TJ)), BM =
                 *reinterpret_cast<float4*>(stg + (lane & 31) * LDF + 32 * j + 8 * q + 4 * g) =
                     make_float4(acc[j][i][4 * q], acc[j][i][4 * q + 1], acc[j][i][4 * q + 2], acc[j][i][4 * q + 3]);
         const int row0 = m0 + wm + 32 * i;
-        if (a.slices > 1) {
 #pragma unroll
-            for (int k = 0; k < 4 * TJ; ++k) {
-                const int v = lane + 64 * k, r = v / (8 * TJ), c = (v - r * (8 * TJ)) * 4;
-                if (row0 + r < a.M && n0 + wn + c < a.N)
-                    *reinterpret_cast<float4*>(part + (int64_t)(row0 + r) * a.N + n0 + wn + c) =
-                        *reinterpret_cast<const float4*>(stg + r * LDF + c);
-            }
-        } else {
-#pragma unroll
-            for (int k = 0; k < 2 * TJ; ++k) {
-                const int v = lane + 64 * k, r = v / (4 * TJ), c = (v - r * (4 * TJ)) * 8;
-                if (row0 + r < a.M && n0 + wn + c < a.N) {
-                    const float4 lo = *reinterpret_cast<const float4*>(stg + r * LDF + c);
-                    const float4 hi = *reinterpret_cast<const float4*>(stg + r * LDF + c + 4);
-                    st16(a.C + (int64_t)(row0 + r) * a.ldc + n0 + wn + c,
-                         make_uint4(pack_bf16x2(lo.x, lo.y), pack_bf16x2(lo.z, lo.w), pack_bf16x2(hi.x, hi.y),
-                                    pack_bf16x2(hi.z, hi.w)));
-                }
+        for (int k = 0; k < 2 * TJ; ++k) {
+            const int v = lane + 64 * k, r = v / (4 * TJ), c = (v - r * (4 * TJ)) * 8;
+            if (row0 + r < a.M && n0 + wn + c < a.N) {
+                const float4 lo = *reinterpret_cast<const float4*>(stg + r * LDF + c);
+                const float4 hi = *reinterpret_cast<const float4*>(stg + r * LDF + c + 4);
+                st16(a.C + (int64_t)(row0 + r) * a.ldc + n0 + wn + c,
+                     make_uint4(pack_bf16x2(lo.x, lo.y), pack_bf16x2(lo.z, lo.w), pack_bf16x2(hi.x, hi.y),
+                                pack_bf16x2(hi.z, hi.w)));
             }
         }
     }
@@ -219,6 +248,12 @@ int mid_forward(const MidArgs& a, int tile, int epi, hipStream_t s) {
 }
 
 int mid_dgrad(const MidArgs& a, int tile, int gate, hipStream_t s) {
+    if (a.slices > 1) {
+        if (gate != 0 || tile != kMidBig) return set_error(FX_EINVAL, "mid_dgrad: slices with a gate or small tiles");
+        hipLaunchKernelGGL((gemm_mid_kernel<256, 128, 2, 2, 3, kRowK, kColK, 128>), dim3(tiles_of(a, 256, 128) * a.slices),
+                           dim3(512), 0, s, a);
+        return check_launch("gemm_mid_dgrad");
+    }
 #define FX_MID(E)                                                                                                       \
     if (tile == kMidBig)                                                                                                \
         hipLaunchKernelGGL((gemm_mid_kernel<256, 128, 2, 2, 3, kRowK, kColK, E>), dim3(tiles_of(a, 256, 128)), dim3(512), 0, s, a); \

@@ -16,6 +16,7 @@
 #include <vector>
 
 #include "../../include/fx_abi.h"
+#include "fx_internal.h"
 
 namespace {
 
@@ -279,20 +280,40 @@ Tensor wgrad(const Tensor& dy, const Tensor& x) {
     return dW;
 }
 
-// dx = dy2 w (times g), or None when a layout check fails
-OptT dgrad(const Tensor& dy2, const Tensor& w, const OptT& g) {
+// dx = dy2 w (times g), or None when a layout check fails.  whole: a shape of fx_linear_dgrad
+OptT dgrad(const Tensor& dy2, const Tensor& w, const OptT& g, bool whole) {
     if (!dy2.is_cuda() || !w.is_contiguous() || !aligned(w) || dy2.stride(1) != 1 || dy2.stride(0) % 8 || !aligned(dy2) ||
-        (g.has_value() && (!g->is_contiguous() || !aligned(*g))))
+        !is_bf(dy2) || !is_bf(w) || (g.has_value() && (!g->is_contiguous() || !aligned(*g) || !is_bf(*g))))
         return std::nullopt;
     const int64_t M = dy2.size(0), K = dy2.size(1), N = w.size(1);
     Tensor dx = at::empty({M, N}, dy2.options());
-    if (g.has_value())
-        check(fx_linear_dgrad_gate(bf(dy2), dy2.stride(0), bf(w), N, bf(*g), bf(dx), N, M, N, K, stream_of(dy2)),
-              "fx_linear_dgrad_gate");
-    else
-        check(fx_linear_dgrad(bf(dy2), dy2.stride(0), bf(w), N, nullptr, bf(dx), N, M, N, K, stream_of(dy2)),
-              "fx_linear_dgrad");
+    if (whole) {
+        if (g.has_value())
+            check(fx_linear_dgrad_gate(bf(dy2), dy2.stride(0), bf(w), N, bf(*g), bf(dx), N, M, N, K, stream_of(dy2)),
+                  "fx_linear_dgrad_gate");
+        else
+            check(fx_linear_dgrad(bf(dy2), dy2.stride(0), bf(w), N, nullptr, bf(dx), N, M, N, K, stream_of(dy2)),
+                  "fx_linear_dgrad");
+        return dx;
+    }
+    const int64_t nbytes = fx::input_grad_workspace(M, N, K, g.has_value());
+    Tensor work;
+    if (nbytes) work = at::empty({nbytes / 4}, as_f32(dy2));
+    check(fx::input_grad(bf(dy2), dy2.stride(0), bf(w), bf(g), bf(dx), nbytes ? f32(work) : nullptr, M, N, K,
+                         stream_of(dy2)),
+          "input_grad");
     return dx;
+}
+
+// db = the column sums of g (rows, cols) in g's type
+Tensor column_sums(const Tensor& g) {
+    const int64_t R = g.size(0), C = g.size(1);
+    if (!is_bf(g) || !g.is_cuda() || !g.is_contiguous() || !aligned(g) || R < 1 || R > 64 * 65535 || C < 8 || C % 8)
+        return g.sum(0);
+    Tensor out = at::empty({C}, g.options());
+    Tensor work = at::empty({fx::column_sums_workspace(R, C) / 4}, as_f32(g));
+    check(fx::column_sums(bf(g), R, C, f32(work), bf(out), stream_of(g)), "column_sums");
+    return out;
 }
 
 // ---- cross-entropy ---------------------------------------------------------------------
@@ -439,6 +460,7 @@ PYBIND11_MODULE(_host, m) {
     FX_DEF(gather_fwd);
     FX_DEF(wgrad);
     FX_DEF(dgrad);
+    FX_DEF(column_sums);
     FX_DEF(ce_inv_nvalid);
     FX_DEF(ce_rows);
     FX_DEF(ce_finalize);

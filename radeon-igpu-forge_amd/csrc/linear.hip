@@ -24,6 +24,7 @@
 
 #include "fx_mfma.h"
 #include "gemm_asm.h"
+#include "fx_internal.h"
 #include "gemm_mid.h"
 
 namespace fx {
@@ -2026,6 +2027,20 @@ extern "C" int64_t fx_linear_wgrad_workspace(int64_t M, int64_t N, int64_t K) {
     return p.slices > 1 ? (int64_t)p.slices * M * N * (int64_t)sizeof(float) : 0;
 }
 
+// C (rows x N, row stride ldc) = bf16(sum of the slices' partials)
+static int reduce_slices(const float* part, int slices, int64_t rows, int64_t N, uint16_t* C, int64_t ldc, hipStream_t s) {
+    const bool wide = rows * N / 8 >= 512 * (int64_t)device_cus();
+    int64_t blocks = (rows * N / (wide ? 8 : 4) + 255) / 256;
+    if (blocks > 4096) blocks = 4096;
+    if (wide)
+        hipLaunchKernelGGL(wgrad_reduce_kernel<8>, dim3((unsigned)blocks), dim3(256), 0, s, part, slices, rows * N, (int)N, C,
+                           ldc);
+    else
+        hipLaunchKernelGGL(wgrad_reduce_kernel<4>, dim3((unsigned)blocks), dim3(256), 0, s, part, slices, rows * N, (int)N, C,
+                           ldc);
+    return check_launch("wgrad_reduce");
+}
+
 extern "C" int fx_linear_wgrad(const uint16_t* dY, int64_t ldy, const uint16_t* X, int64_t ldx, uint16_t* dW,
                                int64_t ldw, float* work, int64_t M, int64_t N, int64_t K, void* stream) {
     FX_REQUIRE(dW && (K == 0 || (dY && X)), "fx_linear_wgrad: null pointer");
@@ -2084,16 +2099,7 @@ extern "C" int fx_linear_wgrad(const uint16_t* dY, int64_t ldy, const uint16_t* 
         }
         if (int e = check_launch("gemm_wgrad")) return e;
         if (slices == 1) return 0;
-        const bool wide = rows * N / 8 >= 512 * (int64_t)device_cus();
-        int64_t blocks = (rows * N / (wide ? 8 : 4) + 255) / 256;
-        if (blocks > 4096) blocks = 4096;
-        if (wide)
-            hipLaunchKernelGGL(wgrad_reduce_kernel<8>, dim3((unsigned)blocks), dim3(256), 0, s, (const float*)work, slices,
-                               rows * N, (int)N, a.C, ldw);
-        else
-            hipLaunchKernelGGL(wgrad_reduce_kernel<4>, dim3((unsigned)blocks), dim3(256), 0, s, (const float*)work, slices,
-                               rows * N, (int)N, a.C, ldw);
-        return check_launch("wgrad_reduce");
+        return reduce_slices(work, slices, rows, N, a.C, ldw, s);
     };
     if (!plan.split_rows) return product(0, M, plan.slices);
     if (int e = product(0, plan.split_rows, 1)) return e;
@@ -2175,6 +2181,130 @@ extern "C" int fx_linear_dgrad_gate(const uint16_t* dY, int64_t ldy, const uint1
                                     void* stream) {
     return dgrad_run("fx_linear_dgrad_gate", dY, ldy, W, ldw, G, 2, dX, ldx, M, N, K, stream);
 }
+
+namespace fx {
+
+// K slices of input_grad: a long K over few tiles (a head's 4096 x 512 x 8192: 64 tiles of
+// 256 x 128) fills the chip in 2 to 8 slices of at least 8 K steps, the partials' way through
+// memory counted as in mid_wgrad_cost.  4096 x 512 x 8192: 64 us unsliced, 46 in 4 slices
+// (58 on the library GEMM).
+static int input_grad_slices(int64_t M, int64_t N, int64_t K, bool gated, int* tile) {
+    float best = mid_cost(M, N, K, tile);
+    const float cus = (float)device_cus(), nb = (float)(((M + 255) / 256) * ((N + 127) / 128));
+    const int64_t nk = (K + 63) / 64;
+    int slices = 1;
+    for (int sl = 2; sl <= 8 && !gated && nk / sl >= 8; sl *= 2) {
+        const float t = ceilf(nb * sl / cus) * (4.4f + 0.8f * (float)((nk + sl - 1) / sl)) + 3.f +
+                        (float)sl * (float)M * (float)N * 8.f / 5e6f;
+        if (t < 0.9f * best) {
+            best = t;
+            slices = sl;
+            *tile = kMidBig;
+        }
+    }
+    return slices;
+}
+
+int64_t input_grad_workspace(int64_t M, int64_t N, int64_t K, bool gated) {
+    int tile;
+    if (M <= 0 || N <= 0 || K <= 0) return 0;
+    const int sl = input_grad_slices(M, N, K, gated, &tile);
+    return sl > 1 ? (int64_t)sl * M * N * (int64_t)sizeof(float) : 0;
+}
+
+int input_grad(const uint16_t* dY, int64_t ldy, const uint16_t* W, const uint16_t* G, uint16_t* dX, float* work, int64_t M,
+               int64_t N, int64_t K, void* stream) {
+    FX_REQUIRE(M >= 0 && N >= 8 && K >= 8 && N % 8 == 0 && K % 8 == 0 && M < 0x7fffffffLL && N < 0x7fffffffLL &&
+                   K < 0x7fffffffLL && ldy >= K && ldy % 8 == 0,
+               "input_grad: bad shape M=%lld N=%lld K=%lld ldy=%lld", (long long)M, (long long)N, (long long)K,
+               (long long)ldy);
+    if (M == 0) return 0;
+    FX_REQUIRE(dY && W && dX && ((((uintptr_t)dY) | ((uintptr_t)W) | ((uintptr_t)G) | ((uintptr_t)dX) | ((uintptr_t)work)) & 15) == 0,
+               "input_grad: null or misaligned pointer");
+    MidArgs m{};
+    int tile;
+    m.slices = input_grad_slices(M, N, K, G != nullptr, &tile);
+    FX_REQUIRE(m.slices == 1 || work, "input_grad: null workspace (%d slices)", m.slices);
+    m.A = MidOperand{dY, ldy, (int)M, nullptr, 0, 0};
+    m.B = MidOperand{W, N, (int)N, nullptr, 0, 0};
+    m.C = dX;
+    m.ldc = N;
+    m.G = G;
+    m.ldg = N;
+    m.part = work;
+    m.M = (int)M;
+    m.N = (int)N;
+    m.K = (int)K;
+    m.vec_c = true;
+    if (int e = mid_dgrad(m, tile, G ? 2 : 0, (hipStream_t)stream)) return e;
+    return m.slices > 1 ? reduce_slices(work, m.slices, M, N, dX, N, (hipStream_t)stream) : 0;
+}
+
+// Column sums: a workgroup sums a strip of rows for 512 columns (64 lanes of 8, its 4 waves'
+// rows merged in LDS) into fp32 partials; a second launch sums the strips in order.  8192 x 256:
+// 15.6 + 1.5 us of torch's reduction and its memset, 6 here.
+constexpr int kSumRows = 64;   // rows per workgroup
+template <bool LAST>
+__global__ void __launch_bounds__(256) column_sums_kernel(const uint16_t* __restrict__ g, const float* __restrict__ in,
+                                                          int64_t rows, int64_t cols, float* __restrict__ part,
+                                                          uint16_t* __restrict__ out) {
+    __shared__ float sh[4][64 * 8];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int64_t c = ((int64_t)blockIdx.x * 64 + lane) * 8;
+    const int64_t r0 = (int64_t)blockIdx.y * kSumRows, r1 = LAST ? rows : (r0 + kSumRows < rows ? r0 + kSumRows : rows);
+    float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    if (c < cols) {
+#pragma unroll 8
+        for (int64_t r = r0 + w; r < r1; r += 4) {
+            float f[8];
+            if constexpr (LAST) {
+                const float4 lo = *reinterpret_cast<const float4*>(in + r * cols + c);
+                const float4 hi = *reinterpret_cast<const float4*>(in + r * cols + c + 4);
+                f[0] = lo.x; f[1] = lo.y; f[2] = lo.z; f[3] = lo.w;
+                f[4] = hi.x; f[5] = hi.y; f[6] = hi.z; f[7] = hi.w;
+            } else {
+                unpack8(ld16(g + r * cols + c), f);
+            }
+#pragma unroll
+            for (int e = 0; e < 8; ++e) s[e] += f[e];
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) sh[w][lane * 8 + e] = s[e];
+    __syncthreads();
+    if (w != 0 || c >= cols) return;
+#pragma unroll
+    for (int v = 1; v < 4; ++v)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s[e] += sh[v][lane * 8 + e];
+    if constexpr (LAST) {
+        st16(out + c, pack8(s));
+    } else {
+        float* p = part + (int64_t)blockIdx.y * cols + c;
+        *reinterpret_cast<float4*>(p) = make_float4(s[0], s[1], s[2], s[3]);
+        *reinterpret_cast<float4*>(p + 4) = make_float4(s[4], s[5], s[6], s[7]);
+    }
+}
+
+int64_t column_sums_workspace(int64_t rows, int64_t cols) {
+    return rows > 0 && cols > 0 ? (rows + kSumRows - 1) / kSumRows * cols * (int64_t)sizeof(float) : 0;
+}
+
+int column_sums(const uint16_t* g, int64_t rows, int64_t cols, float* work, uint16_t* out, void* stream) {
+    const int64_t strips = (rows + kSumRows - 1) / kSumRows;
+    FX_REQUIRE(rows >= 1 && cols >= 8 && cols % 8 == 0 && strips <= 65535 && g && work && out &&
+                   ((((uintptr_t)g) | ((uintptr_t)work) | ((uintptr_t)out)) & 15) == 0,
+               "column_sums: bad arguments (rows=%lld cols=%lld)", (long long)rows, (long long)cols);
+    const unsigned nb = (unsigned)((cols + 511) / 512);
+    hipStream_t s = (hipStream_t)stream;
+    hipLaunchKernelGGL(column_sums_kernel<false>, dim3(nb, (unsigned)strips), dim3(256), 0, s, g, nullptr, rows, cols, work,
+                       nullptr);
+    if (int e = check_launch("column_sums")) return e;
+    hipLaunchKernelGGL(column_sums_kernel<true>, dim3(nb), dim3(256), 0, s, nullptr, work, strips, cols, nullptr, out);
+    return check_launch("column_sums");
+}
+
+}  // namespace fx
 
 extern "C" int fx_gelu_bwd(const uint16_t* dy, const uint16_t* h, uint16_t* dh, int64_t n, void* stream) {
     FX_REQUIRE(n >= 0 && (n == 0 || (dy && h && dh)), "fx_gelu_bwd: null pointer");

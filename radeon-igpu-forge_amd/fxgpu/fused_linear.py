@@ -97,12 +97,12 @@ NATIVE_SMALL_INPUT_GRAD = True
 
 
 def small_dgrad(M, N, K):
-    """Plain input gradients where fx_linear_dgrad (small tiles) is at least as fast as the
-    library GEMM, up to 8,192 rows, K up to 3072 and 40 GFLOP: 4096 x 512 x 1536 15.9 us, 8192 x 256 x 768
-    9.2 (torch.mm: 19 us of host time alone), 4096 x 768 x 3072 35.3 against 37.0, 8192 x 3072
-    x 768 43.9 / 48.5, 8192 x 768 x 3072 47.2 / 48.2; not 4096 x 512 x 8192 (69.3 / 58.3) nor
-    16384 x 768 x 768 (1 % on a block's forward and backward)."""
-    return M <= 8192 and K <= 3072 and M * N * K <= 20 * 10 ** 9 and dgrad_tiles(M, N, K)
+    """Input gradients of up to 8,192 rows and 40 GFLOP, any row count, run on the small tiles
+    (a long K in slices), at least as fast there as the library GEMM: 4096 x 512 x 1536 15.9 us,
+    8192 x 256 x 768 9.2 (torch.mm: 19 us of host time alone), 4096 x 768 x 3072 35.3 against
+    37.0, 8192 x 3072 x 768 43.9 / 48.5, 8192 x 768 x 3072 47.2 / 48.2, 4096 x 512 x 8192 in 4
+    slices 46 / 58; not 16384 x 768 x 768 (1 % on a block's forward and backward)."""
+    return 0 < M <= 8192 and M * N * K <= 20 * 10 ** 9 and N % 8 == 0 and K % 8 == 0
 
 
 def dgrad_tiles(M, N, K):
@@ -122,11 +122,16 @@ def input_grad(dy2, weight, g=None):
     fx_gelu_bwd, 125.5 against 133.6 from HBM); else torch.mm, then fx_gelu_bwd_gate for g."""
     M, K = dy2.shape
     N = weight.shape[1]
-    wanted = ((NATIVE_INPUT_GRAD and (g is not None or N <= 1024)) or (NATIVE_GELU_INPUT_GRAD and g is not None)
-              or (NATIVE_SMALL_INPUT_GRAD and g is None and small_dgrad(M, N, K)))
-    if wanted and dgrad_tiles(M, N, K):
-        dx = host.dgrad(dy2, weight, g)     # None: a layout the kernel does not take
-        if dx is not None:
+    tiles = dgrad_tiles(M, N, K)
+    if g is not None:
+        native = (NATIVE_GELU_INPUT_GRAD or NATIVE_INPUT_GRAD) and (tiles or small_dgrad(M, N, K))
+    else:
+        native = ((NATIVE_SMALL_INPUT_GRAD and small_dgrad(M, N, K))
+                  or (NATIVE_INPUT_GRAD and N <= 1024 and tiles))
+    if native:
+        # whole tiles of a K up to 3072 through fx_linear_dgrad(_gate), which picks the tile width
+        dx = host.dgrad(dy2, weight, g, tiles and (K <= 3072 or g is not None))
+        if dx is not None:     # None: a layout the kernels do not take
             return dx
     dx = torch.mm(dy2, weight)
     if g is None:
@@ -228,7 +233,7 @@ class FusedGatherLinear(torch.autograd.Function):
         (Xg,) = ctx.saved_tensors
         g = g.contiguous()
         dW = linear_wgrad(g, Xg)          # (N, K)
-        db = g.sum(0)
+        db = host.column_sums(g)
         return None, None, dW, db
 
 
@@ -281,7 +286,7 @@ class FusedLinear(torch.autograd.Function):
             dh = dy2
         dx = input_grad(dh, weight).view(ctx.xshape) if ctx.needs_input_grad[0] else None
         dW = linear_wgrad(dh, x2) if ctx.needs_input_grad[1] else None
-        db = dh.sum(0) if (ctx.has_bias and ctx.needs_input_grad[2]) else None
+        db = host.column_sums(dh) if (ctx.has_bias and ctx.needs_input_grad[2]) else None
         return dx, dW, db, None
 
 

@@ -22,7 +22,7 @@ behaviour, ml/fxlm/cross_entropy.py:41-44 and ml/fxlm/kernels/ce.hip:43).
 import torch
 
 from fxgpu.abi import call, host, lib, ptr, stream_of
-from fxgpu.fused_linear import linear_wgrad
+from fxgpu.fused_linear import _native_fwd, input_grad, linear_wgrad, native_fwd
 
 # rows per linear-CE chunk: bound the chunk's bf16 logits to this many bytes
 _CHUNK_BYTES = 2 << 30
@@ -159,6 +159,17 @@ def _auto_chunk(D, V):
 _FUSED_LIN_GRAD_SCALE = True
 
 
+def _logits(x, weight):
+    """x W^T on this build's kernels up to 16 GFLOP (a small vocabulary: native_fwd() has them
+    ahead), else on the library GEMM (16384 x 50304 x 768: 1,108 against 1,648 us)."""
+    M, K = x.shape
+    V = weight.shape[0]
+    if (M * V * K <= 8 << 30 and K % 8 == 0 and M > 0 and native_fwd(M, V, K)
+            and (x.data_ptr() | weight.data_ptr()) % 16 == 0):
+        return _native_fwd(x, weight)
+    return torch.mm(x, weight.t())
+
+
 class _LinearCE(torch.autograd.Function):
     """loss = CE(x @ W.T, target); the (N, V) logits never exist beyond one chunk."""
 
@@ -170,7 +181,7 @@ class _LinearCE(torch.autograd.Function):
             chunk_rows = _auto_chunk(D, V)
         inv_n, mul = _inv_nvalid(target, ignore_index, grad_scale)
         row_loss = torch.empty(N, device=dev, dtype=torch.float32)
-        dx = torch.empty(N, D, device=dev, dtype=torch.bfloat16)
+        dx = torch.empty(N, D, device=dev, dtype=torch.bfloat16) if chunk_rows < N or N == 0 else None
         dW = None
         fused = FUSED_LINEAR_CE_TRAIN and _lce_fused_ok(x, weight)
         dl_buf = torch.empty(min(chunk_rows, N), V, device=dev, dtype=torch.bfloat16) if fused else None
@@ -182,9 +193,12 @@ class _LinearCE(torch.autograd.Function):
                 lg = dl_buf[:r1 - r0]
                 _lce_grad(xc, weight, target[r0:r1], ignore_index, stat, mul, lg)
             else:
-                lg = torch.mm(xc, weight.t())                   # (C, V) bf16
+                lg = _logits(xc, weight)                        # (C, V) bf16
                 _ce_rows(lg, target[r0:r1], lg, row_loss[r0:r1], mul, ignore_index)  # in place
-            torch.mm(lg, weight, out=dx[r0:r1])                 # dx_c
+            if r1 - r0 == N:
+                dx = input_grad(lg, weight)
+            else:
+                torch.mm(lg, weight, out=dx[r0:r1])             # dx_c
             # the reference's dW.add_(torch.mm(dl.t(), xc).float()): a bf16 product,
             # accumulated over the chunks in fp32 (ml/fxlm/cross_entropy.py:135); a single
             # chunk's product stays bf16 (exact in fp32) and the backward reads it as such
@@ -273,7 +287,7 @@ def _linear_ce_loss_only(x, weight, target, ignore_index, chunk_rows):
         return _finalize(row_loss, inv_n)
     for r0 in range(0, N, chunk_rows):
         r1 = min(r0 + chunk_rows, N)
-        lg = torch.mm(x[r0:r1], weight.t())
+        lg = _logits(x[r0:r1], weight)
         _ce_rows(lg, target[r0:r1], None, row_loss[r0:r1], _mul, ignore_index)
     return _finalize(row_loss, inv_n)
 

@@ -384,7 +384,7 @@ def test_rows_cut_inside_a_16_byte_chunk(dev, V, off, ld_pad, in_place):
     p = x.softmax(-1)
     p.scatter_add_(1, t.clamp_min(0)[:, None], torch.full((N, 1), -1.0, device=dev, dtype=torch.float64))
     ref = p * 0.25 * ok[:, None]
-    # one bf16 rounding (2^-9 of the value) and fp32 sums and exponentials (1e-5 of the scale)
+    # one bf16 rounding (2^-8 of the value) and fp32 sums and exponentials (1e-5 of the scale)
     assert bool(((gr.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-5 * 0.25).all())
     keep = torch.ones_like(flat, dtype=torch.bool)
     keep[off:off + N * ld].view(N, ld)[:, :V] = False

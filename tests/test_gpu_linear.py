@@ -702,3 +702,37 @@ def test_few_rows_tile_choices(dev, M, K, N, norm, res, act):
     if res:
         z = z + r.double()
     assert oracle_close(y, z.cpu(), FRAC_OUT)
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (1, 8, 8),            # one row, one chunk
+    (300, 72, 200),       # partial tiles, a K tail
+    (2829, 640, 2560),    # ragged rows of a layer of 640
+    (1031, 264, 8200),    # a long K: slices, the last with a tail of 8
+    (4096, 512, 8192),    # slices of whole steps
+])
+def test_input_grad_any_rows(dev, M, N, K):
+    import fxgpu.fused_linear as FL
+    g = torch.Generator(device=dev).manual_seed(M + N + K)
+    dy = torch.randn(M, K, device=dev, generator=g).bfloat16()
+    W = (torch.randn(K, N, device=dev, generator=g) * K ** -0.5).bfloat16()
+    gd = (torch.rand(M, N, device=dev, generator=g) * 1.3 - 0.15).bfloat16()
+    print(f"input_grad M={M} N={N} K={K}", flush=True)
+    assert FL.small_dgrad(M, N, K)
+    dx, dg = FL.input_grad(dy, W), FL.input_grad(dy, W, gd)
+    ref = dy.double() @ W.double()
+    assert oracle_close(dx, ref.cpu(), FRAC_OUT)
+    # the gate multiplies the rounded product of the unsliced kernel: one more bf16 rounding
+    assert oracle_close(dg, (ref * gd.double()).cpu(), 2 * FRAC_OUT + 2.0 ** -8)
+
+
+@pytest.mark.parametrize("R,C", [(1, 8), (63, 16), (64, 520), (65, 512), (8192, 256), (70000, 24)])
+def test_column_sums(dev, R, C):
+    from fxgpu.abi import host
+    g = torch.Generator(device=dev).manual_seed(R + C)
+    x = torch.randn(R, C, device=dev, generator=g).bfloat16()
+    s, ref = host.column_sums(x), x.double().sum(0)
+    # one bf16 rounding (8 significant bits: 2^-8 of the value), and fp32 sums (2^-24 of the sum of
+    # magnitudes per addition, at most 16 + 3 additions deep per strip and R / 256 strips)
+    bound = 2.0 ** -8 * ref.abs() + 2.0 ** -24 * (19 + R / 256) * x.double().abs().sum(0)
+    assert bool(((s.double() - ref).abs() <= 1.01 * bound).all())
