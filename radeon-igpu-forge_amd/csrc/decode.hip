@@ -20,6 +20,7 @@
 #include <math.h>
 
 #include "fx_device.h"
+#include "fx_internal.h"
 
 namespace fx {
 
@@ -233,6 +234,47 @@ static int decode_launch(const fxAttnDecodeArgs& a, const DecodeShape& s, hipStr
     if (s.nseg == 1) return 0;
     hipLaunchKernelGGL((attn_decode_merge_kernel<D>), dim3(nbh), dim3(64), 0, st, a, s.nseg, s.seglen);
     return check_launch("attn_decode_merge");
+}
+
+// The step's inputs into the graph's static buffers, and the token and position embeddings' sum:
+// a launch each.  As torch operations they were three and three, of 2.5 to 8.6 us (the two
+// index kernels), 28 us of a 12-layer step's 463.
+__global__ void __launch_bounds__(256) decode_inputs_kernel(const int64_t* tok, int64_t n, int64_t pos, int64_t* tok_out,
+                                                            int64_t* pos_out, int32_t* lens) {
+    for (int64_t i = threadIdx.x; i < n; i += 256) {
+        tok_out[i] = tok[i];
+        lens[i] = (int32_t)(pos + 1);
+    }
+    if (threadIdx.x == 0) *pos_out = pos;
+}
+
+__global__ void __launch_bounds__(128) decode_embed_kernel(const int64_t* tok, const int64_t* pos, const uint16_t* E,
+                                                           int64_t V, const uint16_t* P, int64_t T, uint16_t* x, int64_t D) {
+    const int64_t t = tok[blockIdx.x], p = *pos;
+    if (t < 0 || t >= V || p < 0 || p >= T) __builtin_trap();
+    for (int64_t c = (int64_t)threadIdx.x * 8; c < D; c += 128 * 8) {
+        float e[8], q[8];
+        unpack8(ld16(E + t * D + c), e);
+        unpack8(ld16(P + p * D + c), q);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) e[j] += q[j];
+        st16(x + (int64_t)blockIdx.x * D + c, pack8(e));
+    }
+}
+
+int decode_inputs(const int64_t* tok, int64_t n, int64_t pos, int64_t* tok_out, int64_t* pos_out, int32_t* lens, void* stream) {
+    FX_REQUIRE(n >= 0 && (n == 0 || (tok && tok_out && lens)) && pos_out, "decode_inputs: bad arguments (n=%lld)", (long long)n);
+    hipLaunchKernelGGL(decode_inputs_kernel, dim3(1), dim3(256), 0, (hipStream_t)stream, tok, n, pos, tok_out, pos_out, lens);
+    return check_launch("decode_inputs");
+}
+
+int decode_embed(const int64_t* tok, const int64_t* pos, const uint16_t* E, int64_t V, const uint16_t* P, int64_t T, uint16_t* x,
+                 int64_t n, int64_t D, void* stream) {
+    FX_REQUIRE(n >= 1 && n < 0x7fffffffLL && D >= 8 && D % 8 == 0 && tok && pos && E && P && x &&
+                   ((((uintptr_t)E) | ((uintptr_t)P) | ((uintptr_t)x)) & 15) == 0,
+               "decode_embed: bad arguments (n=%lld D=%lld)", (long long)n, (long long)D);
+    hipLaunchKernelGGL(decode_embed_kernel, dim3((unsigned)n), dim3(128), 0, (hipStream_t)stream, tok, pos, E, V, P, T, x, D);
+    return check_launch("decode_embed");
 }
 
 }  // namespace fx

@@ -376,6 +376,49 @@ void ce_lin_scale_inplace(const Tensor& dW, const Tensor& dx, const Tensor& g32,
           "fx_ce_lin_grad_scale_inplace");
 }
 
+// ---- a decode step's ends ----------------------------------------------------------------
+
+// the step's inputs into a graph's static buffers; false: not tensors the kernel takes
+bool decode_inputs(const Tensor& tok, int64_t pos, const Tensor& tok_out, const Tensor& pos_out, const Tensor& lens) {
+    if (tok.scalar_type() != at::kLong || !tok.is_contiguous() || tok.device() != tok_out.device() ||
+        tok.sizes() != tok_out.sizes())
+        return false;
+    check(fx::decode_inputs(static_cast<int64_t*>(tok.data_ptr()), tok.numel(), pos, static_cast<int64_t*>(tok_out.data_ptr()),
+                            static_cast<int64_t*>(pos_out.data_ptr()), static_cast<int32_t*>(lens.data_ptr()),
+                            stream_of(tok)),
+          "decode_inputs");
+    return true;
+}
+
+// E[tok] + P[pos] as (B, 1, D), or None when a check fails
+OptT decode_embed(const Tensor& tok, const Tensor& pos, const Tensor& E, const Tensor& P) {
+    if (tok.dim() != 1 || tok.scalar_type() != at::kLong || !tok.is_contiguous() || !tok.is_cuda() || tok.numel() < 1 ||
+        pos.numel() != 1 || pos.scalar_type() != at::kLong || !pos.is_cuda() || !is_bf(E) || !is_bf(P) || !E.is_cuda() ||
+        !P.is_cuda() || E.dim() != 2 || P.dim() != 2 || E.size(1) != P.size(1) || E.size(1) % 8 || E.size(1) < 8 ||
+        !E.is_contiguous() || !P.is_contiguous() || !aligned(E) || !aligned(P))
+        return std::nullopt;
+    const int64_t B = tok.numel(), D = E.size(1);
+    Tensor x = at::empty({B, 1, D}, E.options());
+    check(fx::decode_embed(static_cast<int64_t*>(tok.data_ptr()), static_cast<int64_t*>(pos.data_ptr()), bf(E), E.size(0), bf(P),
+                           P.size(0), bf(x), B, D, stream_of(E)),
+          "decode_embed");
+    return x;
+}
+
+// norm(x) W^T as fp32 for x (B, D) rows, or None when a check fails
+OptT few_rows_logits(const Tensor& x, const Tensor& w, const Tensor& norm_w, double eps) {
+    if (x.dim() != 2 || w.dim() != 2 || norm_w.dim() != 1 || !is_bf(x) || !is_bf(w) || !is_bf(norm_w) || !x.is_cuda() ||
+        !w.is_cuda() || !norm_w.is_cuda() || x.size(0) < 1 || x.size(0) > 64 || w.size(1) != x.size(1) ||
+        norm_w.size(0) != x.size(1) || x.size(1) % 8 || x.stride(1) != 1 || x.stride(0) % 8 || !w.is_contiguous() ||
+        !norm_w.is_contiguous() || !aligned(x) || !aligned(w) || !aligned(norm_w))
+        return std::nullopt;
+    Tensor out = at::empty({x.size(0), w.size(0)}, as_f32(x));
+    check(fx::few_rows_logits(bf(x), x.stride(0), bf(w), bf(norm_w), (float)eps, f32(out), x.size(0), w.size(0), x.size(1),
+                              stream_of(x)),
+          "few_rows_logits");
+    return out;
+}
+
 // ---- optimiser -------------------------------------------------------------------------
 
 // The flat layout of FlatAdamW: per parameter its offset, size and weight-decay flag.
@@ -461,6 +504,9 @@ PYBIND11_MODULE(_host, m) {
     FX_DEF(wgrad);
     FX_DEF(dgrad);
     FX_DEF(column_sums);
+    FX_DEF(decode_inputs);
+    FX_DEF(decode_embed);
+    FX_DEF(few_rows_logits);
     FX_DEF(ce_inv_nvalid);
     FX_DEF(ce_rows);
     FX_DEF(ce_finalize);

@@ -73,6 +73,7 @@ struct GemmArgs {
     float eps;
     bool vec_c, vec_h;   // C / H rows start 16-byte aligned (16-byte epilogue stores)
     bool vec_r;          // residual rows start 16-byte aligned (16-byte epilogue loads)
+    float* C32;          // few-row kernels: the rounded outputs as fp32 (row stride N) in place of C, or null
 };
 
 // tile t -> (row panel, column tile).  Workgroups are dealt round-robin to the 8 XCDs, so
@@ -1448,7 +1449,9 @@ __device__ __forceinline__ void skinny_store(const GemmArgs& a, float sum, int m
         if (a.act == 1) y = gelu_tanh(h);
     }
     if (a.res) y += bf16_to_f32(a.res[(int64_t)m * a.ldres + n]);
-    a.C[(int64_t)m * a.ldc + n] = f32_to_bf16(y);
+    const uint16_t o = f32_to_bf16(y);
+    if (a.C32) a.C32[(int64_t)m * a.N + n] = bf16_to_f32(o);
+    else a.C[(int64_t)m * a.ldc + n] = o;
 }
 
 // rstd of the rows of X from the operands of one batch that spans each wave's K range: the sum
@@ -2183,6 +2186,26 @@ extern "C" int fx_linear_dgrad_gate(const uint16_t* dY, int64_t ldy, const uint1
 }
 
 namespace fx {
+
+int few_rows_logits(const uint16_t* X, int64_t ldx, const uint16_t* W, const uint16_t* norm_w, float eps, float* out, int64_t M,
+                    int64_t N, int64_t K, void* stream) {
+    FX_REQUIRE(X && W && norm_w && out && M >= 1 && M <= kSKMaxM && N >= 1 && N < 0x7fffffffLL && K >= 8 && K % 8 == 0 &&
+                   K < 0x7fffffffLL && ldx >= K && ldx % 8 == 0 && eps >= 0.f && eps < __builtin_huge_valf() &&
+                   ((((uintptr_t)X) | ((uintptr_t)W) | ((uintptr_t)norm_w)) & 15) == 0,
+               "few_rows_logits: bad arguments (M=%lld N=%lld K=%lld)", (long long)M, (long long)N, (long long)K);
+    GemmArgs a{};
+    a.A = X;
+    a.lda = ldx;
+    a.B = W;
+    a.ldb = K;
+    a.C32 = out;
+    a.M = (int)M;
+    a.N = (int)N;
+    a.K = (int)K;
+    a.nw = norm_w;
+    a.eps = eps;
+    return linear_skinny(a, (hipStream_t)stream);
+}
 
 // K slices of input_grad: a long K over few tiles (a head's 4096 x 512 x 8192: 64 tiles of
 // 256 x 128) fills the chip in 2 to 8 slices of at least 8 K steps, the partials' way through

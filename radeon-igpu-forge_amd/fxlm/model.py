@@ -16,6 +16,7 @@ import torch
 import torch.nn.functional as Fn
 from torch import nn
 
+from fxgpu.abi import host
 from fxgpu.fused_linear import FEW_ROWS, fused_linear, fused_mlp, linear, linear_ex
 
 from .attention import decode_attention, flash_attention_qkv
@@ -265,10 +266,16 @@ class GPT(nn.Module):
         """Cached step with the position in device memory: tok (B,) int64, pos (1,) int64,
         lens (B,) int32 = pos + 1; returns the logits (B, V) fp32."""
         B = tok.shape[0]
-        x = self.tok_emb(tok.view(B, 1)) + self.pos_emb.index_select(0, pos)
+        fused = bool(self.blocks) and self.blocks[0]._fused_step(B)
+        x = host.decode_embed(tok, pos, self.tok_emb.weight, self.pos_emb) if fused and tok.is_cuda else None
+        if x is None:
+            x = self.tok_emb(tok.view(B, 1)) + self.pos_emb.index_select(0, pos)
         for blk, kv in zip(self.blocks, cache):
             x = blk.step(x, kv, pos, lens)
-        if self.blocks and self.blocks[0]._fused_step(B):   # final norm inside the head GEMM
+        if fused:   # final norm inside the head GEMM, which writes its bf16 values as fp32
+            logits = host.few_rows_logits(x[:, 0], self._head_w(), self.lnf_w, self.cfg.eps)
+            if logits is not None:
+                return logits
             return linear_ex(x[:, 0], self._head_w(), norm_weight=self.lnf_w, eps=self.cfg.eps).float()
         x = self._norm_f(x)
         return self._head(x[:, 0]).float()
@@ -357,8 +364,9 @@ class _DecodeGraph:
     def __call__(self, tok, pos):
         if pos >= self.cache_len:
             raise ValueError(f"position {pos} is past the cache ({self.cache_len})")
-        self.tok.copy_(tok)
-        self.pos.fill_(pos)
-        self.lens.fill_(pos + 1)
+        if not (torch.is_tensor(tok) and host.decode_inputs(tok, pos, self.tok, self.pos, self.lens)):
+            self.tok.copy_(tok)
+            self.pos.fill_(pos)
+            self.lens.fill_(pos + 1)
         self.graph.replay()
         return self.logits

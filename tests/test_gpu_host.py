@@ -65,3 +65,22 @@ def test_optimizer_deepcopy_takes_the_same_step(dev):
             p.grad = torch.ones_like(p)
         o.step()
     assert torch.equal(opt.master, twin.master) and float(opt._step_ctr) == 1
+
+
+@pytest.mark.parametrize("B,V,D", [(1, 256, 64), (17, 50304, 768), (64, 1003, 1032)])
+def test_decode_step_ends_equal_the_torch_operations(dev, B, V, D):
+    # bit for bit: the embedding sum, the graph's inputs, and the head's bf16 logits as fp32
+    from fxgpu.abi import host
+    from fxgpu.fused_linear import linear_ex
+    g = torch.Generator(device=dev).manual_seed(B + V)
+    E, P = (torch.randn(n, D, device=dev, generator=g).bfloat16() for n in (V, 96))
+    tok = torch.randint(0, V, (B,), device=dev, generator=g)
+    tok_out, pos, lens = torch.zeros_like(tok), torch.zeros(1, dtype=torch.int64, device=dev), \
+        torch.zeros(B, dtype=torch.int32, device=dev)
+    assert host.decode_inputs(tok, 41, tok_out, pos, lens)
+    assert torch.equal(tok, tok_out) and int(pos) == 41 and bool((lens == 42).all())
+    assert not host.decode_inputs(tok.int(), 41, tok_out, pos, lens)
+    x = host.decode_embed(tok_out, pos, E, P)
+    assert torch.equal(x, torch.nn.functional.embedding(tok, E)[:, None] + P.index_select(0, pos))
+    w = torch.ones(D, device=dev).bfloat16()
+    assert torch.equal(host.few_rows_logits(x[:, 0], E, w, 1e-6), linear_ex(x[:, 0], E, norm_weight=w, eps=1e-6).float())
