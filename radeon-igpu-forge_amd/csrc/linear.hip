@@ -2264,30 +2264,21 @@ int input_grad(const uint16_t* dY, int64_t ldy, const uint16_t* W, const uint16_
 }
 
 // Column sums: a workgroup sums a strip of rows for 512 columns (64 lanes of 8, its 4 waves'
-// rows merged in LDS) into fp32 partials; a second launch sums the strips in order.  8192 x 256:
-// 15.6 + 1.5 us of torch's reduction and its memset, 6 here.
+// rows merged in LDS) into fp32 partials; a second launch sums the strips in a fixed order.
+// 8192 x 256: 15.6 + 1.5 us of torch's reduction and its memset, 3.7 + 2.7 here.
 constexpr int kSumRows = 64;   // rows per workgroup
-template <bool LAST>
-__global__ void __launch_bounds__(256) column_sums_kernel(const uint16_t* __restrict__ g, const float* __restrict__ in,
-                                                          int64_t rows, int64_t cols, float* __restrict__ part,
-                                                          uint16_t* __restrict__ out) {
+__global__ void __launch_bounds__(256) column_sums_kernel(const uint16_t* __restrict__ g, int64_t rows, int64_t cols,
+                                                          float* __restrict__ part) {
     __shared__ float sh[4][64 * 8];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int64_t c = ((int64_t)blockIdx.x * 64 + lane) * 8;
-    const int64_t r0 = (int64_t)blockIdx.y * kSumRows, r1 = LAST ? rows : (r0 + kSumRows < rows ? r0 + kSumRows : rows);
+    const int64_t r0 = (int64_t)blockIdx.y * kSumRows, r1 = r0 + kSumRows < rows ? r0 + kSumRows : rows;
     float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     if (c < cols) {
 #pragma unroll 8
         for (int64_t r = r0 + w; r < r1; r += 4) {
             float f[8];
-            if constexpr (LAST) {
-                const float4 lo = *reinterpret_cast<const float4*>(in + r * cols + c);
-                const float4 hi = *reinterpret_cast<const float4*>(in + r * cols + c + 4);
-                f[0] = lo.x; f[1] = lo.y; f[2] = lo.z; f[3] = lo.w;
-                f[4] = hi.x; f[5] = hi.y; f[6] = hi.z; f[7] = hi.w;
-            } else {
-                unpack8(ld16(g + r * cols + c), f);
-            }
+            unpack8(ld16(g + r * cols + c), f);
 #pragma unroll
             for (int e = 0; e < 8; ++e) s[e] += f[e];
         }
@@ -2300,13 +2291,45 @@ __global__ void __launch_bounds__(256) column_sums_kernel(const uint16_t* __rest
     for (int v = 1; v < 4; ++v)
 #pragma unroll
         for (int e = 0; e < 8; ++e) s[e] += sh[v][lane * 8 + e];
-    if constexpr (LAST) {
-        st16(out + c, pack8(s));
-    } else {
-        float* p = part + (int64_t)blockIdx.y * cols + c;
-        *reinterpret_cast<float4*>(p) = make_float4(s[0], s[1], s[2], s[3]);
-        *reinterpret_cast<float4*>(p + 4) = make_float4(s[4], s[5], s[6], s[7]);
+    float* p = part + (int64_t)blockIdx.y * cols + c;
+    *reinterpret_cast<float4*>(p) = make_float4(s[0], s[1], s[2], s[3]);
+    *reinterpret_cast<float4*>(p + 4) = make_float4(s[4], s[5], s[6], s[7]);
+}
+
+// The strips' sums: 8 columns (two lanes of 4) by 128 strips a workgroup, so that the partials
+// are one load per thread for up to 128 strips.  A chain of loads bounds this launch, not the
+// bytes: one workgroup per 512 columns, 32 loads behind one another, took 10.3 us.
+__global__ void __launch_bounds__(256) column_sums_last_kernel(const float* __restrict__ part, int64_t strips, int64_t cols,
+                                                               uint16_t* __restrict__ out) {
+    __shared__ float4 red[4][2];
+    const int cg = threadIdx.x & 1;
+    const int64_t col = (int64_t)blockIdx.x * 8 + cg * 4;   // cols is a multiple of 8: always inside
+    float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 4
+    for (int64_t r = threadIdx.x >> 1; r < strips; r += 128) {
+        const float4 v = *reinterpret_cast<const float4*>(part + r * cols + col);
+        s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
     }
+#pragma unroll
+    for (int off = 2; off < 64; off <<= 1) {
+        s.x += __shfl_xor(s.x, off, 64);
+        s.y += __shfl_xor(s.y, off, 64);
+        s.z += __shfl_xor(s.z, off, 64);
+        s.w += __shfl_xor(s.w, off, 64);
+    }
+    if ((threadIdx.x & 63) < 2) red[threadIdx.x >> 6][cg] = s;
+    __syncthreads();
+    if (threadIdx.x >= 2) return;
+    float4 t = red[0][cg];
+#pragma unroll
+    for (int k = 1; k < 4; ++k) {
+        const float4 v = red[k][cg];
+        t.x += v.x; t.y += v.y; t.z += v.z; t.w += v.w;
+    }
+    uint2 u;
+    u.x = pack_bf16x2(t.x, t.y);
+    u.y = pack_bf16x2(t.z, t.w);
+    *reinterpret_cast<uint2*>(out + col) = u;
 }
 
 int64_t column_sums_workspace(int64_t rows, int64_t cols) {
@@ -2318,12 +2341,11 @@ int column_sums(const uint16_t* g, int64_t rows, int64_t cols, float* work, uint
     FX_REQUIRE(rows >= 1 && cols >= 8 && cols % 8 == 0 && strips <= 65535 && g && work && out &&
                    ((((uintptr_t)g) | ((uintptr_t)work) | ((uintptr_t)out)) & 15) == 0,
                "column_sums: bad arguments (rows=%lld cols=%lld)", (long long)rows, (long long)cols);
-    const unsigned nb = (unsigned)((cols + 511) / 512);
     hipStream_t s = (hipStream_t)stream;
-    hipLaunchKernelGGL(column_sums_kernel<false>, dim3(nb, (unsigned)strips), dim3(256), 0, s, g, nullptr, rows, cols, work,
-                       nullptr);
+    hipLaunchKernelGGL(column_sums_kernel, dim3((unsigned)((cols + 511) / 512), (unsigned)strips), dim3(256), 0, s, g, rows,
+                       cols, work);
     if (int e = check_launch("column_sums")) return e;
-    hipLaunchKernelGGL(column_sums_kernel<true>, dim3(nb), dim3(256), 0, s, nullptr, work, strips, cols, nullptr, out);
+    hipLaunchKernelGGL(column_sums_last_kernel, dim3((unsigned)(cols / 8)), dim3(256), 0, s, work, strips, cols, out);
     return check_launch("column_sums");
 }
 
