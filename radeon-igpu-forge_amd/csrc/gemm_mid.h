@@ -4,7 +4,7 @@
 //
 // A 4096 x 512 output is 32 tiles of 256 x 256: one CU in eight works, each through the whole
 // K loop and a 256 x 256 epilogue.  These kernels cut the output into 64 x 128, 128 x 128 or
-// 256 x 128 tiles of 4 or 8 waves.  A K step is 64 values: an operand row is one 128-byte line
+// 256 x 128 tiles of 8 waves.  A K step is 64 values: an operand row is one 128-byte line
 // in memory and in LDS, where its eight 16-byte chunks are permuted (mid_swz), so row reads
 // (ds_read_b128) and transposed reads (ds_read_b64_tr_b16) are both free of bank conflicts
 // without padding.  Stages are filled by direct global -> LDS loads two or three steps ahead;
@@ -15,6 +15,12 @@
 // of both together (256 x 128 tiles), so it is the overlap of the two inside a step; at the
 // small sizes it is the ends: of 12.6 us at 4096 x 2048 x 512, 1.5 are the launch, 4.5 the
 // first loads and the epilogue.
+//
+// The small tiles have 8 waves too, of 32 x 32 (64 x 128) or 64 x 32 (128 x 128) each: they read
+// a third to a half more from LDS than 4 waves of twice the width, but two waves a SIMD cover
+// each other's waits.  Input gradients 4096 x 512 x 1536 15.0 -> 13.7 us, 2048 x 768 x 3072
+// 25.2 -> 22.6; weight gradients 4096 x 1536 x 512 21.0 -> 20.1, 2048 x 3072 x 768 25.1 -> 23.0;
+// forwards 4096 x 512 x 2048 18.6 -> 16.3.
 #pragma once
 
 #include "fx_mfma.h"
@@ -122,7 +128,10 @@ struct MidRead {
         if constexpr (kind == kColK) {
             const uint16_t* t = tile + (r0 >> 6) * 4096 + kc * 1024;
             const int m = (r0 >> 5) & 1;
-            return cat8(lds_tr16(t + o[2 * m]), lds_tr16(t + o[2 * m + 1]));
+            // selected, not indexed: m differs between waves where a wave is 32 wide, and an array
+            // indexed at run time goes to LDS (8 KB a workgroup: + 10 us a product)
+            const int oa = m ? o[2] : o[0], ob = m ? o[3] : o[1];
+            return cat8(lds_tr16(t + oa), lds_tr16(t + ob));
         } else {
             return *reinterpret_cast<const bf16x8*>(tile + r0 * 64 + o[kc]);
         }

@@ -258,7 +258,7 @@ int mid_dgrad(const MidArgs& a, int tile, int gate, hipStream_t s) {
     if (tile == kMidBig)                                                                                                \
         hipLaunchKernelGGL((gemm_mid_kernel<256, 128, 2, 2, 3, kRowK, kColK, E>), dim3(tiles_of(a, 256, 128)), dim3(512), 0, s, a); \
     else                                                                                                                \
-        hipLaunchKernelGGL((gemm_mid_kernel<64, 128, 1, 2, 3, kRowK, kColK, E>), dim3(tiles_of(a, 64, 128)), dim3(256), 0, s, a);
+        hipLaunchKernelGGL((gemm_mid_kernel<64, 128, 1, 1, 3, kRowK, kColK, E>), dim3(tiles_of(a, 64, 128)), dim3(512), 0, s, a);
     if (gate == 2) {
         FX_MID(32)
     } else if (gate == 1) {
@@ -274,7 +274,7 @@ int mid_wgrad(const MidArgs& a, int tile, hipStream_t s) {
     if (tile == kMidBig)
         hipLaunchKernelGGL((gemm_mid_wgrad_kernel<256, 128, 2, 2, 3>), dim3(tiles_of(a, 256, 128) * a.slices), dim3(512), 0, s, a);
     else
-        hipLaunchKernelGGL((gemm_mid_wgrad_kernel<128, 128, 2, 2, 4>), dim3(tiles_of(a, 128, 128) * a.slices), dim3(256), 0, s, a);
+        hipLaunchKernelGGL((gemm_mid_wgrad_kernel<128, 128, 2, 1, 4>), dim3(tiles_of(a, 128, 128) * a.slices), dim3(512), 0, s, a);
     return check_launch("gemm_mid_wgrad");
 }
 

@@ -98,8 +98,8 @@ NATIVE_SMALL_INPUT_GRAD = True
 
 def small_dgrad(M, N, K):
     """Input gradients of up to 8,192 rows and 40 GFLOP, any row count, run on the small tiles
-    (a long K in slices), at least as fast there as the library GEMM: 4096 x 512 x 1536 15.9 us,
-    8192 x 256 x 768 9.2 (torch.mm: 19 us of host time alone), 4096 x 768 x 3072 35.3 against
+    (a long K in slices), at least as fast there as the library GEMM: 4096 x 512 x 1536 13.7 us,
+    8192 x 256 x 768 7.9 (torch.mm: 19 us of host time alone), 4096 x 768 x 3072 35.3 against
     37.0, 8192 x 3072 x 768 43.9 / 48.5, 8192 x 768 x 3072 47.2 / 48.2, 4096 x 512 x 8192 in 4
     slices 46 / 58; not 16384 x 768 x 768 (1 % on a block's forward and backward)."""
     return 0 < M <= 8192 and M * N * K <= 20 * 10 ** 9 and N % 8 == 0 and K % 8 == 0
