@@ -29,7 +29,6 @@ constexpr int kAttThreads = 64 * kAttWaves;
 constexpr int kBM = 32 * kAttWaves;  // queries per workgroup (forward, dQ)
 constexpr int kBN = 64;              // keys per streamed tile (forward, dQ)
 constexpr int kBK = 32 * kAttWaves;  // keys per workgroup (dK/dV)
-constexpr int kBQ = 64;              // queries per streamed tile (dK/dV)
 constexpr float kNegInfA = -__builtin_huge_valf();
 
 // Lazy rescaling (forward): the running max only moves when a row's new max exceeds
@@ -70,9 +69,17 @@ __device__ __forceinline__ void mask_rows(f32x16& x, int lo, int hi) {
 // heads for the end: 63 -> 50 us at [16,12,1024,64] causal forward).  Workgroups are
 // dealt round-robin to the 8 XCDs, so with nbh % 8 == 0 every tile of one head runs
 // on the same XCD and shares its L2.
-__device__ __forceinline__ void grid_map(int ntiles, int nbh, int& bh, int& tile) {
-    (void)ntiles;
-    const int x = blockIdx.x;
+//
+// REV (D = 128, two workgroups a CU): a causal grid of 257 to 512 workgroups is resident at
+// once, so nothing is left to fill a CU that got two light tiles; the second 256 are dealt
+// backwards (in groups of 8: a workgroup keeps its XCD), heavy beside light: 227.2 -> 219.4 us
+// for forward and backward at [4, 2048, 8, 128].  Not at D = 64, whose grids of that size hold
+// a third or fourth workgroup a CU (dK/dV 87.1 -> 89.9 us at [16, 1024, 12, 64] with it).
+template <bool REV>
+__device__ __forceinline__ void grid_map(bool causal, int nbh, int& bh, int& tile) {
+    int x = blockIdx.x;
+    const int total = gridDim.x;
+    if (REV && causal && x >= 256 && total <= 512 && total % 8 == 0) x = 256 + ((total - 264 - ((x - 256) & ~7)) | (x & 7));
     tile = x / nbh;
     bh = x - tile * nbh;
 }
@@ -120,7 +127,13 @@ __device__ __forceinline__ void store_rows(const f32x16 (&acc)[D / 32], float mu
 // Against the padded layout this drops one slot in nine from every tile load (the loads'
 // cost grows faster than their byte count: half the loads measured a third of their cost)
 // and the 2-way conflicts of the transposed reads.
-// D = 128: row stride D + 8 elements (the pad keeps the operand reads conflict-free).
+// Padded (the D = 64 forward): row stride D + 8 elements (the pad keeps the operand reads
+// conflict-free).
+// D = 128: 256-byte rows, each a full turn of the 64 banks, logical chunk c
+// of row r at c ^ swz(r), swz(r) = the low 4 bits of r reversed.  16 consecutive rows have 16
+// values of swz (row reads); the 4 rows of a transposed read differ in its two high bits and
+// its 4 chunks in the two low ones.  Against padded rows the forward and dQ took 225.1 -> 220.4 us
+// with dK/dV at [4, 2048, 8, 128] causal, 110.5 -> 107.5 at [2, 1000, 16, 128].
 template <int D, bool SW>
 struct TileLayout {
     static constexpr int LD = D + 8;       // row stride (elements)
@@ -142,6 +155,16 @@ struct TileLayout<64, true> {
     __device__ __forceinline__ static int chunk(int row, int slot) { return slot ^ swz(row); }
 };
 
+template <>
+struct TileLayout<128, true> {
+    static constexpr int LD = 128;
+    static constexpr int SPR = 16;
+    __device__ __forceinline__ static int swz(int row) {
+        return ((row & 1) << 3) | ((row & 2) << 1) | ((row & 4) >> 1) | ((row & 8) >> 3);
+    }
+    __device__ __forceinline__ static int chunk(int row, int slot) { return slot ^ swz(row); }
+};
+
 // MFMA operands from a tile in this layout (see fx_mfma.h for the lane mappings): K along a
 // row (8 contiguous elements of row r0 + l%32 at column c0 + 8 (l/32)), or K down the rows
 // (two ds_read_b64_tr_b16; a lane's 4 columns never cross a 16-byte chunk).  The kernels
@@ -151,6 +174,7 @@ struct TileLayout<64, true> {
 template <int D, bool SW>
 struct TileLane {
     __device__ __forceinline__ void init(int) {}
+    __device__ __forceinline__ const TileLane& fresh() const { return *this; }
     __device__ __forceinline__ int row(int r0, int c0, int lane) const {
         return TileLayout<D, SW>::off(r0 + (lane & 31), c0 + 8 * (lane >> 5));
     }
@@ -161,6 +185,7 @@ struct TileLane {
 };
 template <>
 struct TileLane<64, true> {
+    __device__ __forceinline__ const TileLane& fresh() const { return *this; }
     int ro[4];     // row reads at c0 = 16 c, rows 0..31
     int to[2][2];  // transposed reads at m0 = 32 m, rows 0..7 (h = 0) or 8..15 (h = 1)
     __device__ __forceinline__ void init(int lane) {
@@ -179,6 +204,31 @@ struct TileLane<64, true> {
     }
     __device__ __forceinline__ int row(int r0, int c0, int) const { return r0 * 64 + ro[c0 >> 4]; }
     __device__ __forceinline__ int tr(int k0, int m0, int h, int) const { return k0 * 64 + to[m0 >> 5][h]; }
+};
+// D = 128: the swizzle is an exclusive or with bits that the lane's base leaves free, so one
+// base per kind of read and a constant per chunk are enough (r0 and k0 as above)
+template <>
+struct TileLane<128, true> {
+    int rb, tb;
+    // the same bases, unknown to the compiler: the offsets derived from them are computed where
+    // they are used (one instruction each) and not kept in registers over the loop (67 spilled)
+    __device__ __forceinline__ TileLane fresh() const {
+        TileLane t = *this;
+        asm volatile("" : "+v"(t.rb), "+v"(t.tb));
+        return t;
+    }
+    __device__ __forceinline__ void init(int lane) {
+        const int g = lane >> 5, l32 = lane & 31;
+        rb = l32 * 128 + ((g ^ TileLayout<128, true>::swz(l32)) << 3);
+        const int grp = lane >> 4, s = lane & 15;
+        const int r = 4 * (grp >> 1) + (s >> 2);
+        const int cl = 2 * (grp & 1) + ((s & 3) >> 1);
+        tb = r * 128 + ((cl ^ TileLayout<128, true>::swz(r)) << 3) + 4 * (s & 1);
+    }
+    __device__ __forceinline__ int row(int r0, int c0, int) const { return r0 * 128 + (rb ^ c0); }
+    __device__ __forceinline__ int tr(int k0, int m0, int h, int) const {
+        return (k0 + 8 * h) * 128 + (tb ^ (m0 | (h << 3)));
+    }
 };
 template <int D, bool SW>
 __device__ __forceinline__ bf16x8 tile_op_row(const TileLane<D, SW>& tl, const uint16_t* tile, int r0, int c0, int lane) {
@@ -300,9 +350,9 @@ __device__ __forceinline__ float pair_sum(float x) {
 
 template <int D>
 __global__ void __launch_bounds__(kAttThreads) attn_fwd_kernel(fxAttnArgs a) {
-    // padded tiles: the swizzle's per-lane offset table would take the forward past 128
+    // D = 64, padded tiles: the swizzle's per-lane offset table would take the forward past 128
     // VGPRs (3 waves per SIMD instead of 4), and its tile loads cost it little
-    constexpr bool SW = false;
+    constexpr bool SW = D == 128;
     constexpr int LD = TileLayout<D, SW>::LD;
     constexpr int DC = D / 16;  // K chunks of Q.K
     constexpr int DT = D / 32;  // 32-row tiles of O^T
@@ -313,7 +363,7 @@ __global__ void __launch_bounds__(kAttThreads) attn_fwd_kernel(fxAttnArgs a) {
     const int T = a.T;
     const int nqt = (T + kBM - 1) / kBM;
     int bh, qt;
-    grid_map(nqt, a.B * a.H, bh, qt);
+    grid_map<D == 128>(a.causal, a.B * a.H, bh, qt);
     qt = nqt - 1 - qt;  // longest causal tiles first
     const int b = bh / a.H, h = bh - b * a.H;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -355,6 +405,7 @@ __global__ void __launch_bounds__(kAttThreads) attn_fwd_kernel(fxAttnArgs a) {
     for (int dt = 0; dt < DT; ++dt) acc[dt] = f32x16{};
 
     // one 64-key tile: K/V in (K, V); the next tile's loads go to (nK, nV)
+    const TileLane<D, SW> tl0 = tl;
     auto step = [&](int j, const uint16_t* K, const uint16_t* V, uint16_t* nK, uint16_t* nV) {
         const int kb = j * kBN;
         tile_arrive();
@@ -363,6 +414,7 @@ __global__ void __launch_bounds__(kAttThreads) attn_fwd_kernel(fxAttnArgs a) {
         if (j + 1 < nblk) dma.issue(kn, vn, T - kb - kBN, nK, nV);
 #pragma unroll
         for (int hh = 0; hh < 2; ++hh) {
+            const auto tl = tl0.fresh();
             const int kh = kb + 32 * hh;  // first key of this half
             if (kh >= T || (a.causal && kh > q0w + 31)) continue;  // every key masked for this wave
             bf16x8 kop[DC];
@@ -431,7 +483,7 @@ __global__ void __launch_bounds__(kAttThreads) attn_fwd_kernel(fxAttnArgs a) {
     if (qi < T && g == 0)
         a.lse_out[(int64_t)bh * T + qi] = l_tot > 0.f ? (m_run + log2_fast(l_tot)) * kLn2 : kNegInfA;
     __syncthreads();  // every wave is done with the K/V stages: they become store scratch
-    store_rows<D>(acc, l_tot > 0.f ? 1.f / l_tot : 0.f, (wave < 2 ? sk0 : sk1) + (wave & 1) * 32 * LD,
+    store_rows<D>(acc, l_tot > 0.f ? 1.f / l_tot : 0.f, wave == 0 ? sk0 : wave == 1 ? sk1 : wave == 2 ? sv0 : sv1,
                   a.o_out + (((int64_t)b * T + q0w) * a.H + h) * D, (int64_t)a.H * D, T - q0w, lane);
 }
 
@@ -440,7 +492,7 @@ __global__ void __launch_bounds__(kAttThreads) attn_fwd_kernel(fxAttnArgs a) {
 
 template <int D>
 __global__ void __launch_bounds__(kAttThreads, D == 64 ? 2 : 1) attn_bwd_dq_kernel(fxAttnArgs a) {
-    constexpr bool SW = D == 64;  // swizzled tiles: 9 % fewer tile loads, no transposed-read conflicts
+    constexpr bool SW = true;  // swizzled tiles: 9 % fewer tile loads, no transposed-read conflicts
     constexpr int LD = TileLayout<D, SW>::LD;
     constexpr int DC = D / 16;
     constexpr int DT = D / 32;
@@ -451,7 +503,7 @@ __global__ void __launch_bounds__(kAttThreads, D == 64 ? 2 : 1) attn_bwd_dq_kern
     const int T = a.T;
     const int nqt = (T + kBM - 1) / kBM;
     int bh, qt;
-    grid_map(nqt, a.B * a.H, bh, qt);
+    grid_map<D == 128>(a.causal, a.B * a.H, bh, qt);
     qt = nqt - 1 - qt;
     const int b = bh / a.H, h = bh - b * a.H;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -516,6 +568,7 @@ __global__ void __launch_bounds__(kAttThreads, D == 64 ? 2 : 1) attn_bwd_dq_kern
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) acc[dt] = f32x16{};
 
+    const TileLane<D, SW> tl0 = tl;
     auto step = [&](int j, const uint16_t* K, const uint16_t* V, uint16_t* nK, uint16_t* nV) {
         const int kb = j * kBN;
         tile_arrive();
@@ -524,6 +577,7 @@ __global__ void __launch_bounds__(kAttThreads, D == 64 ? 2 : 1) attn_bwd_dq_kern
         if (j + 1 < nblk) dma.issue(kn, vn, T - kb - kBN, nK, nV);
 #pragma unroll
         for (int hh = 0; hh < 2; ++hh) {
+            const auto tl = tl0.fresh();
             const int kh = kb + 32 * hh;
             if (kh >= T || (a.causal && kh > q0w + 31)) continue;
             // S^T = K Q^T and dP^T = V dO^T, operands read chunk by chunk (few live registers)
@@ -564,25 +618,36 @@ __global__ void __launch_bounds__(kAttThreads, D == 64 ? 2 : 1) attn_bwd_dq_kern
 
 // ---------------------------------------------------------------------------
 // backward, key side: dK and dV
+//
+// D = 128: the two accumulators take 128 registers and the K and V operands 64 more, which
+// left one wave per SIMD (294 registers) and every LDS and MFMA latency in the open.  The V
+// rows stay in LDS instead, read as an operand like the streamed tiles, and the streamed tiles
+// have 32 queries, so that two workgroups fit a CU (67 KB, <= 256 registers): 70.0 -> 59.4 us
+// at [8, 1000, 8, 128] causal (468 -> 552 TFLOP/s), the same bits.
 
 template <int D>
-__global__ void __launch_bounds__(kAttThreads, D == 64 ? 2 : 1) attn_bwd_dkv_kernel(fxAttnArgs a) {
-    constexpr bool SW = D == 64;
+__global__ void __launch_bounds__(kAttThreads, 2) attn_bwd_dkv_kernel(fxAttnArgs a) {
+    constexpr bool SW = true;
+    constexpr bool VL = D == 128;          // V rows in LDS
+    constexpr int kBQ = D == 64 ? 64 : 32;  // queries per streamed tile
     constexpr int LD = TileLayout<D, SW>::LD;
     constexpr int DC = D / 16;
     constexpr int DT = D / 32;
     __shared__ __attribute__((aligned(16))) uint16_t sq0[kBQ * LD], sq1[kBQ * LD];
     __shared__ __attribute__((aligned(16))) uint16_t sdo0[kBQ * LD], sdo1[kBQ * LD];
-    static_assert(32 * (D + 8) <= kBQ * LD, "a stage buffer holds one wave's output staging");
+    static_assert(VL || 32 * (D + 8) <= kBQ * LD, "a stage buffer holds one wave's output staging");
+    // a wave's 32 rows of V, and with them its output staging (32 x (D + 8))
+    constexpr int VW = 32 * (D + 8);
+    __shared__ __attribute__((aligned(16))) uint16_t sv[VL ? kAttWaves * VW : 8];
     __shared__ __attribute__((aligned(16))) float slse[2][kBQ];
     __shared__ __attribute__((aligned(16))) float sdelta[2][kBQ];
 
     const int T = a.T;
-    const int nkt = (T + kBK - 1) / kBK;
     int bh, kt;
-    grid_map(nkt, a.B * a.H, bh, kt);  // key tile 0 (most causal work) first
+    grid_map<D == 128>(a.causal, a.B * a.H, bh, kt);  // key tile 0 (most causal work) first
     const int b = bh / a.H, h = bh - b * a.H;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int wave_u = __builtin_amdgcn_readfirstlane(wave);
     const int g = lane >> 5, ln = lane & 31;
     TileLane<D, SW> tl;
     tl.init(lane);
@@ -623,9 +688,20 @@ __global__ void __launch_bounds__(kAttThreads, D == 64 ? 2 : 1) attn_bwd_dkv_ker
     };
     if (nblk > 0) issue(qstart, sq0, sdo0);
 
+    if constexpr (VL) {  // this wave's V rows, slot by slot (rows past T: zeros); arrived at the first tile's wait
+        const uint16_t* vrows = a.v + b * a.vsb + h * a.vsh;
+#pragma unroll
+        for (int i = 0; i < 32 * (D / 8) / 64; ++i) {
+            const int s = i * 64 + lane, r = s / (D / 8), c = TileLayout<D, SW>::chunk(r, s % (D / 8));
+            const int key = k0w + r;
+            dma16(key < T ? (const void*)(vrows + (int64_t)key * a.vst + c * 8) : (const void*)g_zero_line,
+                  lds_addr(sv + wave_u * VW + i * 64 * 8));
+        }
+    }
+
     // K and V rows of this lane's key: every load issued before any is used (rows past T
     // read row 0 and are zeroed after)
-    bf16x8 kop[DC], vop[DC];
+    bf16x8 kop[DC], vop[VL ? 1 : DC];
     {
         const uint16_t* krow = a.k + b * a.ksb + h * a.ksh + (int64_t)(kok ? ki : 0) * a.kst;
         const uint16_t* vrow = a.v + b * a.vsb + h * a.vsh + (int64_t)(kok ? ki : 0) * a.vst;
@@ -633,13 +709,13 @@ __global__ void __launch_bounds__(kAttThreads, D == 64 ? 2 : 1) attn_bwd_dkv_ker
 #pragma unroll
         for (int c = 0; c < DC; ++c) {
             kv[c] = ld16(krow + 16 * c + 8 * g);
-            vv[c] = ld16(vrow + 16 * c + 8 * g);
+            if constexpr (!VL) vv[c] = ld16(vrow + 16 * c + 8 * g);
         }
         const uint32_t keep = kok ? ~0u : 0u;
 #pragma unroll
         for (int c = 0; c < DC; ++c) {
             kop[c] = as_bf16x8(mask16(kv[c], keep));
-            vop[c] = as_bf16x8(mask16(vv[c], keep));
+            if constexpr (!VL) vop[c] = as_bf16x8(mask16(vv[c], keep));
         }
     }
     const float sl2 = a.scale * kLog2e;
@@ -651,6 +727,9 @@ __global__ void __launch_bounds__(kAttThreads, D == 64 ? 2 : 1) attn_bwd_dkv_ker
         adk[dt] = f32x16{};
     }
 
+    // the wave's V rows start at a multiple of the 128 elements that the swizzle stays within
+    static_assert(VW % 128 == 0, "V rows of a wave");
+    const TileLane<D, SW> tl0 = tl;
     auto step = [&](int j, const uint16_t* Q, const uint16_t* DO, uint16_t* nQ, uint16_t* nDO) {
         const int qb = qstart + j * kBQ;
         const int st = j & 1;
@@ -662,7 +741,8 @@ __global__ void __launch_bounds__(kAttThreads, D == 64 ? 2 : 1) attn_bwd_dkv_ker
         __syncthreads();
         if (j + 1 < nblk) issue(qb + kBQ, nQ, nDO);
 #pragma unroll
-        for (int hh = 0; hh < 2; ++hh) {
+        for (int hh = 0; hh < kBQ / 32; ++hh) {
+            const TileLane<D, SW> tl = tl0.fresh();
             const int qh = qb + 32 * hh;  // first query of this half
             if (qh >= T || (a.causal && qh + 31 < k0w)) continue;  // all of this wave's keys follow these queries
             // S = Q K^T and dP = dO V^T, operands read chunk by chunk (few live registers)
@@ -672,7 +752,8 @@ __global__ void __launch_bounds__(kAttThreads, D == 64 ? 2 : 1) attn_bwd_dkv_ker
                 const bf16x8 qa = tile_op_row(tl, Q, 32 * hh, 16 * c, lane);
                 const bf16x8 da = tile_op_row(tl, DO, 32 * hh, 16 * c, lane);
                 s = mfma32(qa, kop[c], s);
-                dp = mfma32(da, vop[c], dp);
+                if constexpr (VL) dp = mfma32(da, tile_op_row(tl, sv + wave_u * VW, 0, 16 * c, lane), dp);
+                else dp = mfma32(da, vop[c], dp);
             }
             if ((qh + 32 > T) || (a.causal && qh < k0w + 31))  // queries past T or before the key
                 mask_rows(s, a.causal ? ki - qh - 4 * g : INT32_MIN, T - 1 - qh - 4 * g);
@@ -714,7 +795,7 @@ __global__ void __launch_bounds__(kAttThreads, D == 64 ? 2 : 1) attn_bwd_dkv_ker
     }
 
     __syncthreads();  // every wave is done with the Q/dO stages: they become store scratch
-    uint16_t* tmp = wave == 0 ? sq0 : wave == 1 ? sq1 : wave == 2 ? sdo0 : sdo1;
+    uint16_t* tmp = VL ? sv + wave * VW : wave == 0 ? sq0 : wave == 1 ? sq1 : wave == 2 ? sdo0 : sdo1;
     store_rows<D>(adk, a.scale, tmp, a.dk + b * a.dkb + h * a.dkh + (int64_t)k0w * a.dkt, a.dkt, T - k0w, lane);
     store_rows<D>(adv, 1.f, tmp, a.dv + b * a.dvb + h * a.dvh + (int64_t)k0w * a.dvt, a.dvt, T - k0w, lane);
 }

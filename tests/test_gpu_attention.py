@@ -63,6 +63,14 @@ def test_against_oracle(dev, causal, B, T, H, Dh):
     _check(got, (ro, rl, rdq, rdk, rdv))
 
 
+# D = 128: key tiles of 128 and query tiles of 32 that end early, more workgroups than CUs
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("B,T,H,Dh", [(12, 300, 8, 128), (24, 200, 8, 128), (1, 31, 2, 128), (1, 32, 1, 128),
+                                      (2, 161, 3, 128), (1, 1, 1, 128)])
+def test_d128_tile_ends(dev, causal, B, T, H, Dh):
+    test_against_oracle(dev, causal, B, T, H, Dh)
+
+
 @pytest.mark.parametrize("causal", [True, False])
 def test_qkv_variant(dev, causal):
     from fxlm.attention import flash_attention_qkv
