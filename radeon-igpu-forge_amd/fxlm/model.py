@@ -364,7 +364,7 @@ class _DecodeGraph:
     def __call__(self, tok, pos):
         if pos >= self.cache_len:
             raise ValueError(f"position {pos} is past the cache ({self.cache_len})")
-        if not (torch.is_tensor(tok) and host.decode_inputs(tok, pos, self.tok, self.pos, self.lens)):
+        if not (torch.is_tensor(tok) and host.decode_inputs(tok, int(pos), self.tok, self.pos, self.lens)):
             self.tok.copy_(tok)
             self.pos.fill_(pos)
             self.lens.fill_(pos + 1)

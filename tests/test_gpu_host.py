@@ -84,3 +84,17 @@ def test_decode_step_ends_equal_the_torch_operations(dev, B, V, D):
     assert torch.equal(x, torch.nn.functional.embedding(tok, E)[:, None] + P.index_select(0, pos))
     w = torch.ones(D, device=dev).bfloat16()
     assert torch.equal(host.few_rows_logits(x[:, 0], E, w, 1e-6), linear_ex(x[:, 0], E, norm_weight=w, eps=1e-6).float())
+
+
+def test_decode_graph_takes_positions_of_any_number_type(dev):
+    # a position as a float, a numpy integer or a 0-d tensor, as fill_() takes them
+    import numpy as np
+    from fxlm import GPT, GPTConfig
+    torch.manual_seed(3)
+    with torch.device(dev):
+        model = GPT(GPTConfig(vocab_size=256, seq_len=64, n_layer=1, n_head=2, d_model=128)).bfloat16()
+    cache = [tuple(torch.zeros(2, 64, 2, 64, device=dev).bfloat16() for _ in range(2))]
+    step, tok = model.decode_graph(cache, 2), torch.tensor([5, 9], device=dev)
+    want = step(tok, 7).clone()
+    for pos in (7.0, np.int64(7), torch.tensor(7), torch.tensor(7, device=dev)):
+        assert torch.equal(step(tok, pos), want), type(pos)
