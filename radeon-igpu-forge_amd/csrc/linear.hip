@@ -1387,10 +1387,10 @@ wgrad_reduce_kernel(const float* __restrict__ part, int slices, int64_t MN, int 
 // global memory in 16-byte row chunks (lane l takes row l%16 and k = k0 + 8(l/16) +
 // 0..7 in both operands: the K order inside one instruction is the same for the two,
 // so the product is the plain contraction); the accumulator lane l holds column
-// (X row) l%16 and rows (W rows) 4(l/16) + 0..3.  A workgroup owns 16 NT rows of W and
-// its sw waves split the K steps of 32; each wave keeps NT x MT accumulator tiles.
-// The partial tiles meet in LDS and are summed in wave order (deterministic), then
-// + bias, activation and the stores.  Gathered rows work as in the tiled kernel; the
+// (X row) l%16 and rows (W rows) 4(l/16) + 0..3.  The K steps of 32 are split into sw ranges
+// (skinny_waves); a range is one chain of MFMAs and the ranges' sums are added in order, then
+// + bias, activation and the stores.  Tiles, waves and kernels below differ in who runs a range,
+// not in the ranges or their order, so an output's bits are a function of M, N, K and the CU count.  Gathered rows work as in the tiled kernel; the
 // first workgroup writes them out (Xg) while it streams them.
 constexpr int kSKMaxM = 64;
 constexpr int kSKMaxTiles = 16;  // sw * NT * MT: 1 KB of LDS per accumulator tile
@@ -1409,6 +1409,8 @@ __device__ __forceinline__ const uint16_t* xrow_base(const GemmArgs& a, int m) {
     return a.A + (int64_t)m * a.lda;
 }
 
+// K steps per load batch: as many as the 128 registers of 16 waves hold (one round trip to
+// memory per batch; most layers' waves have a single one)
 static constexpr int skinny_batch(int nt, int mt, bool norm) {
     return nt * mt >= 8 && norm ? 1 : nt * mt >= (norm ? 3 : 4) ? 2 : nt * mt == 1 && !norm ? 8 : 4;
 }
@@ -1420,10 +1422,18 @@ __device__ __forceinline__ uint4 ld16_if(bool ok, const uint16_t* p) {
     return v;
 }
 
-// sum over the sw waves' partials (stride `vals` floats), in wave order; four at a time so that
-// their LDS reads overlap
+// sum over the sw K ranges' partials (stride `vals` floats; sw a power of two), in their order; all
+// of 16 (or 4) are read before the first is added, one LDS round trip and not one per four
 __device__ __forceinline__ float skinny_sum(const float* p, int vals, int sw) {
     float sum = 0.f;
+    if (sw == 16) {
+        float v[16];
+#pragma unroll
+        for (int w = 0; w < 16; ++w) v[w] = p[w * vals];
+#pragma unroll
+        for (int w = 0; w < 16; ++w) sum += v[w];
+        return sum;
+    }
     int w = 0;
     for (; w + 4 <= sw; w += 4) {
         const float v0 = p[w * vals], v1 = p[(w + 1) * vals], v2 = p[(w + 2) * vals], v3 = p[(w + 3) * vals];
@@ -1436,8 +1446,8 @@ __device__ __forceinline__ float skinny_sum(const float* p, int vals, int sw) {
     return sum;
 }
 
-// bias, activation, residual and the store of one output value
-__device__ __forceinline__ void skinny_store(const GemmArgs& a, float sum, int m, int n) {
+// bias, activation and residual of one output value: its bf16 result (H is stored on the way)
+__device__ __forceinline__ uint16_t skinny_value(const GemmArgs& a, float sum, int m, int n) {
     const float h = sum + (a.bias ? bf16_to_f32(a.bias[n]) : 0.f);
     float y = h;
     if (a.act == 2) {
@@ -1449,68 +1459,116 @@ __device__ __forceinline__ void skinny_store(const GemmArgs& a, float sum, int m
         if (a.act == 1) y = gelu_tanh(h);
     }
     if (a.res) y += bf16_to_f32(a.res[(int64_t)m * a.ldres + n]);
-    const uint16_t o = f32_to_bf16(y);
-    if (a.C32) a.C32[(int64_t)m * a.N + n] = bf16_to_f32(o);
-    else a.C[(int64_t)m * a.ldc + n] = o;
+    return f32_to_bf16(y);
 }
 
-// rstd of the rows of X from the operands of one batch that spans each wave's K range: the sum
-// of squares over a wave's lanes, then over the waves in order.  `red` is scratch (free again
-// after the call's last barrier).
-template <int U, int MT>
-__device__ __forceinline__ void skinny_rstd(const GemmArgs& a, const uint4 (&xv)[U][MT], float* red, int sw, int w, int lane,
-                                            float (&rs)[MT]) {
-    const int r = lane & 15, kg = lane >> 4;
+template <int CTRL>
+__device__ __forceinline__ float dpp_move(float v) {
+    return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), CTRL, 0xf, 0xf, true));
+}
+// group_sum<64>'s sum, pairing for pairing (so bit for bit), without its six LDS round trips
+__device__ __forceinline__ float wave_sum_alu(float x) {
+    const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    x = __uint_as_float(h[0]) + __uint_as_float(h[1]);
+    const auto q = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    x = __uint_as_float(q[0]) + __uint_as_float(q[1]);
+    x += dpp_move<0x128>(x);                   // lane ^ 8: rotated by 8 in its row of 16
+    x += dpp_move<0x1b>(dpp_move<0x141>(x));   // ^ 4: half rows mirrored (^ 7), quads mirrored (^ 3)
+    x += dpp_move<0x4e>(x);                    // ^ 2
+    x += dpp_move<0xb1>(x);                    // ^ 1
+    return x;
+}
+
+// rstd of every row of X into srstd: wave v of nw sums rows v, v + nw, ... (a lane's chunks of 8 in
+// order, then a butterfly over the lanes: the same sum at any number of waves).  R rows of C
+// chunks a lane are loaded at a time (unconditionally, at a clamped address: a wait for loads
+// behind branches would cover the operands' loads too); where that is all of a wave's rows,
+// load_first() asks for them before the kernel asks for its operands, whose way the sums then
+// overlap: 16 rows of 768 into 2304 6.8 -> 5.6 us, 64 rows 24.7 -> 11.0 (row by row, before the
+// operands' loads).
+template <int R, int C>
+struct SkinnyRstd {
+    uint4 v[C][R];
+    // one group of loads has all of a wave's rows
+    __device__ __forceinline__ static bool one(const GemmArgs& a, int nw) { return a.M <= R * nw && a.K <= 512 * C; }
+    __device__ __forceinline__ void load(const GemmArgs& a, int mb, int c0, int nw, int lane) {
 #pragma unroll
-    for (int j = 0; j < MT; ++j) {
-        float q = 0.f;
+        for (int t = 0; t < R; ++t) {
+            const uint16_t* row = a.A + (int64_t)min(mb + t * nw, a.M - 1) * a.lda;
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            float f[8];
-            unpack8(xv[u][j], f);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) q = fmaf(f[e], f[e], q);
+            for (int i = 0; i < C; ++i) v[i][t] = ld16(row + (int64_t)min(c0 + 64 * i + lane, a.K / 8 - 1) * 8);
         }
-        q += __shfl_xor(q, 16, 64);
-        q += __shfl_xor(q, 32, 64);
-        if (kg == 0) red[w * (16 * MT) + 16 * j + r] = q;
     }
-    __syncthreads();
+    __device__ __forceinline__ void add(const GemmArgs& a, int c0, int lane, float (&q)[R]) const {
 #pragma unroll
-    for (int j = 0; j < MT; ++j) {
-        const float q = skinny_sum(red + 16 * j + r, 16 * MT, sw);
-        rs[j] = 16 * j + r < a.M ? 1.f / sqrtf(q / (float)a.K + a.eps) : 0.f;
+        for (int i = 0; i < C; ++i) {
+            const bool in = c0 + 64 * i + lane < a.K / 8;
+#pragma unroll
+            for (int t = 0; t < R; ++t) {
+                float f[8], p = q[t];
+                unpack8(v[i][t], f);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) p = fmaf(f[e], f[e], p);
+                q[t] = in ? p : q[t];
+            }
+        }
     }
-    __syncthreads();
-}
+    __device__ __forceinline__ static void put(const GemmArgs& a, int mb, int nw, int lane, const float (&q)[R], float* srstd) {
+#pragma unroll
+        for (int t = 0; t < R; ++t) {
+            const float sum = wave_sum_alu(q[t]);
+            if (lane == 0 && mb + t * nw < a.M) srstd[mb + t * nw] = 1.f / sqrtf(sum / (float)a.K + a.eps);
+        }
+    }
+    __device__ __forceinline__ void load_first(const GemmArgs& a, int nw, int w, int lane) {
+        if (one(a, nw)) load(a, w, 0, nw, lane);
+    }
+    __device__ __forceinline__ void finish(const GemmArgs& a, int nw, int w, int lane, float* srstd) const {
+        if (one(a, nw)) {
+            float q[R] = {};
+            add(a, 0, lane, q);
+            put(a, w, nw, lane, q, srstd);
+        } else {
+            using Some = SkinnyRstd<4, 1>;
+            for (int mb = w; mb < a.M; mb += 4 * nw) {
+                float q[4] = {};
+                for (int c0 = 0; c0 < a.K / 8; c0 += 64) {
+                    Some s;
+                    s.load(a, mb, c0, nw, lane);
+                    s.add(a, c0, lane, q);
+                }
+                Some::put(a, mb, nw, lane, q, srstd);
+            }
+        }
+        __syncthreads();
+    }
+};
 
-// x * rstd * nw of one K step, rounded to bf16 as the norm kernel writes them
-template <int MT>
-__device__ __forceinline__ void skinny_normalise(uint4 (&xv)[MT], const uint4& nv, const float (&rs)[MT]) {
-    float fw[8];
+// x * rstd * nw of 8 values, rounded to bf16 as the norm kernel writes them
+__device__ __forceinline__ uint4 skinny_normalise(const uint4& x, const uint4& nv, float rs) {
+    float f[8], fw[8];
+    unpack8(x, f);
     unpack8(nv, fw);
 #pragma unroll
-    for (int j = 0; j < MT; ++j) {
-        float f[8];
-        unpack8(xv[j], f);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) f[e] = f[e] * rs[j] * fw[e];
-        xv[j] = pack8(f);
-    }
+    for (int e = 0; e < 8; ++e) f[e] = f[e] * rs * fw[e];
+    return pack8(f);
 }
 
-template <int NT, int MT, bool NORM>
+// rows of X that a wave sums at a time with the norm (two chunks of 64 lanes each)
+static constexpr int skinny_rows(int mt) { return mt <= 2 ? 2 : 4; }
+
+// A workgroup owns tr NT rows of W (tr < 16: the MFMAs' other rows are zeros); its wave w takes the K
+// range w of sw and keeps NT x MT accumulator tiles, which meet in LDS; waves past sw (with the
+// norm) only help to sum the squares.  U: K steps per load batch.
+template <int NT, int MT, bool NORM, int U>
 __global__ void __launch_bounds__(1024) gemm_skinny_kernel(GemmArgs a, int sw, int tr) {
-    // K steps per load batch: as many as the 128 registers of 16 waves hold (one round trip to
-    // memory per batch; most layers' waves have a single one)
-    constexpr int U = skinny_batch(NT, MT, NORM);
     __shared__ __attribute__((aligned(16))) float red[kSKMaxTiles * 256];
     const int lane = threadIdx.x & 63;
-    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
     const int r = lane & 15, kg = lane >> 4;
     const int n0 = blockIdx.x * tr * NT;
     const int ks = (a.K + 31) / 32;
-    const int kb = w * ks / sw, ke = (w + 1) * ks / sw;
+    const int kb = min(w, sw) * ks / sw, ke = min(w + 1, sw) * ks / sw;
 
     const uint16_t* wrow[NT];
 #pragma unroll
@@ -1539,47 +1597,19 @@ __global__ void __launch_bounds__(1024) gemm_skinny_kernel(GemmArgs a, int sw, i
             if constexpr (NORM) nv[u] = ld16_if(ok, a.nw + s * 32 + 8 * kg);
         }
     };
-    load(kb);
-
     // NORM: A rows are RMS-normalised on the fly, x * rstd[m] * nw[k] rounded to bf16 as
-    // the norm kernel writes them.  Each workgroup first computes rstd of every row.  Where the
-    // first batch is a wave's whole K range (the host asks for that many waves when it can), the
-    // squares come from the operands just loaded: lanes, then waves, in a fixed order, and no
-    // second read of x (a 768 x 2304 product of 16 rows 6.4 -> 4.7 us, 4.0 without the norm).
-    // Otherwise wave v sums rows v, v + sw, ..., four rows' loads issued at a time.
+    // the norm kernel writes them; each workgroup computes rstd of every row itself
     __shared__ float srstd[kSKMaxM];
     float rs[MT];
     if constexpr (NORM) {
-        if ((ks + sw - 1) / sw <= U) {
-            skinny_rstd<U, MT>(a, xv, red, sw, w, lane, rs);
-        } else {
-            for (int mb = w; mb < a.M; mb += 4 * sw) {
-                const uint16_t* row[4];
-                float q[4] = {0.f, 0.f, 0.f, 0.f};
+        SkinnyRstd<skinny_rows(MT), 2> sums;
+        sums.load_first(a, nw, w, lane);
+        load(kb);
+        sums.finish(a, nw, w, lane, srstd);
 #pragma unroll
-                for (int t = 0; t < 4; ++t) row[t] = mb + t * sw < a.M ? xrow_base(a, mb + t * sw) : nullptr;
-                for (int c = lane; c < a.K / 8; c += 64) {
-                    uint4 v[4];
-#pragma unroll
-                    for (int t = 0; t < 4; ++t) v[t] = ld16_if(row[t] != nullptr, row[t] + c * 8);
-#pragma unroll
-                    for (int t = 0; t < 4; ++t) {
-                        float f[8];
-                        unpack8(v[t], f);
-#pragma unroll
-                        for (int e = 0; e < 8; ++e) q[t] = fmaf(f[e], f[e], q[t]);
-                    }
-                }
-#pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    const float sum = group_sum<64>(q[t]);
-                    if (lane == 0 && mb + t * sw < a.M) srstd[mb + t * sw] = 1.f / sqrtf(sum / (float)a.K + a.eps);
-                }
-            }
-            __syncthreads();
-#pragma unroll
-            for (int j = 0; j < MT; ++j) rs[j] = 16 * j + r < a.M ? srstd[16 * j + r] : 0.f;
-        }
+        for (int j = 0; j < MT; ++j) rs[j] = 16 * j + r < a.M ? srstd[16 * j + r] : 0.f;
+    } else {
+        load(kb);
     }
 
     f32x4 acc[NT][MT];
@@ -1591,7 +1621,9 @@ __global__ void __launch_bounds__(1024) gemm_skinny_kernel(GemmArgs a, int sw, i
         if (s0 > kb) load(s0);
         if constexpr (NORM) {
 #pragma unroll
-            for (int u = 0; u < U; ++u) skinny_normalise<MT>(xv[u], nv[u], rs);
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int j = 0; j < MT; ++j) xv[u][j] = skinny_normalise(xv[u][j], nv[u], rs[j]);
         }
         if (wxg) {
 #pragma unroll
@@ -1612,11 +1644,13 @@ __global__ void __launch_bounds__(1024) gemm_skinny_kernel(GemmArgs a, int sw, i
 #pragma unroll
                 for (int j = 0; j < MT; ++j) acc[i][j] = mfma16(wv[u][i], xv[u][j], acc[i][j]);
     }
+    if (w < sw) {
 #pragma unroll
-    for (int i = 0; i < NT; ++i)
+        for (int i = 0; i < NT; ++i)
 #pragma unroll
-        for (int j = 0; j < MT; ++j)
-            *reinterpret_cast<f32x4*>(&red[((w * NT + i) * MT + j) * 256 + lane * 4]) = acc[i][j];
+            for (int j = 0; j < MT; ++j)
+                *reinterpret_cast<f32x4*>(&red[((w * NT + i) * MT + j) * 256 + lane * 4]) = acc[i][j];
+    }
     __syncthreads();
     // value (tile, m_local, n_local), n_local fastest so neighbouring threads store
     // neighbouring columns; in the accumulator layout it sits at lane m_local +
@@ -1626,131 +1660,241 @@ __global__ void __launch_bounds__(1024) gemm_skinny_kernel(GemmArgs a, int sw, i
         const int tile = v >> 8, ml = (v >> 4) & 15, nl = v & 15;
         const int off = tile * 256 + (ml + 16 * (nl >> 2)) * 4 + (nl & 3);
         const int n = n0 + 16 * (tile / MT) + nl, m = 16 * (tile % MT) + ml;
-        if (n < a.N && m < a.M && nl < tr) skinny_store(a, skinny_sum(red + off, kVals, sw), m, n);
-    }
-}
-
-// The same product for a wide W (a head: 50,304 rows of 768): a workgroup keeps its X operands
-// (normalised once) in registers and walks the 16-row tiles of W, the next tile's rows loading
-// during the current one's products and sums.  One workgroup per tile read X and summed its
-// squares 1,572 times over: 40 us for 16 rows, 26 this way (3 TB/s of W).  Every wave's K
-// range is one batch of kSKLoopU steps (the host checks); the partial tiles alternate between
-// two LDS buffers, so a tile costs one barrier.
-constexpr int kSKLoopU = 4;
-template <int MT, bool NORM>
-__global__ void __launch_bounds__(1024) gemm_skinny_loop_kernel(GemmArgs a, int sw, int ntiles) {
-    constexpr int U = kSKLoopU, kVals = MT * 256;
-    extern __shared__ __attribute__((aligned(16))) float lred[];   // 2 x sw x kVals
-    const int lane = threadIdx.x & 63;
-    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int r = lane & 15, kg = lane >> 4;
-    const int ks = (a.K + 31) / 32;
-    const int kb = w * ks / sw, ke = (w + 1) * ks / sw;
-    uint4 wv[U], xv[U][MT];
-    auto load_w = [&](int t) {
-        const int n = 16 * t + r;
-        const uint16_t* row = a.B + (int64_t)(n < a.N ? n : 0) * a.ldb + 8 * kg;
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-            wv[u] = ld16_if(t < ntiles && n < a.N && kb + u < ke && (kb + u) * 32 + 8 * kg < a.K, row + (kb + u) * 32);
-    };
-    load_w(blockIdx.x);
-#pragma unroll
-    for (int j = 0; j < MT; ++j) {
-        const int m = 16 * j + r;
-        const uint16_t* row = a.A + (int64_t)(m < a.M ? m : 0) * a.lda + 8 * kg;
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-            xv[u][j] = ld16_if(m < a.M && kb + u < ke && (kb + u) * 32 + 8 * kg < a.K, row + (kb + u) * 32);
-    }
-    if constexpr (NORM) {
-        uint4 nv[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-            nv[u] = ld16_if(kb + u < ke && (kb + u) * 32 + 8 * kg < a.K, a.nw + (kb + u) * 32 + 8 * kg);
-        float rs[MT];
-        skinny_rstd<U, MT>(a, xv, lred, sw, w, lane, rs);
-#pragma unroll
-        for (int u = 0; u < U; ++u) skinny_normalise<MT>(xv[u], nv[u], rs);
-    }
-    int p = 0;
-    for (int t = blockIdx.x; t < ntiles; t += gridDim.x, p ^= 1) {
-        f32x4 acc[MT];
-#pragma unroll
-        for (int j = 0; j < MT; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-#pragma unroll
-            for (int j = 0; j < MT; ++j) acc[j] = mfma16(wv[u], xv[u][j], acc[j]);
-        load_w(t + gridDim.x);
-        float* red = lred + p * sw * kVals;
-#pragma unroll
-        for (int j = 0; j < MT; ++j) *reinterpret_cast<f32x4*>(&red[(w * MT + j) * 256 + lane * 4]) = acc[j];
-        __syncthreads();
-        for (int v = threadIdx.x; v < kVals; v += blockDim.x) {
-            const int tile = v >> 8, ml = (v >> 4) & 15, nl = v & 15;
-            const int off = tile * 256 + (ml + 16 * (nl >> 2)) * 4 + (nl & 3);
-            const int n = 16 * t + nl, m = 16 * tile + ml;
-            if (n < a.N && m < a.M) skinny_store(a, skinny_sum(red + off, kVals, sw), m, n);
+        if (n < a.N && m < a.M && nl < tr) {
+            const uint16_t o = skinny_value(a, skinny_sum(red + off, kVals, sw), m, n);
+            if (a.C32) a.C32[(int64_t)m * a.N + n] = bf16_to_f32(o);
+            else a.C[(int64_t)m * a.ldc + n] = o;
         }
     }
 }
 
-template <int MT, bool NORM>
-static int skinny_loop_launch(const GemmArgs& a, int sw, hipStream_t st) {
-    const int64_t ntiles = ((int64_t)a.N + 15) / 16, cus = device_cus();
-    const int64_t per = (ntiles + 2 * cus - 1) / (2 * cus);
-    hipLaunchKernelGGL((gemm_skinny_loop_kernel<MT, NORM>), dim3((unsigned)((ntiles + per - 1) / per)), dim3(64 * sw),
-                       2 * sw * MT * 256 * sizeof(float), st, a, sw, (int)ntiles);
-    return check_launch("gemm_skinny_loop");
+// The same product for a wide W (a head: 50,304 rows of 768).  A workgroup puts its X operands
+// into LDS once, normalised and in the order of the reads below (a K step of 16 rows is 1 KB, lane
+// l's 16 bytes at 16 l: no bank conflicts), and its waves then walk the 16-row tiles of W by
+// themselves, each K range of a tile in turn: no partial sums in LDS and no barrier, two batches of
+// U steps of W in flight per wave.  HBM bounds it (W is read once), and the first loads.  One
+// workgroup per pair of tiles reads X and sums its squares 1,572 times over: 768 into 50,304 40.7 us
+// for 16 rows with the norm, 106.8 for 64; here 20.3 (3.8 TB/s of W) and 35.9.
+static constexpr int skinny_walk_kb(int64_t K, int mt) { return (int)((K + 31) / 32) * mt; }   // 1 KB blocks of X
+
+template <int MT, bool NORM, int KB>
+__global__ void __launch_bounds__(512, KB <= 64 ? 4 : 2) gemm_skinny_walk_kernel(GemmArgs a, int sw, int ntiles) {
+    constexpr int U = MT == 2 && KB <= 64 ? 4 : 8, NW = 8;   // 4: within the 128 registers of 16 waves a CU
+    __shared__ __attribute__((aligned(16))) uint16_t sx[KB * 512];
+    __shared__ float srstd[kSKMaxM];
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = lane & 15, kg = lane >> 4;
+    const int ks = (a.K + 31) / 32, nb = (ks + U - 1) / U, stride = NW * gridDim.x;
+    uint4 wv[2][U];
+    auto load_w = [&](uint4 (&v)[U], int t, int b) {
+        const int n = 16 * t + r;
+        const bool ok = t < ntiles && n < a.N;
+        const uint16_t* row = a.B + (int64_t)(ok ? n : 0) * a.ldb + 8 * kg;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int k = 32 * (b * U + u);
+            v[u] = ld16_if(ok && k + 8 * kg < a.K, row + k);
+        }
+    };
+    // the batch after (t, b)
+    auto next = [&](int& t, int& b) {
+        if (++b == nb) {
+            b = 0;
+            t += stride;
+        }
+    };
+    int t = blockIdx.x + w * gridDim.x, b = 0, tl = t, bl = 0;
+    // X's blocks in batches of F a wave; the squares' rows and the first batch before W
+    constexpr int F = 4;
+    uint4 fx[F], fn[F];
+    auto fill_load = [&](int i0) {
+#pragma unroll
+        for (int f = 0; f < F; ++f) {
+            const int i = min(i0 + NW * f, ks * MT - 1), s = i / MT, m = 16 * (i - s * MT) + r;
+            const int k = min(32 * s + 8 * kg, a.K - 8);
+            fx[f] = ld16(a.A + (int64_t)min(m, a.M - 1) * a.lda + k);
+            if constexpr (NORM) fn[f] = ld16(a.nw + k);
+        }
+    };
+    auto fill_store = [&](int i0) {
+#pragma unroll
+        for (int f = 0; f < F; ++f) {
+            const int i = i0 + NW * f, s = i / MT, m = 16 * (i - s * MT) + r;
+            if (i >= ks * MT) break;
+            uint4 x = fx[f];
+            if constexpr (NORM) x = skinny_normalise(x, fn[f], srstd[min(m, a.M - 1)]);
+            if (m >= a.M || 32 * s + 8 * kg >= a.K) x = make_uint4(0u, 0u, 0u, 0u);
+            *reinterpret_cast<uint4*>(sx + i * 512 + lane * 8) = x;
+        }
+    };
+    SkinnyRstd<MT == 1 ? 2 : 4, 2> sums;
+    if constexpr (NORM) sums.load_first(a, NW, w, lane);
+    fill_load(w);
+    load_w(wv[0], tl, bl);
+    next(tl, bl);
+    if constexpr (NORM) sums.finish(a, NW, w, lane, srstd);
+    fill_store(w);
+    for (int i = w + NW * F; i < ks * MT; i += NW * F) {
+        fill_load(i);
+        fill_store(i);
+    }
+    __syncthreads();
+    f32x4 acc[MT], sum[MT];
+    // 4 outputs in one store: whole quads of rows that start 8 (bf16) or 16 bytes (fp32) aligned
+    const bool wide = a.N % 4 == 0 && (a.C32 ? ((uintptr_t)a.C32 & 15) == 0 : a.ldc % 4 == 0 && ((uintptr_t)a.C & 7) == 0);
+    int seg = 0, cut = 0;   // the K range that acc is in, its first step past the end
+    auto start = [&]() {
+        seg = 0;
+        cut = ks / sw;
+#pragma unroll
+        for (int j = 0; j < MT; ++j) acc[j] = sum[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    };
+    auto fold = [&]() {
+#pragma unroll
+        for (int j = 0; j < MT; ++j) {
+            sum[j] += acc[j];
+            acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+    };
+    auto cross = [&]() {   // into the next K range
+        fold();
+        ++seg;
+        cut = (seg + 1) * ks / sw;
+    };
+    auto batch = [&](const uint4 (&cur)[U], uint4 (&nxt)[U]) {
+        load_w(nxt, tl, bl);
+        next(tl, bl);
+        const int s0 = b * U;
+        auto step = [&](int u) {
+#pragma unroll
+            for (int j = 0; j < MT; ++j)
+                acc[j] = mfma16(cur[u], *reinterpret_cast<const uint4*>(sx + ((s0 + u) * MT + j) * 512 + lane * 8), acc[j]);
+        };
+        if (s0 == cut) cross();
+        if (s0 + U <= ks && s0 + U <= cut) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) step(u);
+        } else {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                if (s0 + u >= ks) break;
+                if (u > 0 && s0 + u == cut) cross();
+                step(u);
+            }
+        }
+        if (b + 1 == nb) {
+            fold();
+            // lane: row r of X, 4 consecutive rows n of W
+            const int n = 16 * t + 4 * kg;
+#pragma unroll
+            for (int j = 0; j < MT; ++j) {
+                const int m = 16 * j + r;
+                if (m >= a.M) continue;
+                uint16_t o[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o[e] = n + e < a.N ? skinny_value(a, sum[j][e], m, n + e) : (uint16_t)0;
+                if (wide) {
+                    if (n >= a.N) continue;
+                    if (a.C32)
+                        *reinterpret_cast<float4*>(a.C32 + (int64_t)m * a.N + n) =
+                            make_float4(bf16_to_f32(o[0]), bf16_to_f32(o[1]), bf16_to_f32(o[2]), bf16_to_f32(o[3]));
+                    else
+                        *reinterpret_cast<uint2*>(a.C + (int64_t)m * a.ldc + n) =
+                            make_uint2(o[0] | (uint32_t)o[1] << 16, o[2] | (uint32_t)o[3] << 16);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        if (n + e >= a.N) continue;
+                        if (a.C32) a.C32[(int64_t)m * a.N + n + e] = bf16_to_f32(o[e]);
+                        else a.C[(int64_t)m * a.ldc + n + e] = o[e];
+                    }
+                }
+            }
+            start();
+        }
+        next(t, b);
+    };
+    start();
+    while (t < ntiles) {
+        batch(wv[0], wv[1]);
+        if (t >= ntiles) break;
+        batch(wv[1], wv[0]);
+    }
+}
+
+// K ranges of a product: as many as, at 16 nt rows of W and one wave a range, make 4 waves per CU, of a
+// K step or more each, their partials within LDS
+static int skinny_waves(const GemmArgs& a, int nt) {
+    const int mt = (a.M + 15) / 16;
+    const int64_t nblk = ((int64_t)a.N + 16 * nt - 1) / (16 * nt), ks = (a.K + 31) / 32, target = 4LL * device_cus();
+    int sw = 1;
+    while (sw < 16 && nblk * sw < target && 2 * sw <= ks && 2 * sw * nt * mt <= kSKMaxTiles) sw *= 2;
+    return sw;
 }
 
 template <int NT, bool NORM>
 static int skinny_launch(const GemmArgs& a, hipStream_t st) {
-    const int mt = (a.M + 15) / 16;
-    const int64_t cus = device_cus(), ks = (a.K + 31) / 32;
-    // A narrow layer's tiles take 8 or 4 rows of W (the MFMA's other rows are zeros) until half
-    // the CUs have one: a workgroup's bytes, not the MFMAs, set its time (768 x 3072 of 16 rows,
-    // 98 KB of W and 98 KB of X in each of 48 workgroups: 9.0 -> 7.5 us; 768 x 768 4.1 -> 3.8).
-    // 144 tiles of 2304 x 768 stay whole (5.5 us, 6.5 in 288 halves).
+    // A narrow layer's tiles take 8 or 4 rows of W until half the CUs have one: a workgroup's bytes, not
+    // the MFMAs, set its time, from a K on where they outweigh the launch of more workgroups (16 rows,
+    // in tiles of 16, 8 and 4, us: 3072 into 768 8.0, 7.2, 6.9; 2048 into 512 6.3, 5.7, 5.6; 1024 into 256
+    // 4.2, 3.9, 4.0; 768 into 768 4.10, 3.95, 3.97; 512 into 512 3.4, 3.4, 3.5; 768 into 2304 5.5, 7.0, 10.0)
     int tr = 16;
-    while (NT == 1 && tr > 4 && ((int64_t)a.N + tr - 1) / tr * 2 < cus) tr /= 2;
+    const int least = a.K >= 1536 ? 4 : a.K >= 768 ? 8 : 16;
+    while (NT == 1 && tr > least && ((int64_t)a.N + tr - 1) / tr * 2 < device_cus()) tr /= 2;
     const int64_t nblk = ((int64_t)a.N + tr * NT - 1) / (tr * NT);
-    const int64_t target = 4 * cus;  // waves
-    // with the norm, as many waves as make a wave's K range one batch, where LDS allows
-    const int64_t want = NORM ? (ks + skinny_batch(NT, mt, true) - 1) / skinny_batch(NT, mt, true) : 1;
-    int sw = 1;
-    while (sw < 16 && (nblk * sw < target || sw < want) && 2 * sw <= ks && 2 * sw * NT * mt <= kSKMaxTiles) sw *= 2;
-    const dim3 grid((unsigned)nblk), block(64 * sw);
-    switch (mt) {
-        case 1: hipLaunchKernelGGL((gemm_skinny_kernel<NT, 1, NORM>), grid, block, 0, st, a, sw, tr); break;
-        case 2: hipLaunchKernelGGL((gemm_skinny_kernel<NT, 2, NORM>), grid, block, 0, st, a, sw, tr); break;
-        case 3: hipLaunchKernelGGL((gemm_skinny_kernel<NT, 3, NORM>), grid, block, 0, st, a, sw, tr); break;
-        default: hipLaunchKernelGGL((gemm_skinny_kernel<NT, 4, NORM>), grid, block, 0, st, a, sw, tr); break;
+    const int sw = skinny_waves(a, NT);
+    // with the norm as many waves as hold X's rows in one load
+    int nw = sw;
+    while (NORM && nw < 16 && nw * skinny_rows((a.M + 15) / 16) < a.M) nw *= 2;
+    const dim3 grid((unsigned)nblk), block(64 * nw);
+    // ranges of one or two steps: the longer batch's empty slots cost 512 into 512 0.6 us of 3.9
+    const bool few = ((a.K + 31) / 32 + sw - 1) / sw <= 2;
+#define FX_SKINNY(MT)                                                                                                        \
+    {                                                                                                                        \
+        constexpr int u = skinny_batch(NT, MT, NORM);                                                                        \
+        if (few) hipLaunchKernelGGL((gemm_skinny_kernel<NT, MT, NORM, u < 2 ? u : 2>), grid, block, 0, st, a, sw, tr);        \
+        else hipLaunchKernelGGL((gemm_skinny_kernel<NT, MT, NORM, u>), grid, block, 0, st, a, sw, tr);                        \
+        break;                                                                                                               \
     }
+    switch ((a.M + 15) / 16) {
+        case 1: FX_SKINNY(1)
+        case 2: FX_SKINNY(2)
+        case 3: FX_SKINNY(3)
+        default: FX_SKINNY(4)
+    }
+#undef FX_SKINNY
     return check_launch("gemm_skinny");
 }
 
-template <bool NORM>
-static int skinny_loop(const GemmArgs& a, int sw, hipStream_t st) {
-    const int mt = (a.M + 15) / 16;
-    if (mt == 1) return skinny_loop_launch<1, NORM>(a, sw, st);
-    if (NORM || mt == 2) return skinny_loop_launch<2, NORM>(a, sw, st);
-    return mt == 3 ? skinny_loop_launch<3, false>(a, sw, st) : skinny_loop_launch<4, false>(a, sw, st);
+template <int MT, bool NORM>
+static int skinny_walk(const GemmArgs& a, int sw, hipStream_t st) {
+    const int64_t ntiles = ((int64_t)a.N + 15) / 16, cus = device_cus();
+    // two workgroups a CU where X takes at most 64 KB (and the accumulators leave registers for 16 waves)
+    constexpr int kb = MT <= 2 ? 64 : 128;
+    const bool two = skinny_walk_kb(a.K, MT) <= 64 && kb == 64;
+    const dim3 grid((unsigned)((two ? 2 : 1) * cus < ntiles ? (two ? 2 : 1) * cus : ntiles));
+    if (two) hipLaunchKernelGGL((gemm_skinny_walk_kernel<MT, NORM, kb>), grid, dim3(512), 0, st, a, sw, (int)ntiles);
+    else hipLaunchKernelGGL((gemm_skinny_walk_kernel<MT, NORM, 128>), grid, dim3(512), 0, st, a, sw, (int)ntiles);
+    return check_launch("gemm_skinny_walk");
 }
 
-// the walking kernel from four 16-row tiles of W per CU on, where 16 waves hold K in one batch
-// each (and with the norm X fits the registers beside it); else two W row tiles per workgroup once there are enough workgroups (fewer re-reads
-// of X)
+// Two W row tiles per workgroup once there are enough workgroups (fewer re-reads of X).  The walking
+// kernel where X fits LDS (128 KB) and there are four 16-row tiles of W per CU, or two with more rows
+// of X (768 into 8192 with the norm, tiles / walking, us: 16 rows 8.7 / 9.5, 32 17.6 / 14.6, 64 28.7 / 17.8).
 static int linear_skinny(const GemmArgs& a, hipStream_t st) {
-    const int64_t ks = (a.K + 31) / 32;
-    if (((int64_t)a.N + 15) / 16 >= 4LL * device_cus() && ks <= 16 * kSKLoopU && !a.idx && !a.Xg &&
-        !(a.nw && a.M > 32)) {
-        int sw = 4;
-        while (sw < 16 && sw * kSKLoopU < ks) sw *= 2;
-        return a.nw ? skinny_loop<true>(a, sw, st) : skinny_loop<false>(a, sw, st);
+    const int mt = (a.M + 15) / 16;
+    const int64_t cus = device_cus();
+    const bool two = (a.N + 31) / 32 >= 2 * cus;
+    if (((int64_t)a.N + 15) / 16 >= (mt == 1 ? 4 : 2) * cus && skinny_walk_kb(a.K, mt) <= 128 && !a.idx && !a.Xg) {
+        const int sw = skinny_waves(a, two ? 2 : 1);
+        switch (mt) {
+            case 1: return a.nw ? skinny_walk<1, true>(a, sw, st) : skinny_walk<1, false>(a, sw, st);
+            case 2: return a.nw ? skinny_walk<2, true>(a, sw, st) : skinny_walk<2, false>(a, sw, st);
+            case 3: return a.nw ? skinny_walk<3, true>(a, sw, st) : skinny_walk<3, false>(a, sw, st);
+            default: return a.nw ? skinny_walk<4, true>(a, sw, st) : skinny_walk<4, false>(a, sw, st);
+        }
     }
-    const bool two = (a.N + 31) / 32 >= 2LL * device_cus();
     if (a.nw) return two ? skinny_launch<2, true>(a, st) : skinny_launch<1, true>(a, st);
     return two ? skinny_launch<2, false>(a, st) : skinny_launch<1, false>(a, st);
 }

@@ -675,11 +675,13 @@ def test_small_tile_dgrad_matches_whole_tiles(dev, monkeypatch, M, N, K, pad):
 @pytest.mark.parametrize("M,K,N,norm,res,act", [
     (1, 8, 16400, True, False, None),             # the walking kernel: one K chunk, most waves without work
     (17, 768, 16391, True, True, "gelu_tanh"),    # a last tile of 7 rows, two row tiles of X
-    (32, 2048, 16384, True, False, None),         # the deepest K: four steps in each of 16 waves
-    (33, 768, 16400, True, False, None),          # past its rows with the norm
+    (32, 2048, 16384, True, False, None),         # X in 128 KB of LDS, the most it takes
+    (33, 768, 16400, True, False, None),          # three row tiles of X
     (64, 520, 16400, False, True, None),          # four row tiles of X, a K tail of 8
-    (16, 2056, 16400, False, False, None),        # K past its registers
-    (16, 3072, 768, True, False, None),           # tiles of 4 rows; the norm in a second read of x
+    (48, 1536, 16400, False, False, None),        # X past LDS: the tiles
+    (64, 1024, 8200, True, False, None),          # two tiles of W a CU, X in 128 KB
+    (16, 2056, 16400, False, False, None),        # K past 64 KB of LDS: one workgroup a CU
+    (16, 3072, 768, True, False, None),           # tiles of 4 rows; the norm's sums row by row
     (5, 72, 3, False, True, "gelu_tanh"),         # less than one tile of 4 rows
 ])
 def test_few_rows_tile_choices(dev, M, K, N, norm, res, act):
@@ -702,6 +704,91 @@ def test_few_rows_tile_choices(dev, M, K, N, norm, res, act):
     if res:
         z = z + r.double()
     assert oracle_close(y, z.cpu(), FRAC_OUT)
+
+
+def _few_row_ranges(M, N, K):
+    """K ranges that a few-row product sums in order."""
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    nt = 2 if -(-N // 32) >= 2 * cus else 1
+    sw = 1
+    while sw < 16 and -(-N // (16 * nt)) * sw < 4 * cus and 2 * sw <= -(-K // 32) and 2 * sw * nt * -(-M // 16) <= 16:
+        sw *= 2
+    return sw
+
+
+@pytest.mark.parametrize("M,K,N", [
+    (64, 768, 16400), (64, 264, 8200),                        # the walking kernel
+    (16, 768, 2304), (16, 768, 768), (16, 3072, 768), (64, 3080, 768), (3, 512, 512), (33, 264, 40), (16, 2048, 512),
+])
+def test_few_rows_ranges(dev, M, K, N):
+    # sums that are exact inside a K range (8-bit integers of one exponent) and round between ranges of
+    # different exponents, most of which cancels: the result shows the ranges and their order, which
+    # no choice of tiles, waves or kernel may change
+    from fxgpu.fused_linear import linear_ex
+    g = torch.Generator(device=dev).manual_seed(M + K + N)
+    ks, sw = -(-K // 32), _few_row_ranges(M, N, K)
+    assert sw > 1
+    at = torch.tensor([min(32 * s + s * 7 % 32, K - 1) for s in range(ks)], device=dev)
+    of = torch.zeros(ks, dtype=torch.int64, device=dev)
+    for w in range(sw):
+        of[w * ks // sw:(w + 1) * ks // sw] = w
+    e = torch.randint(-12, 12, (N, sw), device=dev, generator=g)
+    c = torch.randint(-255, 256, (N, ks), device=dev, generator=g) * 2.0 ** e[:, of]
+    c[:, of == sw - 1] = 0.0
+    c[:, -1] = -c.double().sum(1).bfloat16().float()
+    part = torch.zeros(N, sw, device=dev, dtype=torch.float64).index_add_(1, of, c.double()).float()
+    want = torch.zeros(N, device=dev)
+    for w in range(sw):
+        want = want + part[:, w]
+    W, x = torch.zeros(N, K, device=dev).bfloat16(), torch.zeros(M, K, device=dev).bfloat16()
+    W[:, at], x[:, at] = c.bfloat16(), 1.0
+    assert torch.equal(W[:, at].float(), c)
+    print(f"few rows ranges M={M} K={K} N={N}: {sw}", flush=True)
+    assert torch.equal(linear_ex(x, W), want.bfloat16().expand(M, N))
+
+
+@pytest.mark.parametrize("M,K,N", [(1, 768, 16400), (16, 768, 50304), (17, 1000, 16400), (32, 768, 8200), (64, 2048, 8208), (48, 1024, 32000)])
+def test_few_rows_walking_matches_tiles(dev, M, K, N):
+    # gathered rows stay on the tiles: the same rows as one window each give the same bits
+    from fxgpu.abi import call, ptr, stream_of
+    g = torch.Generator(device=dev).manual_seed(M + K + N)
+    x = torch.randn(M, K, device=dev, generator=g).bfloat16()
+    W = (torch.randn(N, K, device=dev, generator=g) * K ** -0.5).bfloat16()
+    b = torch.randn(N, device=dev, generator=g).bfloat16()
+    idx = torch.arange(M, device=dev, dtype=torch.int32)
+    y = torch.empty(M, N, device=dev, dtype=torch.bfloat16)
+    print(f"walking M={M} K={K} N={N}", flush=True)
+    call("fx_linear_fwd", ptr(x), K, ptr(idx), K, M, ptr(W), ptr(b), ptr(y), None, None, M, N, K, 1, stream_of(x))
+    assert torch.equal(y, _linear_fwd(x, W, b, 1, False)[0])
+
+
+@pytest.mark.parametrize("M,K,N", [(16, 768, 2304), (16, 768, 50304), (32, 512, 8200), (64, 1032, 48), (5, 72, 3), (33, 3072, 96)])
+def test_few_rows_norm_order(dev, M, K, N):
+    # W of unit rows: the outputs are the normalised x, whose sum of squares is a lane's chunks of 8
+    # in order, then a butterfly over 64 lanes, in fp32, for every kernel and number of waves
+    import numpy as np
+    from fxgpu.fused_linear import linear_ex
+    g = torch.Generator().manual_seed(M + K + N)
+    n = torch.arange(N)
+    W = torch.zeros(N, K).bfloat16()
+    W[n, n % K] = 1.0
+    W = W.to(dev)
+    for _ in range(16):
+        x = torch.randn(M, K, generator=g).bfloat16()
+        nw = (torch.randn(K, generator=g) * 0.1 + 1).bfloat16()
+        sq = np.zeros((M, -(-K // 512) * 512))
+        sq[:, :K] = x.double().square().numpy()
+        sq = sq.reshape(M, -1, 64, 8).transpose(1, 3, 0, 2).reshape(-1, M, 64)   # a lane's values in order
+        q = np.zeros((M, 64), np.float32)
+        for v in sq:
+            q = (q.astype(np.float64) + v).astype(np.float32)                    # an fp32 fma: the square is exact
+        lane = np.arange(64)
+        for off in (32, 16, 8, 4, 2, 1):
+            q = q + q[:, lane ^ off]
+        rstd = np.float32(1) / np.sqrt(q[:, :1] / np.float32(K) + np.float32(1e-6))
+        want = torch.from_numpy(x.float().numpy() * rstd * nw.float().numpy()).bfloat16()[:, n % K]
+        got = linear_ex(x.to(dev), W, norm_weight=nw.to(dev), eps=1e-6).cpu()
+        assert torch.equal(got, want), int((got != want).sum())
 
 
 @pytest.mark.parametrize("M,N,K", [
