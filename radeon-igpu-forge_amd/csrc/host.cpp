@@ -12,6 +12,7 @@
 #include <torch/csrc/utils/pybind.h>
 #include <c10/hip/HIPStream.h>
 
+#include <initializer_list>
 #include <tuple>
 #include <vector>
 
@@ -44,6 +45,20 @@ void check(int rc, const char* name) {
     raise(PyExc_RuntimeError, std::string(name) + " failed: hipError=" + std::to_string(rc) + " (" + msg + ")");
 }
 
+const Tensor* given(const Tensor& t) { return &t; }
+const Tensor* given(const OptT& t) { return t.has_value() ? &*t : nullptr; }
+
+// Every tensor whose pointer a kernel gets lies on the GPU of the first: a host pointer, or another
+// GPU's, is refused here and never launched with
+template <class... Rest>
+void same_gpu(const Tensor& a, const Rest&... rest) {
+    if (!a.is_cuda()) raise(PyExc_RuntimeError, "expected all tensors to be on one GPU, got " + a.device().str());
+    for (const Tensor* t : std::initializer_list<const Tensor*>{given(rest)...})
+        if (t && t->device() != a.device())
+            raise(PyExc_RuntimeError,
+                  "expected all tensors to be on one GPU, got " + a.device().str() + " and " + t->device().str());
+}
+
 // ---- RMSNorm ---------------------------------------------------------------------------
 
 bool norm_ok(const Tensor& x, const Tensor& w) {
@@ -56,6 +71,7 @@ bool norm_ok(const Tensor& x, const Tensor& w) {
 // (y, rstd), or None when x or w need a check or a copy
 std::optional<std::tuple<Tensor, Tensor>> norm_fwd(const Tensor& x, const Tensor& w, double eps) {
     if (!norm_ok(x, w)) return std::nullopt;
+    same_gpu(x, w);
     const int64_t D = x.size(-1), N = x.numel() / D;
     Tensor y = at::empty(x.sizes(), x.options());
     Tensor rstd = at::empty({N}, as_f32(x));
@@ -68,6 +84,7 @@ std::optional<std::tuple<Tensor, Tensor, Tensor>> norm_add_fwd(const Tensor& x, 
                                                                double eps) {
     if (!norm_ok(x, w) || r.sizes() != x.sizes() || !is_bf(r) || !r.is_cuda() || !r.is_contiguous() || !aligned(r))
         return std::nullopt;
+    same_gpu(x, r, w);
     const int64_t D = x.size(-1), N = x.numel() / D;
     Tensor s = at::empty(x.sizes(), x.options());
     Tensor y = at::empty(x.sizes(), x.options());
@@ -88,6 +105,7 @@ Tensor grad_rows(const Tensor& g) {
 // (dx shaped like x, dw); dx += dres in the same pass when given
 std::tuple<Tensor, Tensor> norm_bwd(const Tensor& x, const Tensor& dy, const Tensor& w, const Tensor& rstd,
                                     const OptT& dres) {
+    same_gpu(x, dy, w, rstd, dres);
     const int64_t D = x.size(-1), N = x.numel() / D;
     const Tensor g = grad_rows(dy);
     Tensor dx = at::empty(x.sizes(), x.options());
@@ -168,6 +186,7 @@ std::optional<std::tuple<Tensor, Tensor>> attn_fwd(const Tensor& q, const Tensor
     if ((Dh != 64 && Dh != 128) || q.numel() < 1 || q.numel() >= (int64_t)1 << 31 || !attn_ok(q) || !attn_ok(k) ||
         !attn_ok(v))
         return std::nullopt;
+    same_gpu(q, k, v);
     fxAttnArgs a = split_args(q, k, v, causal, scale);
     return attn_run_fwd(a, q);
 }
@@ -194,6 +213,7 @@ void attn_run_bwd(fxAttnArgs& a, const Tensor& o, const Tensor& lse, const Tenso
 
 std::tuple<Tensor, Tensor, Tensor> attn_bwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o,
                                             const Tensor& lse, const Tensor& dout, bool causal, double scale) {
+    same_gpu(q, k, v, o, lse, dout);
     fxAttnArgs a = split_args(q, k, v, causal, scale);
     Tensor dq = at::empty(q.sizes(), q.options()), dk = at::empty(q.sizes(), q.options()),
            dv = at::empty(q.sizes(), q.options());
@@ -210,6 +230,7 @@ std::tuple<Tensor, Tensor, Tensor> attn_bwd(const Tensor& q, const Tensor& k, co
 
 Tensor attn_bwd_qkv(const Tensor& qkv, const Tensor& o, const Tensor& lse, const Tensor& dout, bool causal,
                     double scale) {
+    same_gpu(qkv, o, lse, dout);
     fxAttnArgs a = packed_args(qkv, causal, scale);
     Tensor dqkv = at::empty(qkv.sizes(), qkv.options());
     a.dq = bf(dqkv);
@@ -233,6 +254,7 @@ Tensor rows(const Tensor& t) {
 
 // y = act(x2 w^T + bias), and h (the pre-activation, act 2: the GELU derivative) when wanted
 std::tuple<Tensor, OptT> linear_fwd(const Tensor& x2, const Tensor& w, const OptT& bias, int64_t act, bool want_h) {
+    same_gpu(x2, w, bias);
     const int64_t M = x2.size(0), K = x2.size(1), N = w.size(0);
     Tensor y = at::empty({M, N}, x2.options());
     OptT h;
@@ -252,6 +274,7 @@ std::optional<std::tuple<Tensor, OptT>> gather_fwd(const Tensor& X, const Tensor
         !X.is_cuda() || !idx.is_cuda() || !w.is_cuda() || !b.is_cuda() || !X.is_contiguous() || !idx.is_contiguous() ||
         !w.is_contiguous() || !b.is_contiguous())
         return std::nullopt;
+    same_gpu(X, idx, w, b);
     Tensor out = at::empty({B, N}, X.options());
     OptT xg;
     if (want_xg) xg = at::empty({B, K}, X.options());
@@ -265,6 +288,7 @@ std::optional<std::tuple<Tensor, OptT>> gather_fwd(const Tensor& X, const Tensor
 Tensor wgrad(const Tensor& dy, const Tensor& x) {
     if (!is_bf(dy) || !is_bf(x)) raise(PyExc_TypeError, "dy and x must be bfloat16");
     if (!dy.is_cuda() || !x.is_cuda()) raise(PyExc_TypeError, "dy and x must be cuda tensors");
+    same_gpu(dy, x);
     const Tensor dy2 = rows(dy), x2 = rows(x);
     if (dy2.size(0) != x2.size(0))
         raise(PyExc_ValueError, "dy has " + std::to_string(dy2.size(0)) + " rows, x has " + std::to_string(x2.size(0)));
@@ -282,7 +306,9 @@ Tensor wgrad(const Tensor& dy, const Tensor& x) {
 
 // dx = dy2 w (times g), or None when a layout check fails.  whole: a shape of fx_linear_dgrad
 OptT dgrad(const Tensor& dy2, const Tensor& w, const OptT& g, bool whole) {
-    if (!dy2.is_cuda() || !w.is_contiguous() || !aligned(w) || dy2.stride(1) != 1 || dy2.stride(0) % 8 || !aligned(dy2) ||
+    if (!dy2.is_cuda()) return std::nullopt;
+    same_gpu(dy2, w, g);
+    if (!w.is_contiguous() || !aligned(w) || dy2.stride(1) != 1 || dy2.stride(0) % 8 || !aligned(dy2) ||
         !is_bf(dy2) || !is_bf(w) || (g.has_value() && (!g->is_contiguous() || !aligned(*g) || !is_bf(*g))))
         return std::nullopt;
     const int64_t M = dy2.size(0), K = dy2.size(1), N = w.size(1);
@@ -320,6 +346,7 @@ Tensor column_sums(const Tensor& g) {
 
 // device scalars (1 / n_valid, that times the gradient scale)
 std::tuple<Tensor, Tensor> ce_inv_nvalid(const Tensor& target, int64_t ignore, const OptT& gs, double gs_value) {
+    same_gpu(target);
     const auto o = target.options().dtype(at::kFloat);
     Tensor inv_n = at::empty({}, o), mul = at::empty({}, o), g;
     if (gs.has_value()) g = gs->detach().to(target.device(), at::kFloat).reshape({});
@@ -331,6 +358,7 @@ std::tuple<Tensor, Tensor> ce_inv_nvalid(const Tensor& target, int64_t ignore, c
 
 void ce_rows(const Tensor& logits, const Tensor& target, const OptT& grad, const Tensor& row_loss, const Tensor& mul,
              int64_t ignore) {
+    same_gpu(logits, target, grad, row_loss, mul);
     fxCEArgs a{};
     a.logits = bf(logits);
     a.target = static_cast<int64_t*>(target.data_ptr());
@@ -346,6 +374,7 @@ void ce_rows(const Tensor& logits, const Tensor& target, const OptT& grad, const
 }
 
 Tensor ce_finalize(const Tensor& row_loss, const Tensor& inv_n) {
+    same_gpu(row_loss, inv_n);
     Tensor loss = at::empty({}, row_loss.options());
     check(fx_ce_loss_finalize(f32(row_loss), row_loss.numel(), f32(inv_n), f32(loss), stream_of(row_loss)),
           "fx_ce_loss_finalize");
@@ -366,11 +395,13 @@ std::optional<std::tuple<Tensor, OptT>> ce_fwd(const Tensor& logits, const Tenso
 }
 
 void ce_scale_grad(const Tensor& grad, const Tensor& g32, const Tensor& applied, int64_t src) {
+    same_gpu(grad, g32, applied);
     check(fx_ce_scale_grad(bf(grad), grad.numel(), f32(g32), f32(applied), (int32_t)src, stream_of(grad)),
           "fx_ce_scale_grad");
 }
 
 void ce_lin_scale_inplace(const Tensor& dW, const Tensor& dx, const Tensor& g32, const OptT& gs, double inv) {
+    same_gpu(dW, dx, g32, gs);
     check(fx_ce_lin_grad_scale_inplace(bf(dW), dW.numel(), bf(dx), dx.numel(), f32(g32), gs.has_value() ? f32(*gs) : nullptr,
                                        (float)inv, stream_of(dx)),
           "fx_ce_lin_grad_scale_inplace");
@@ -383,6 +414,7 @@ bool decode_inputs(const Tensor& tok, int64_t pos, const Tensor& tok_out, const 
     if (tok.scalar_type() != at::kLong || !tok.is_contiguous() || tok.device() != tok_out.device() ||
         tok.sizes() != tok_out.sizes())
         return false;
+    same_gpu(tok_out, pos_out, lens);
     check(fx::decode_inputs(static_cast<int64_t*>(tok.data_ptr()), tok.numel(), pos, static_cast<int64_t*>(tok_out.data_ptr()),
                             static_cast<int64_t*>(pos_out.data_ptr()), static_cast<int32_t*>(lens.data_ptr()),
                             stream_of(tok)),
@@ -397,6 +429,7 @@ OptT decode_embed(const Tensor& tok, const Tensor& pos, const Tensor& E, const T
         !P.is_cuda() || E.dim() != 2 || P.dim() != 2 || E.size(1) != P.size(1) || E.size(1) % 8 || E.size(1) < 8 ||
         !E.is_contiguous() || !P.is_contiguous() || !aligned(E) || !aligned(P))
         return std::nullopt;
+    same_gpu(tok, pos, E, P);
     const int64_t B = tok.numel(), D = E.size(1);
     Tensor x = at::empty({B, 1, D}, E.options());
     check(fx::decode_embed(static_cast<int64_t*>(tok.data_ptr()), static_cast<int64_t*>(pos.data_ptr()), bf(E), E.size(0), bf(P),
@@ -412,6 +445,7 @@ OptT few_rows_logits(const Tensor& x, const Tensor& w, const Tensor& norm_w, dou
         norm_w.size(0) != x.size(1) || x.size(1) % 8 || x.stride(1) != 1 || x.stride(0) % 8 || !w.is_contiguous() ||
         !norm_w.is_contiguous() || !aligned(x) || !aligned(w) || !aligned(norm_w))
         return std::nullopt;
+    same_gpu(x, w, norm_w);
     Tensor out = at::empty({x.size(0), w.size(0)}, as_f32(x));
     check(fx::few_rows_logits(bf(x), x.stride(0), bf(w), bf(norm_w), (float)eps, f32(out), x.size(0), w.size(0), x.size(1),
                               stream_of(x)),
@@ -439,6 +473,7 @@ std::tuple<Tensor, int64_t> adamw_step(FlatLayout& f, const std::vector<Tensor>&
     for (size_t i = 0; i < params.size(); ++i) {
         Tensor g = params[i].grad();
         if (!g.defined()) continue;
+        same_gpu(t[0], g);
         if (!is_bf(g)) return std::make_tuple(work, (int64_t)i);
         if (!g.is_contiguous()) {
             g = g.contiguous();
@@ -456,6 +491,7 @@ std::tuple<Tensor, int64_t> adamw_step(FlatLayout& f, const std::vector<Tensor>&
         l.wd[l.count] = f.wd[i];
         ++l.count;
     }
+    for (const Tensor& s : t) same_gpu(t[0], s);
     fxTensorList none{};
     const fxTensorList* lists = f.lists.empty() ? &none : f.lists.data();
     const int32_t nl = (int32_t)f.lists.size();

@@ -55,6 +55,22 @@ def test_misaligned_and_refused_inputs(dev):
         flash_attention(q, q, q, scale=-1.0)
 
 
+@pytest.mark.parametrize("M", [16, 256, 300])     # few rows, whole tiles, small tiles
+def test_a_weight_on_the_host_is_refused(dev, M):
+    # as torch.mm refuses it, and before any launch
+    from fxgpu.abi import host
+    from fxgpu.fused_linear import fused_linear, input_grad, linear, linear_wgrad
+    x, w = torch.randn(M, 512, device=dev).bfloat16(), torch.randn(512, 512).bfloat16()
+    b = torch.zeros(512).bfloat16()
+    for call in (lambda: linear(x, w), lambda: fused_linear(x, w.to(dev), b, None), lambda: input_grad(x, w),
+                 lambda: input_grad(x, w.to(dev), x.cpu()), lambda: host.linear_fwd(x, w, None, 0, False),
+                 lambda: host.norm_bwd(x, x.cpu(), w[0].to(dev), x[:, 0].float(), None)):
+        with pytest.raises(RuntimeError, match="expected all tensors to be on"):
+            call()
+    with pytest.raises(TypeError, match="cuda tensors"):
+        linear_wgrad(x, x.cpu())
+
+
 def test_optimizer_deepcopy_takes_the_same_step(dev):
     from fxlm.optim import FlatAdamW
     model = torch.nn.Linear(64, 40).to(dev)
