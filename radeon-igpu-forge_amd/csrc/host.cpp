@@ -245,10 +245,19 @@ Tensor attn_bwd_qkv(const Tensor& qkv, const Tensor& o, const Tensor& lse, const
 
 // ---- linear layers ---------------------------------------------------------------------
 
-// t as a (rows, cols) view whose rows are 16-byte aligned and unit-stride
+// rows as the GEMM kernels read them: unit stride, 16-byte aligned starts, none overlapping another
+// (an expanded row, sliding windows)
+bool rows_ok(const Tensor& r) {
+    return r.stride(1) == 1 && r.stride(0) % 8 == 0 && (r.size(0) <= 1 || r.stride(0) >= r.size(1)) && aligned(r);
+}
+
+// t as a (rows, cols) view with such rows, or a copy of it
 Tensor rows(const Tensor& t) {
     Tensor r = t.dim() == 2 ? t : t.reshape({-1, t.size(-1)});
-    if (r.stride(1) != 1 || r.stride(0) % 8 || !aligned(r)) r = r.contiguous();
+    if (!rows_ok(r)) r = r.contiguous();
+    if (!aligned(r)) r = r.clone();   // contiguous, but not where it starts
+    // one row, whose stride may be anything
+    if (r.size(0) == 1 && r.stride(0) != r.size(1)) r = r.reshape({r.size(1)}).unsqueeze(0);
     return r;
 }
 
@@ -308,7 +317,7 @@ Tensor wgrad(const Tensor& dy, const Tensor& x) {
 OptT dgrad(const Tensor& dy2, const Tensor& w, const OptT& g, bool whole) {
     if (!dy2.is_cuda()) return std::nullopt;
     same_gpu(dy2, w, g);
-    if (!w.is_contiguous() || !aligned(w) || dy2.stride(1) != 1 || dy2.stride(0) % 8 || !aligned(dy2) ||
+    if (!w.is_contiguous() || !aligned(w) || !rows_ok(dy2) || dy2.stride(0) < dy2.size(1) ||
         !is_bf(dy2) || !is_bf(w) || (g.has_value() && (!g->is_contiguous() || !aligned(*g) || !is_bf(*g))))
         return std::nullopt;
     const int64_t M = dy2.size(0), K = dy2.size(1), N = w.size(1);

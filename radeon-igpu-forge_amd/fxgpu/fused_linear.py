@@ -34,7 +34,7 @@ _ACTS = {None: 0, "none": 0, "identity": 0, "gelu_tanh": 1}
 
 
 def _rows(t):
-    """t as a (rows, cols) view whose rows are 16-byte aligned and unit-stride."""
+    """t as a (rows, cols) view whose rows are 16-byte aligned, unit-stride and apart, or such a copy."""
     return host.rows(t)
 
 

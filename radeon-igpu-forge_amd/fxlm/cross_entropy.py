@@ -22,7 +22,7 @@ behaviour, ml/fxlm/cross_entropy.py:41-44 and ml/fxlm/kernels/ce.hip:43).
 import torch
 
 from fxgpu.abi import call, host, lib, ptr, stream_of
-from fxgpu.fused_linear import _native_fwd, input_grad, linear_wgrad, native_fwd
+from fxgpu.fused_linear import _native_fwd, _rows, input_grad, linear_wgrad, native_fwd
 
 # rows per linear-CE chunk: bound the chunk's bf16 logits to this many bytes
 _CHUNK_BYTES = 2 << 30
@@ -166,7 +166,7 @@ def _logits(x, weight):
     V = weight.shape[0]
     if (M * V * K <= 8 << 30 and K % 8 == 0 and M > 0 and native_fwd(M, V, K)
             and (x.data_ptr() | weight.data_ptr()) % 16 == 0):
-        return _native_fwd(x, weight)
+        return _native_fwd(_rows(x), weight)
     return torch.mm(x, weight.t())
 
 

@@ -55,6 +55,42 @@ def test_misaligned_and_refused_inputs(dev):
         flash_attention(q, q, q, scale=-1.0)
 
 
+@pytest.mark.parametrize("M", [1, 65, 256, 300])
+@pytest.mark.parametrize("layout", ["offset", "expanded", "windows", "wide", "columns"])
+def test_linear_of_any_layout(dev, M, layout):
+    # what torch.mm takes: contiguous but not 16-byte aligned, one row repeated, overlapping windows, rows of
+    # a wider tensor at an odd stride, a transpose; and gradients that arrive as an expanded row
+    from fxgpu.fused_linear import linear
+    K, N = 64, 192
+    g = torch.Generator(device=dev).manual_seed(M)
+    flat = torch.randn(3 + M * (K + 3) + 8 * M + K, device=dev, generator=g).bfloat16()
+    x = {"offset": flat[3:3 + M * K].view(M, K), "expanded": flat[:K].expand(M, K), "windows": flat[:8 * (M - 1) + K].unfold(0, K, 8),
+         "wide": flat[:M * (K + 3)].view(M, K + 3)[:, :K], "columns": flat[:M * K].view(K, M).t()}[layout]
+    w = (torch.randn(N, K, device=dev, generator=g) * K ** -0.5).bfloat16()
+    ref = x.float() @ w.float().t()
+    # one bf16 rounding of the product, at a result's own size and at the largest's for fp32 sums
+    bound = 2.0 ** -8 * ref.abs() + 1e-5 * ref.abs().max()
+    assert bool(((linear(x, w).float() - ref).abs() <= bound).all())
+    xs, ws = x.detach().requires_grad_(), w.clone().requires_grad_()
+    for frozen in (True, False):     # dy of a column sum: one row expanded
+        y = linear(xs, w if frozen else ws)
+        got = torch.autograd.grad(y.sum(0), [xs] if frozen else [xs, ws], torch.ones(N, device=dev).bfloat16())
+        want = [w.float().sum(0).expand(M, K), x.float().sum(0).expand(N, K)]
+        for a, b in zip(got, want):
+            assert a.shape == b.shape
+            assert bool(((a.float() - b).abs() <= 2.0 ** -8 * b.abs() + 1e-4 * b.abs().max()).all())
+
+
+def test_input_grad_of_rows_that_overlap(dev):
+    from fxgpu.fused_linear import input_grad, small_dgrad
+    w = (torch.randn(64, 72, device=dev) * 0.1).bfloat16()
+    for dy in (torch.randn(64, device=dev).bfloat16().expand(100, 64), torch.randn(900, device=dev).bfloat16().unfold(0, 64, 8)[:100],
+               torch.randn(6403, device=dev).bfloat16()[3:].view(100, 64), torch.randn(1, 64, device=dev).bfloat16().as_strided((1, 64), (0, 1))):
+        assert small_dgrad(len(dy), 72, 64)
+        ref = dy.float() @ w.float()
+        assert bool(((input_grad(dy, w).float() - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-5 * ref.abs().max()).all())
+
+
 @pytest.mark.parametrize("M", [16, 256, 300])     # few rows, whole tiles, small tiles
 def test_a_weight_on_the_host_is_refused(dev, M):
     # as torch.mm refuses it, and before any launch

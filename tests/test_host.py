@@ -35,3 +35,19 @@ def test_tensors_off_the_gpu_are_refused(host):
         assert none is None
     from fxgpu.fused_linear import input_grad
     assert torch.equal(input_grad(x + 1, w + 1), torch.mm(x + 1, w + 1))     # on the CPU as before: torch's product
+
+
+def test_rows(host):
+    # aligned rows that do not overlap: a view where t has them, else a copy
+    flat = torch.arange(4096).bfloat16()
+    base = flat.data_ptr()
+    for t in (flat[:640].view(10, 64), flat[:640].view(2, 5, 64), flat.view(-1, 128)[:, 64:], flat[:64].view(1, 64)):
+        r = host.rows(t)
+        assert r.data_ptr() == t.data_ptr() and torch.equal(r, t.reshape(-1, 64))
+    odd = (flat[3:643].view(10, 64), flat[:64].expand(10, 64), flat.unfold(0, 64, 8)[:10], flat[:640].view(64, 10).t(), flat[:690].view(10, 69)[:, :64],
+           flat[:64].as_strided((1, 64), (0, 1)), flat[3:67].as_strided((1, 64), (1, 1)))
+    for t in odd:
+        r = host.rows(t)
+        assert torch.equal(r, t) and r.stride() == (64, 1) and r.data_ptr() % 16 == 0
+    assert host.rows(odd[-2]).data_ptr() == base       # one row: its stride alone was odd
+    assert host.rows(flat[:0].view(0, 64)).shape == (0, 64)
