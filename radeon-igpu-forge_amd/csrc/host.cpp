@@ -32,17 +32,12 @@ bool aligned(const Tensor& t) { return (reinterpret_cast<uintptr_t>(t.data_ptr()
 bool is_bf(const Tensor& t) { return t.scalar_type() == at::kBFloat16; }
 at::TensorOptions as_f32(const Tensor& t) { return t.options().dtype(at::kFloat); }
 
-[[noreturn]] void raise(PyObject* type, const std::string& msg) {
-    PyErr_SetString(type, msg.c_str());
-    throw py::error_already_set();
-}
-
 // the C ABI's return code as the Python wrappers report it (fxgpu.abi.call)
 void check(int rc, const char* name) {
     if (rc == 0) return;
     const std::string msg = fx_last_error();
-    if (rc == FX_EINVAL) raise(PyExc_ValueError, msg);
-    raise(PyExc_RuntimeError, std::string(name) + " failed: hipError=" + std::to_string(rc) + " (" + msg + ")");
+    if (rc == FX_EINVAL) throw py::value_error(msg);
+    throw std::runtime_error(std::string(name) + " failed: hipError=" + std::to_string(rc) + " (" + msg + ")");
 }
 
 const Tensor* given(const Tensor& t) { return &t; }
@@ -52,11 +47,11 @@ const Tensor* given(const OptT& t) { return t.has_value() ? &*t : nullptr; }
 // GPU's, is refused here and never launched with
 template <class... Rest>
 void same_gpu(const Tensor& a, const Rest&... rest) {
-    if (!a.is_cuda()) raise(PyExc_RuntimeError, "expected all tensors to be on one GPU, got " + a.device().str());
+    if (!a.is_cuda()) throw std::runtime_error("expected all tensors to be on one GPU, got " + a.device().str());
     for (const Tensor* t : std::initializer_list<const Tensor*>{given(rest)...})
         if (t && t->device() != a.device())
-            raise(PyExc_RuntimeError,
-                  "expected all tensors to be on one GPU, got " + a.device().str() + " and " + t->device().str());
+            throw std::runtime_error("expected all tensors to be on one GPU, got " + a.device().str() + " and " +
+                                     t->device().str());
 }
 
 // ---- RMSNorm ---------------------------------------------------------------------------
@@ -295,12 +290,12 @@ std::optional<std::tuple<Tensor, OptT>> gather_fwd(const Tensor& X, const Tensor
 
 // dW = dy^T x
 Tensor wgrad(const Tensor& dy, const Tensor& x) {
-    if (!is_bf(dy) || !is_bf(x)) raise(PyExc_TypeError, "dy and x must be bfloat16");
-    if (!dy.is_cuda() || !x.is_cuda()) raise(PyExc_TypeError, "dy and x must be cuda tensors");
+    if (!is_bf(dy) || !is_bf(x)) throw py::type_error("dy and x must be bfloat16");
+    if (!dy.is_cuda() || !x.is_cuda()) throw py::type_error("dy and x must be cuda tensors");
     same_gpu(dy, x);
     const Tensor dy2 = rows(dy), x2 = rows(x);
     if (dy2.size(0) != x2.size(0))
-        raise(PyExc_ValueError, "dy has " + std::to_string(dy2.size(0)) + " rows, x has " + std::to_string(x2.size(0)));
+        throw py::value_error("dy has " + std::to_string(dy2.size(0)) + " rows, x has " + std::to_string(x2.size(0)));
     const int64_t T = dy2.size(0), N = dy2.size(1), K = x2.size(1);
     if (N % 8 || K % 8) return at::mm(dy2.t(), x2);
     Tensor dW = at::empty({N, K}, x2.options());
@@ -468,17 +463,16 @@ OptT few_rows_logits(const Tensor& x, const Tensor& w, const Tensor& norm_w, dou
 struct FlatLayout {
     std::vector<int64_t> off, n;
     std::vector<int32_t> wd;
-    std::vector<fxTensorList> lists;   // filled anew by every step
 };
 
 // One optimiser step over the parameters that have a gradient.  t: master, m, v, flat16, step,
 // found_inf, grad norm, scale, growth.  h: lr, beta1, beta2, eps, weight decay, max norm,
 // growth interval.  Returns the workspace (grown when too small) and -1, or the index of a
 // parameter whose gradient is not bf16 (-2 - index: not 16-byte aligned), nothing launched.
-std::tuple<Tensor, int64_t> adamw_step(FlatLayout& f, const std::vector<Tensor>& params, const std::vector<Tensor>& t,
+std::tuple<Tensor, int64_t> adamw_step(const FlatLayout& f, const std::vector<Tensor>& params, const std::vector<Tensor>& t,
                                        const std::vector<double>& h, Tensor work) {
     std::vector<Tensor> keep;   // contiguous copies, alive until the launches are queued
-    f.lists.clear();
+    std::vector<fxTensorList> lists;
     for (size_t i = 0; i < params.size(); ++i) {
         Tensor g = params[i].grad();
         if (!g.defined()) continue;
@@ -489,11 +483,11 @@ std::tuple<Tensor, int64_t> adamw_step(FlatLayout& f, const std::vector<Tensor>&
             keep.push_back(g);
         }
         if (!aligned(g)) return std::make_tuple(work, -2 - (int64_t)i);
-        if (f.lists.empty() || f.lists.back().count == FX_ADAMW_MAX_TENSORS) {
-            f.lists.emplace_back();
-            f.lists.back().count = 0;
+        if (lists.empty() || lists.back().count == FX_ADAMW_MAX_TENSORS) {
+            lists.emplace_back();
+            lists.back().count = 0;
         }
-        fxTensorList& l = f.lists.back();
+        fxTensorList& l = lists.back();
         l.g[l.count] = bf(g);
         l.off[l.count] = f.off[i];
         l.n[l.count] = f.n[i];
@@ -501,10 +495,9 @@ std::tuple<Tensor, int64_t> adamw_step(FlatLayout& f, const std::vector<Tensor>&
         ++l.count;
     }
     for (const Tensor& s : t) same_gpu(t[0], s);
-    fxTensorList none{};
-    const fxTensorList* lists = f.lists.empty() ? &none : f.lists.data();
-    const int32_t nl = (int32_t)f.lists.size();
-    const int64_t need = fx_adamw_workspace(lists, nl) / 4;
+    const int32_t nl = (int32_t)lists.size();
+    if (lists.empty()) lists.emplace_back();   // a list to point to
+    const int64_t need = fx_adamw_workspace(lists.data(), nl) / 4;
     if (work.numel() < need) work = at::empty({need}, t[0].options());
     fxAdamWState s{};
     s.master = f32(t[0]);
@@ -526,14 +519,16 @@ std::tuple<Tensor, int64_t> adamw_step(FlatLayout& f, const std::vector<Tensor>&
     s.growth_factor = 2.f;
     s.backoff_factor = 0.5f;
     s.growth_interval = (int32_t)h[6];
-    check(fx_adamw_step(&s, lists, nl, stream_of(t[0])), "fx_adamw_step");
+    check(fx_adamw_step(&s, lists.data(), nl, stream_of(t[0])), "fx_adamw_step");
     return std::make_tuple(work, (int64_t)-1);
 }
 
 }  // namespace
 
-// every function: torch's exceptions (out of memory among them) reach Python as themselves
-#define FX_DEF(name) m.def(#name, torch::wrap_pybind_function(name))
+// every function: torch's exceptions (out of memory among them) reach Python as themselves, and other
+// Python threads run during the call, as during a ctypes call: an allocation that reaches the driver
+// or a launch into a full queue may wait.  So none of them calls Python or keeps state.
+#define FX_DEF(name) m.def(#name, torch::wrap_pybind_function_no_gil(name))
 
 PYBIND11_MODULE(_host, m) {
     FX_DEF(norm_fwd);
@@ -560,12 +555,12 @@ PYBIND11_MODULE(_host, m) {
     FX_DEF(ce_lin_scale_inplace);
     py::class_<FlatLayout>(m, "FlatLayout")
         .def(py::init([](std::vector<int64_t> off, std::vector<int64_t> n, std::vector<int32_t> wd) {
-            return FlatLayout{std::move(off), std::move(n), std::move(wd), {}};
+            return FlatLayout{std::move(off), std::move(n), std::move(wd)};
         }))
         .def(py::pickle([](const FlatLayout& f) { return py::make_tuple(f.off, f.n, f.wd); },
                         [](const py::tuple& t) {
                             return FlatLayout{t[0].cast<std::vector<int64_t>>(), t[1].cast<std::vector<int64_t>>(),
-                                              t[2].cast<std::vector<int32_t>>(), {}};
+                                              t[2].cast<std::vector<int32_t>>()};
                         }));
     FX_DEF(adamw_step);
 }

@@ -1,4 +1,7 @@
 """What the host module refuses before it launches anything (CPU)."""
+import threading
+import time
+
 import pytest
 import torch
 
@@ -51,3 +54,22 @@ def test_rows(host):
         assert torch.equal(r, t) and r.stride() == (64, 1) and r.data_ptr() % 16 == 0
     assert host.rows(odd[-2]).data_ptr() == base       # one row: its stride alone was odd
     assert host.rows(flat[:0].view(0, 64)).shape == (0, 64)
+
+
+def test_other_python_threads_run_during_a_call(host):
+    stamps, stop = [], threading.Event()
+
+    def tick():
+        while not stop.is_set():
+            stamps.append(time.perf_counter())
+            time.sleep(1e-3)
+    other = threading.Thread(target=tick)
+    t = torch.ones(12000, 16000, dtype=torch.bfloat16).t()     # a copy of some 0.1 s
+    other.start()
+    t0 = time.perf_counter()
+    host.rows(t)
+    t1 = time.perf_counter()
+    stop.set()
+    other.join()
+    third = (t1 - t0) / 3     # the call's middle, away from the switches at its ends
+    assert any(t0 + third < s < t1 - third for s in stamps), (t1 - t0, len(stamps))
