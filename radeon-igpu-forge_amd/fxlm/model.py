@@ -154,6 +154,16 @@ class Block(nn.Module):
                 and rows <= FEW_ROWS)
 
 
+def _table_lookup(m):
+    """Whether calling m only reads rows of its weight: torch's embedding with no hook on its call,
+    no forward of its own and no renormalised rows."""
+    hooks = nn.modules.module
+    return (type(m) is nn.Embedding and m.max_norm is None and "forward" not in vars(m)
+            and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
+                     or hooks._global_forward_hooks or hooks._global_forward_pre_hooks
+                     or hooks._global_backward_hooks or hooks._global_backward_pre_hooks))
+
+
 class GPT(nn.Module):
     def __init__(self, cfg: GPTConfig):
         super().__init__()
@@ -267,7 +277,9 @@ class GPT(nn.Module):
         lens (B,) int32 = pos + 1; returns the logits (B, V) fp32."""
         B = tok.shape[0]
         fused = bool(self.blocks) and self.blocks[0]._fused_step(B)
-        x = host.decode_embed(tok, pos, self.tok_emb.weight, self.pos_emb) if fused and tok.is_cuda else None
+        x = None
+        if fused and tok.is_cuda and _table_lookup(self.tok_emb):
+            x = host.decode_embed(tok, pos, self.tok_emb.weight, self.pos_emb)
         if x is None:
             x = self.tok_emb(tok.view(B, 1)) + self.pos_emb.index_select(0, pos)
         for blk, kv in zip(self.blocks, cache):

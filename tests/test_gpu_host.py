@@ -150,3 +150,19 @@ def test_decode_graph_takes_positions_of_any_number_type(dev):
     want = step(tok, 7).clone()
     for pos in (7.0, np.int64(7), torch.tensor(7), torch.tensor(7, device=dev)):
         assert torch.equal(step(tok, pos), want), type(pos)
+
+
+def test_hooks_on_the_embedding_run_in_cached_steps(dev):
+    from fxlm import GPT, GPTConfig
+    torch.manual_seed(3)
+    with torch.device(dev):
+        model = GPT(GPTConfig(vocab_size=256, seq_len=64, n_layer=1, n_head=2, d_model=128)).bfloat16()
+    cache = [tuple(torch.zeros(2, 64, 2, 64, device=dev).bfloat16() for _ in range(2))]
+    tok = torch.tensor([5, 9], device=dev)
+    plain, graph = model.decode_step(tok, cache, 7), model.decode_graph(cache, 2)
+    assert torch.equal(graph(tok, 7), plain)
+    swap = {5: 9, 9: 5}
+    handle = model.tok_emb.register_forward_pre_hook(lambda m, a: (torch.tensor([[swap[int(i)]] for i in a[0].flatten()], device=dev),))
+    assert torch.equal(model.decode_step(tok, cache, 7), plain.flip(0))
+    handle.remove()
+    assert torch.equal(model.decode_step(tok, cache, 7), plain)

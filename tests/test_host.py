@@ -73,3 +73,27 @@ def test_other_python_threads_run_during_a_call(host):
     other.join()
     third = (t1 - t0) / 3     # the call's middle, away from the switches at its ends
     assert any(t0 + third < s < t1 - third for s in stamps), (t1 - t0, len(stamps))
+
+
+def test_a_hooked_embedding_is_no_table_lookup():
+    from torch import nn
+
+    from fxlm.model import _table_lookup
+
+    class Other(nn.Embedding):
+        def forward(self, i):
+            return 2 * super().forward(i)
+    assert _table_lookup(nn.Embedding(8, 8)) and not _table_lookup(Other(8, 8)) and not _table_lookup(nn.Embedding(8, 8, max_norm=1.0))
+    for register in ("register_forward_hook", "register_forward_pre_hook", "register_full_backward_hook"):
+        m = nn.Embedding(8, 8)
+        handle = getattr(m, register)(lambda *a: None)
+        assert not _table_lookup(m)
+        handle.remove()
+        assert _table_lookup(m)
+    m.forward = lambda i: i
+    assert not _table_lookup(m)
+    handle = nn.modules.module.register_module_forward_hook(lambda *a: None)
+    try:
+        assert not _table_lookup(nn.Embedding(8, 8))
+    finally:
+        handle.remove()
