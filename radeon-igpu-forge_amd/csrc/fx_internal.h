@@ -22,8 +22,8 @@ int column_sums(const uint16_t* g, int64_t rows, int64_t cols, float* work, uint
 // A decode step's small ends, one launch each.
 // tok_out[0..n) = tok, *pos_out = pos, lens[0..n) = pos + 1
 int decode_inputs(const int64_t* tok, int64_t n, int64_t pos, int64_t* tok_out, int64_t* pos_out, int32_t* lens, void* stream);
-// x (n, D) = bf16(E[tok[i]] + P[*pos]), E (V, D) and P (T, D) contiguous, D a multiple of 8; an id or
-// a position outside its table traps, as torch's index checks do
+// x (n, D) = bf16(E[tok[i]] + P[*pos]), E (V, D) and P (T, D) contiguous, D a multiple of 8; a row of
+// NaN for an id or a position outside its table
 int decode_embed(const int64_t* tok, const int64_t* pos, const uint16_t* E, int64_t V, const uint16_t* P, int64_t T, uint16_t* x,
                  int64_t n, int64_t D, void* stream);
 // out (M, N) fp32 = the bf16 values of norm(X) W^T (fx_linear_fwd_ex with the norm, M <= 64), X rows

@@ -297,8 +297,7 @@ class GPT(nn.Module):
         """tok (B,) int64 at position pos (< the cache length, every sequence at the same
         position); returns its logits (B, V) in fp32."""
         B = tok.shape[0]
-        if pos >= cache[0][0].shape[1]:
-            raise ValueError(f"position {pos} is past the cache ({cache[0][0].shape[1]})")
+        _check_pos(pos, cache[0][0].shape[1], self.pos_emb.shape[0])
         p = torch.full((1,), pos, dtype=torch.int64, device=tok.device)
         lens = torch.full((B,), pos + 1, dtype=torch.int32, device=tok.device)
         return self._decode(tok, cache, p, lens)
@@ -343,6 +342,14 @@ class GPT(nn.Module):
         return torch.cat(out, dim=1) if out else idx.new_zeros(B, 0)
 
 
+def _check_pos(pos, cache_len, positions):
+    """Refuse a cached step at a position that the cache or the position table does not have."""
+    if pos >= cache_len:
+        raise ValueError(f"position {pos} is past the cache ({cache_len})")
+    if int(pos) < 0 or pos >= positions:
+        raise ValueError(f"position {pos} is not one of the model's {positions}")
+
+
 class _DecodeGraph:
     """One cached decode step captured in a HIP graph (torch.cuda.CUDAGraph).  Inputs
     are copied into static device tensors before each replay; the kernels read the
@@ -351,6 +358,7 @@ class _DecodeGraph:
     def __init__(self, model, cache, batch):
         dev = cache[0][0].device
         self.cache_len = cache[0][0].shape[1]
+        self.positions = model.pos_emb.shape[0]
         self.tok = torch.zeros(batch, dtype=torch.int64, device=dev)
         self.pos = torch.zeros(1, dtype=torch.int64, device=dev)
         self.lens = torch.ones(batch, dtype=torch.int32, device=dev)
@@ -374,8 +382,7 @@ class _DecodeGraph:
                 v[:, :1].copy_(v0)
 
     def __call__(self, tok, pos):
-        if pos >= self.cache_len:
-            raise ValueError(f"position {pos} is past the cache ({self.cache_len})")
+        _check_pos(pos, self.cache_len, self.positions)
         if not (torch.is_tensor(tok) and host.decode_inputs(tok, int(pos), self.tok, self.pos, self.lens)):
             self.tok.copy_(tok)
             self.pos.fill_(pos)

@@ -166,3 +166,22 @@ def test_hooks_on_the_embedding_run_in_cached_steps(dev):
     assert torch.equal(model.decode_step(tok, cache, 7), plain.flip(0))
     handle.remove()
     assert torch.equal(model.decode_step(tok, cache, 7), plain)
+
+
+def test_rows_outside_the_tables(dev):
+    # the graph's call refuses a position on the host; an id that no row has gives NaN to its own sequence
+    from fxgpu.abi import host
+    from fxlm import GPT, GPTConfig
+    with torch.device(dev):
+        model = GPT(GPTConfig(vocab_size=256, seq_len=16, n_layer=1, n_head=2, d_model=128)).bfloat16()
+    step = model.decode_graph([tuple(torch.zeros(2, 32, 2, 64, device=dev).bfloat16() for _ in range(2))], 2)
+    tok = torch.tensor([5, 9], device=dev)
+    for pos in (-1, 16, 32, -1.0, torch.tensor(16)):
+        with pytest.raises(ValueError, match="position"):
+            step(tok, pos)
+    assert bool(step(tok, 15).isfinite().all())
+    E, P = (torch.randn(n, 72, device=dev).bfloat16() for n in (6, 4))
+    ids, pos = torch.tensor([0, -1, 5, 6, 2 ** 40], device=dev), torch.tensor([3], device=dev)
+    x = host.decode_embed(ids, pos, E, P)[:, 0]
+    assert torch.equal(x[[0, 2]], E[[0, 5]] + P[3]) and bool(x[[1, 3, 4]].isnan().all())
+    assert bool(host.decode_embed(ids, pos + 1, E, P).isnan().all())

@@ -97,3 +97,13 @@ def test_a_hooked_embedding_is_no_table_lookup():
         assert not _table_lookup(nn.Embedding(8, 8))
     finally:
         handle.remove()
+
+
+def test_positions_outside_the_model_are_refused():
+    from fxlm import GPT, GPTConfig
+    model = GPT(GPTConfig(vocab_size=64, seq_len=16, n_layer=1, n_head=2, d_model=128))
+    tok = torch.tensor([1, 2])
+    cache = [tuple(torch.zeros(2, 32, 2, 64) for _ in range(2))]     # longer than the position table
+    for pos in (-1, 16, 31, 32):
+        with pytest.raises(ValueError, match="position"):
+            model.decode_step(tok, cache, pos)
