@@ -556,11 +556,6 @@ PYBIND11_MODULE(_host, m) {
     py::class_<FlatLayout>(m, "FlatLayout")
         .def(py::init([](std::vector<int64_t> off, std::vector<int64_t> n, std::vector<int32_t> wd) {
             return FlatLayout{std::move(off), std::move(n), std::move(wd)};
-        }))
-        .def(py::pickle([](const FlatLayout& f) { return py::make_tuple(f.off, f.n, f.wd); },
-                        [](const py::tuple& t) {
-                            return FlatLayout{t[0].cast<std::vector<int64_t>>(), t[1].cast<std::vector<int64_t>>(),
-                                              t[2].cast<std::vector<int32_t>>()};
-                        }));
+        }));
     FX_DEF(adamw_step);
 }

@@ -65,11 +65,23 @@ class FlatAdamW:
         self.scale = torch.full((), float(init_scale), device=dev, dtype=torch.float32)
         self._growth = torch.zeros((), device=dev, dtype=torch.int32)
         self._work = torch.empty(0, device=dev, dtype=torch.float32)
+        self._index()
+
+    # -- helpers -------------------------------------------------------------
+
+    def _index(self):
+        """The parameters and their flat layout as step() hands them to the host module."""
         self._params = [p for _n, p, _o, _el, _w in self._info]
         self._layout = host.FlatLayout([i[2] for i in self._info], [i[3] for i in self._info],
                                        [i[4] for i in self._info])
 
-    # -- helpers -------------------------------------------------------------
+    def __getstate__(self):
+        # pickles and copies hold neither: _info has both, and files from before _index() load too
+        return {k: v for k, v in self.__dict__.items() if k not in ("_params", "_layout")}
+
+    def __setstate__(self, state):
+        self.__dict__.update(state)
+        self._index()
 
     def _lists(self):
         """Tensor lists (<= 64 entries each) over the parameters that have a gradient."""

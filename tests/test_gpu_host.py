@@ -119,6 +119,28 @@ def test_optimizer_deepcopy_takes_the_same_step(dev):
     assert torch.equal(opt.master, twin.master) and float(opt._step_ctr) == 1
 
 
+def test_optimizer_pickles_hold_tensors_and_numbers_only(dev):
+    # whole-object files, those written before the host module among them: its objects are made anew
+    import pickle
+    from fxlm.optim import FlatAdamW
+    model = torch.nn.Linear(64, 40).to(dev)
+    opt = FlatAdamW(model, init_scale=1.0)
+    assert b"_host" not in pickle.dumps(opt)
+    old = FlatAdamW.__new__(FlatAdamW)
+    old.__setstate__({k: v for k, v in opt.__dict__.items() if k not in ("_params", "_layout")})
+    for p in model.parameters():
+        p.grad = torch.ones_like(p)
+    old.step()
+    assert int(opt._step_ctr) == 1 and old._params[0] is opt._params[0]
+    back = pickle.loads(pickle.dumps((model, opt)))[1]
+    assert back._params[0] is not opt._params[0] and torch.equal(back.master, opt.master)
+    for o in (back, opt):
+        for p in o._params:
+            p.grad = torch.ones_like(p)
+        o.step()
+    assert torch.equal(back.master, opt.master) and int(back._step_ctr) == 2
+
+
 @pytest.mark.parametrize("B,V,D", [(1, 256, 64), (17, 50304, 768), (64, 1003, 1032)])
 def test_decode_step_ends_equal_the_torch_operations(dev, B, V, D):
     # bit for bit: the embedding sum, the graph's inputs, and the head's bf16 logits as fp32
