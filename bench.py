@@ -110,15 +110,14 @@ def graph_time_us(torch, fn, reps=20, iters=10):
 
 
 def bench_attention(torch):
-    from fxlm.attention import _bwd, _fwd
+    from fxgpu.abi import host   # what the autograd function calls
     B, T, H, D = 16, 1024, 12, 64
     g = torch.Generator(device="cuda").manual_seed(2)
     q, k, v, do = (torch.randn(B, T, H, D, device="cuda", generator=g).bfloat16() for _ in range(4))
     scale = 1.0 / math.sqrt(D)
-    o, lse = _fwd(q, k, v, True, scale)
-    dq, dk, dv = (torch.empty_like(q) for _ in range(3))
-    t_fwd = time_us(torch, lambda: _fwd(q, k, v, True, scale))
-    t_bwd = time_us(torch, lambda: _bwd(q, k, v, o, lse, do, True, scale, dq, dk, dv))
+    o, lse = host.attn_fwd(q, k, v, True, scale)
+    t_fwd = time_us(torch, lambda: host.attn_fwd(q, k, v, True, scale))
+    t_bwd = time_us(torch, lambda: host.attn_bwd(q, k, v, o, lse, do, True, scale))
     f_fwd = 4.0 * B * H * T * T * D * 0.5          # causal half of QK^T and PV
     f_bwd = 2.5 * f_fwd                            # dV, dP, dK, dQ (+ recomputed S)
     return {

@@ -47,8 +47,7 @@ def linear_wgrad(dy, x):
 
 
 # Up to this many rows the forward GEMM is a stream over the weight (decoding, small
-# batches) and runs on this build's few-row kernel; above it on the library GEMM, except
-# for the shapes of whole_tiles().
+# batches) and runs on this build's few-row kernels; above it native_fwd() decides.
 FEW_ROWS = 64
 
 
@@ -92,7 +91,7 @@ NATIVE_PROJ_FWD = True
 # faster); evaluating the derivative from the pre-activation in that epilogue had measured
 # 0.04 ms slower than the library GEMM and fx_gelu_bwd.
 NATIVE_GELU_INPUT_GRAD = True
-# NATIVE_SMALL_INPUT_GRAD: the plain input gradients of small_dgrad() on fx_linear_dgrad.
+# NATIVE_SMALL_INPUT_GRAD: the plain input gradients of small_dgrad() on this build's kernels.
 NATIVE_SMALL_INPUT_GRAD = True
 
 
@@ -113,7 +112,10 @@ def dgrad_tiles(M, N, K):
 def input_grad(dy2, weight, g=None):
     """dx = dy2 @ weight (bf16), and with g (the GELU(tanh) derivative at the output of the
     layer feeding this one, as fx_linear_fwd with act 2 stores it) bf16(dx) * g.  The
-    small_dgrad() products run on fx_linear_dgrad; with NATIVE_INPUT_GRAD, on fx_linear_dgrad for dgrad_tiles() shapes where it measured at
+    small_dgrad() products run on this build's kernels: the dgrad_tiles() ones of a K up to 3072
+    (any K with g) on fx_linear_dgrad(_gate), which takes the small tiles or the whole ones, the
+    ragged and the longer ones on fx::input_grad.  With NATIVE_INPUT_GRAD, larger dgrad_tiles()
+    shapes on fx_linear_dgrad where it measured at
     least as fast as the library GEMM with the operands in the caches (input widths up to
     1024 columns: the cfg5 qkv, proj and fc input gradients, 52.1 / 22.9 / 66.0 us against
     60.5 / 25.4 / 67.2 us; from HBM 72.3 / 31.6 / 93.7 against 64.5 / 30.3 / 82.4 us); with

@@ -66,23 +66,6 @@ def _fwd(q, k, v, causal, scale):
     return o, lse
 
 
-def _bwd(q, k, v, o, lse, do, causal, scale, dq, dk, dv):
-    B, T, H, Dh = q.shape
-    do = do.contiguous()
-    if do.dtype != torch.bfloat16:
-        do = do.to(torch.bfloat16)
-    delta = torch.empty(B, H, T, device=q.device, dtype=torch.float32)
-    a = _args(q, k, v, causal, scale)
-    a.o, a.dout = o.data_ptr(), do.data_ptr()
-    a.lse, a.delta = lse.data_ptr(), delta.data_ptr()
-    a.dq, a.dk, a.dv = dq.data_ptr(), dk.data_ptr(), dv.data_ptr()
-    a.dqb, a.dqt, a.dqh = _strides3(dq)
-    a.dkb, a.dkt, a.dkh = _strides3(dk)
-    a.dvb, a.dvt, a.dvh = _strides3(dv)
-    call("fx_attn_bwd", ctypes.byref(a), stream_of(q))
-    return dq, dk, dv
-
-
 class _FlashAttn(torch.autograd.Function):
     """flash_attention(q, k, v): o (B,T,H,Dh) contiguous bf16."""
 

@@ -20,9 +20,10 @@ def abi():
     from fxgpu import abi as _abi
     srcs = os.path.join(ROOT, "radeon-igpu-forge_amd", "csrc")
     newest = max(os.path.getmtime(os.path.join(srcs, f)) for f in os.listdir(srcs)
-                 if f.endswith((".hip", ".h")))
+                 if f.endswith((".hip", ".h", ".cpp")))
     newest = max(newest, os.path.getmtime(HEADER))
-    if not os.path.exists(_abi.LIB_PATH) or os.path.getmtime(_abi.LIB_PATH) < newest:
+    host = os.path.join(os.path.dirname(_abi.__file__), "_host.so")
+    if any(not os.path.exists(p) or os.path.getmtime(p) < newest for p in (_abi.LIB_PATH, host)):
         subprocess.run(["python", os.path.join(srcs, "build.py")], check=True)
     return _abi
 
